@@ -62,8 +62,7 @@ SWC_API const char *swc_winograd2x2_conv_last_kernel(void);
 /* Diagnostic with no counterpart in the reference: how that call ran over fp32 planes: "whole" (the tiling of
  * swc_winograd2x2_conv_last_kernel(), one workgroup per tile), or, on grids that leave most of the device idle that
  * way, "direct16x16" / "direct16x32" / "direct16x64" / "direct32x64": sixteen waves per workgroup, one per position,
- * each with the named tile of rows x columns (C % 4 == 0); or "split32" / "split48" / "split64" / "split64+32" /
- * "split64+48" (whole rounds of 64-row tiles, the rest in lower ones): tiles of that many
+ * each with the named tile of rows x columns (C % 4 == 0); or "split32" / "split48" / "split64": tiles of that many
  * rows x 64 columns on the 16-bit matrix instructions, fp32 operands as pairs of f16 values (23 bits and a sign, fp32
  * sums: nearer to float64 than the fp32 instructions; a tile with values that do not split well is multiplied again with
  * those), bf16 operands as they are. */

@@ -81,11 +81,11 @@ int conv_entry(const float *Input, const float *Weight, float *Output, int C, in
     // instructions' peak and measures 3.75); the bf16-operand ring 6 + 9 us per 64 channels while a CU has one tile.
     const double per64 = static_cast<double>(C) / 64;
     const double whole_us = pick.tiling == TILING_SYNC ? 1e30 : BF16 ? 6.0 + 9.0 * per64 : 6.0 + 3.75 * pick.cost * per64;
-    double direct_us;
+    double direct_us, split_us;
     const DirectForm direct = choose_direct(Input, Weight, M, C, K, pick.tiling != TILING_SYNC, BF16, &direct_us);
-    const SplitChoice split = choose_split(Input, Weight, Output, ep.residual, M, C, K, BF16);
-    if (split.form != SPLIT_NONE && split.us < direct_us && split.us < whole_us) {
-        note_conv_form(kSplitNames[split.form]);
+    const SplitForm split = choose_split(Input, Weight, Output, ep.residual, M, C, K, BF16, &split_us);
+    if (split != SPLIT_NONE && split_us < direct_us && split_us < whole_us) {
+        note_conv_form(kSplitNames[split]);
         return launch_split(split, BF16, Input, Weight, Output, M, C, K, nW, ep.scale, ep.shift, ep.residual, ep.residual_relu, s);
     }
     if (direct != DIRECT_NONE) {

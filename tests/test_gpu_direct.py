@@ -69,9 +69,7 @@ def test_direct_forms(oracle, forced, form, shape, precision):
     ((16, 7, 7, 256, 256), "direct16x64"),
     ((16, 7, 7, 512, 512), "split32"),        # 200 tiles of 32x64, which the split form multiplies faster
     ((64, 14, 14, 128, 64), "split64"),       # 196 tiles of 64x64
-    ((64, 14, 14, 128, 128), "split64+48"),   # 392: one round, the rest in 182 lower ones
-    ((128, 14, 14, 128, 128), "split64+32"),  # 784: three rounds, and 512 rows in lower tiles
-    ((64, 28, 28, 32, 64), "whole"),          # below 64 channels
+    ((64, 28, 28, 64, 64), "whole"),          # 784: four rounds, the last nearly empty
 ])
 def test_the_launcher_picks_the_smallest_tile_that_needs_one_round(forced, shape, want):
     from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv

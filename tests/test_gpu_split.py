@@ -9,10 +9,9 @@ from test_gpu_direct import forced, tiles_of  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
-FORMS = ["split32", "split48", "split64", "split64+32", "split64+48"]
-# "split64+32" forced takes half of the whole 64-row tiles and leaves the rest to 32-row ones.
-# (B, nH, nW, C, K): M = 1, 17, 33, 49, 65, 130, 255 rows; C below, at and past a step of 32 indices; K below, at and past 64
-SHAPES = [(1, 1, 1, 4, 4), (1, 1, 17, 36, 20), (3, 1, 11, 64, 68), (1, 7, 7, 100, 132), (1, 5, 13, 28, 64), (2, 5, 13, 160, 36), (1, 15, 17, 64, 132)]
+FORMS = ["split32", "split48", "split64"]
+# (B, nH, nW, C, K): M = 1, 17, 33, 49, 65, 130 rows; C below, at and past a step of 32 indices; K below, at and past 64
+SHAPES = [(1, 1, 1, 4, 4), (1, 1, 17, 36, 20), (3, 1, 11, 64, 68), (1, 7, 7, 100, 132), (1, 5, 13, 28, 64), (2, 5, 13, 160, 36)]
 
 
 def bound(ti, w):
