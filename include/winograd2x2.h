@@ -62,10 +62,8 @@ SWC_API const char *swc_winograd2x2_conv_last_kernel(void);
 /* Diagnostic with no counterpart in the reference: how that call ran over fp32 planes: "whole" (the tiling of
  * swc_winograd2x2_conv_last_kernel(), one workgroup per tile), or, on grids that leave most of the device idle that
  * way, "direct16x16" / "direct16x32" / "direct16x64" / "direct32x64": sixteen waves per workgroup, one per position,
- * each with the named tile of rows x columns (C % 4 == 0); or "split32" / "split48" / "split64": tiles of that many
- * rows x 64 columns on the 16-bit matrix instructions, fp32 operands as pairs of f16 values (23 bits and a sign, fp32
- * sums: nearer to float64 than the fp32 instructions; a tile with values that do not split well is multiplied again with
- * those), bf16 operands as they are. */
+ * each with the named tile of rows x columns (C % 4 == 0); or, with bf16 operands, "split32" / "split48" / "split64": tiles
+ * of that many rows x 64 columns, the positions split over eight waves. */
 SWC_API const char *swc_winograd2x2_conv_last_form(void);
 /* Diagnostic with no counterpart in the reference, for benchmarks and tests that compare the tilings: makes
  * the calling thread's later swc_winograd2x2_conv calls
@@ -289,7 +287,7 @@ SWC_API int swc_winograd2x2_pointwise_conv(const float *Input, const float *Weig
  * The model's first two layers in one kernel: Output [B,Hp,Wp,64] = 3x3 stride-2 max-pool of the 7x7 stride-2
  * convolution of Input [B,H,W,3] (NHWC) with Weight [64,3,7,7], both with TensorFlow's SAME padding
  * (ResNet-18-var/imagenet-resnet-transWino-prune.py:113-115); Hp = ceil(ceil(H/2)/2), Wp alike.  fp32; the products are
- * taken as in the "split" forms of the convolution.  Output 16-byte aligned (SWC_ERR_UNSUPPORTED otherwise).
+ * taken as three of pairs of f16 values.  Output 16-byte aligned (SWC_ERR_UNSUPPORTED otherwise).
  */
 SWC_API int swc_stem_conv_pool(const float *Input, const float *Weight, float *Output, int B, int H, int W,
                                swc_stream_t stream);

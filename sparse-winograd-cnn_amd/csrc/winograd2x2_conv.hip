@@ -77,16 +77,15 @@ int conv_entry(const float *Input, const float *Weight, float *Output, int C, in
     TilingChoice pick = {ring_eligible<Tile32>(Input, Weight, C, K, true) ? TILING_RING32 : TILING_SYNC, Tile32::BM};
     if (!BF16) pick = choose_tiling(Input, Weight, M, C, K, true, true);
     note_conv_kernel(tiling_name(pick.tiling));
-    // What the ring and wide kernels take, from their cost in MFMA units (a unit is 3.4 us per 64 channels at the fp32
-    // instructions' peak and measures 3.75); the bf16-operand ring 6 + 9 us per 64 channels while a CU has one tile.
-    const double per64 = static_cast<double>(C) / 64;
-    const double whole_us = pick.tiling == TILING_SYNC ? 1e30 : BF16 ? 6.0 + 9.0 * per64 : 6.0 + 3.75 * pick.cost * per64;
-    double direct_us, split_us;
+    double direct_us, split_us = 1e30;
     const DirectForm direct = choose_direct(Input, Weight, M, C, K, pick.tiling != TILING_SYNC, BF16, &direct_us);
-    const SplitForm split = choose_split(Input, Weight, Output, ep.residual, M, C, K, BF16, &split_us);
-    if (split != SPLIT_NONE && split_us < direct_us && split_us < whole_us) {
+    const SplitForm split = BF16 ? choose_split(Input, Weight, Output, ep.residual, M, C, K, &split_us) : SPLIT_NONE;
+    // The bf16-operand ring takes 6 us + 9 per 64 channels at best (one tile per CU); below 64 channels that is less than
+    // the split forms' 6.5 to 8.5 + 4.1 to 5.  A direct form is offered only where it takes less than the ring.
+    const double ring_us = pick.tiling == TILING_SYNC ? 1e30 : 6.0 + 9.0 * C / 64;
+    if (split != SPLIT_NONE && split_us < direct_us && split_us < ring_us) {
         note_conv_form(kSplitNames[split]);
-        return launch_split(split, BF16, Input, Weight, Output, M, C, K, nW, ep.scale, ep.shift, ep.residual, ep.residual_relu, s);
+        return launch_split(split, Input, Weight, Output, M, C, K, nW, ep.scale, ep.shift, ep.residual, ep.residual_relu, s);
     }
     if (direct != DIRECT_NONE) {
         note_conv_form(kDirectNames[direct]);

@@ -63,20 +63,23 @@ def test_direct_forms(oracle, forced, form, shape, precision):
     assert np.array_equal(ep, oracle.affine(got, scale, shift) + np.maximum(res, 0))
 
 
-@pytest.mark.parametrize("shape,want", [
-    ((1, 8, 8, 64, 64), "direct16x16"),       # 16 tiles of 16x16
-    ((5, 14, 16, 96, 72), "direct16x32"),     # 350 tiles of 16x16, 210 of 16x32
-    ((16, 7, 7, 256, 256), "direct16x64"),
-    ((16, 7, 7, 512, 512), "split32"),        # 200 tiles of 32x64, which the split form multiplies faster
-    ((64, 14, 14, 128, 64), "split64"),       # 196 tiles of 64x64
-    ((64, 28, 28, 64, 64), "whole"),          # 784: four rounds, the last nearly empty
+@pytest.mark.parametrize("shape,precision,want", [
+    ((1, 8, 8, 64, 64), "fp32", "direct16x16"),       # 16 tiles of 16x16
+    ((5, 14, 16, 96, 72), "fp32", "direct16x32"),     # 350 tiles of 16x16, 210 of 16x32
+    ((16, 7, 7, 256, 256), "fp32", "direct16x64"),
+    ((16, 7, 7, 512, 512), "fp32", "direct32x64"),    # 200 tiles of 32x64
+    ((64, 28, 28, 64, 64), "fp32", "whole"),          # 1568 of them
+    ((16, 7, 7, 512, 512), "bf16", "split32"),
+    ((64, 7, 7, 256, 256), "bf16", "split64"),        # 196 tiles of 64x64
+    ((64, 14, 14, 128, 128), "bf16", "whole"),        # 392
+    ((64, 14, 14, 32, 64), "bf16", "whole"),          # below 64 channels the ring takes less
 ])
-def test_the_launcher_picks_the_smallest_tile_that_needs_one_round(forced, shape, want):
+def test_the_launcher_picks_the_smallest_tile_that_needs_one_round(forced, shape, precision, want):
     from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv
     if torch.cuda.get_device_properties(0).multi_processor_count != 256:
         pytest.skip("the picks are those of 256 CUs")
     B, nH, nW, C, K = shape
-    winograd2x2_conv(torch.zeros((16, B, nH, nW, C), device="cuda"), torch.zeros((16, C, K), device="cuda"))
+    winograd2x2_conv(torch.zeros((16, B, nH, nW, C), device="cuda"), torch.zeros((16, C, K), device="cuda"), precision=precision)
     assert forced.swc_winograd2x2_conv_last_form().decode() == want
 
 
