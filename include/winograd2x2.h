@@ -286,8 +286,9 @@ SWC_API int swc_winograd2x2_pointwise_conv(const float *Input, const float *Weig
 /*
  * The model's first two layers in one kernel: Output [B,Hp,Wp,64] = 3x3 stride-2 max-pool of the 7x7 stride-2
  * convolution of Input [B,H,W,3] (NHWC) with Weight [64,3,7,7], both with TensorFlow's SAME padding
- * (ResNet-18-var/imagenet-resnet-transWino-prune.py:113-115); Hp = ceil(ceil(H/2)/2), Wp alike.  fp32; the products are
- * taken as three of pairs of f16 values.  Output 16-byte aligned (SWC_ERR_UNSUPPORTED otherwise).
+ * (ResNet-18-var/imagenet-resnet-transWino-prune.py:113-115); Hp = ceil(ceil(H/2)/2), Wp alike.  fp32: the products are
+ * taken of three bf16 pieces of each operand, which hold all its bits.  Output 16-byte aligned (SWC_ERR_UNSUPPORTED
+ * otherwise).
  */
 SWC_API int swc_stem_conv_pool(const float *Input, const float *Weight, float *Output, int B, int H, int W,
                                swc_stream_t stream);

@@ -25,10 +25,10 @@ def test_against_float64(shape, scale):
     got = resnet18_var.stem_conv_pool(image.cuda(), w.cuda()).cpu()
     want = expected(image.double(), w.double())
     assert got.shape == want.shape
-    # 147 products: fp32 sums of them in any order are within 147 half units of the sum of magnitudes, a product of
-    # split operands within 12 more; typical errors are far smaller, so the norm is held to 1e-6
+    # 147 products: fp32 sums of them in any order are within 147 half units of the sum of magnitudes, a product within one
+    # more; typical errors are far smaller, so the norm is held to 1e-6
     mag = expected_magnitude(image, w)
-    assert ((got - want).abs() <= (147 + 12 + 4) * 2.0 ** -24 * mag).all()
+    assert ((got - want).abs() <= (147 + 1 + 4) * 2.0 ** -24 * mag).all()
     assert (got - want).norm() <= 1e-6 * want.norm()
     ints = torch.randint(-8, 9, shape + (3,), generator=gen).float()
     wi = torch.randint(-4, 5, w.shape, generator=gen).float()
@@ -53,9 +53,53 @@ def test_values_that_do_not_split():
     assert torch.equal(got[inf], want[inf])
     ok = torch.isfinite(want)
     assert ((got - want)[ok].abs() <= 2 * 147 * 2.0 ** -24 * expected_magnitude(torch.nan_to_num(image, posinf=0.0), w)[ok]).all()
-    w[3] *= 1e-30                                            # a channel outside the scales' range
+    w[3] *= 1e-30                                            # a channel of tiny weights
     got, want = resnet18_var.stem_conv_pool(image[1:].cuda(), w.cuda()).cpu()[..., 3], expected(image[1:].double(), w.double())[..., 3]
     assert ((got - want).abs() <= 147 * 2.0 ** -24 * expected_magnitude(image[1:], w)[..., 3]).all()
+
+
+@pytest.mark.parametrize("bright", [24, 28, 34, 46, 60, 100])
+@pytest.mark.parametrize("positive", [False, True])
+def test_a_pixel_changes_only_what_sees_it(bright, positive):
+    """One value 2^bright times the others: every pooled pixel that does not see it comes out bit for bit as without it."""
+    import resnet18_var
+    gen = torch.Generator().manual_seed(83)
+    image, w = torch.randn((1, 90, 61, 3), generator=gen), torch.randn((64, 3, 7, 7), generator=gen) * 0.1
+    if positive:
+        image, w = image.abs(), w.abs()
+    seen = torch.zeros_like(image)
+    image[0, 40, 33, 1], seen[0, 40, 33, 1] = 0.0, 1.0
+    without = resnet18_var.stem_conv_pool(image.cuda(), w.cuda()).cpu()
+    image[0, 40, 33, 1] = 2.0 ** bright
+    got = resnet18_var.stem_conv_pool(image.cuda(), w.cuda()).cpu()
+    sees = expected(seen, torch.ones_like(w)) > 0
+    same = torch.equal(got[~sees], without[~sees])
+    assert same
+    assert (got != without)[sees].any()
+
+
+def test_all_24_bits_count_and_powers_of_two_commute():
+    import resnet18_var
+    gen = torch.Generator().manual_seed(84)
+    run = lambda image, w: resnet18_var.stem_conv_pool(image.cuda(), w.cuda()).cpu()   # noqa: E731
+    # single products: pixels far enough apart that a window holds one, one tap per channel
+    for image_bits, w_bits in ((24, 1), (1, 24), (12, 12)):
+        image, w = torch.zeros((1, 96, 96, 3)), torch.zeros((64, 3, 7, 7))
+        image[0, ::16, ::16, 1] = (torch.randint(2 ** (image_bits - 1), 2 ** image_bits, (6, 6), generator=gen) | 1).float()
+        w[:, 1, 3, 3] = (torch.randint(2 ** (w_bits - 1), 2 ** w_bits, (64,), generator=gen) | 1).float()
+        same = torch.equal(run(image, w), expected(image.double(), w.double()).float())
+        assert same, (image_bits, w_bits)
+    # tiles of any magnitude, channels of any magnitude
+    image, w = torch.randn((2, 64, 80, 3), generator=gen), torch.randn((64, 3, 7, 7), generator=gen)
+    plain = run(image, w)
+    for image_exp, w_exp in ((40, -60), (-60, 30), (0, -100), (-100, 60), (90, 20)):
+        wide = w.clone()
+        wide[5] *= 2.0 ** w_exp
+        got = run(image * 2.0 ** image_exp, wide)
+        want = plain * 2.0 ** image_exp
+        want[..., 5] *= 2.0 ** w_exp
+        same = torch.equal(got, want)
+        assert same, (image_exp, w_exp)
 
 
 def test_the_model_takes_it_and_the_library_path_agrees():
