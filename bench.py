@@ -52,10 +52,9 @@ MEASURED_TRAFFIC = {
 }
 
 
-def conv_ran(L, stored=False):
-    """The kernel of this thread's last convolution: the form over fp32 planes, or the tiling where it ran whole."""
-    form = "whole" if stored else L.swc_winograd2x2_conv_last_form().decode()
-    return L.swc_winograd2x2_conv_last_kernel().decode() if form == "whole" else form
+def conv_ran(L):
+    """The kernel of this thread's last convolution."""
+    return L.swc_winograd2x2_conv_last_kernel().decode()
 
 
 def measured_traffic(workload, precision, op, variant=None):
@@ -566,7 +565,7 @@ def main():
                          "mfma_TFLOPs": round(tf_conv, 2), "mfma_peak_TFLOPs": BF16_MFMA_PEAK_TF}
     if rotated is not None:
         conv_roofline["frac_rotated"] = round(conv_roofline["frac"] * ms_conv / rotated["ms_conv"], 4)
-    conv_variant = conv_ran(L, stored)
+    conv_variant = conv_ran(L)
     conv_roofline.update({"traffic": measured_traffic(name, args.precision, "conv", conv_variant), "kernel_variant": conv_variant,
                           "algorithmic_flop_per_launch": gemm_flops, "algorithmic_bytes_per_launch": conv_bytes})
 

@@ -41,26 +41,24 @@ SWC_API const char *swc_strerror(int status);
 SWC_API int swc_last_hip_error(void);
 /* Library version, "major.minor". */
 SWC_API const char *swc_version(void);
-/* Diagnostic with no counterpart in the reference: the convolution tiling that the calling
- * thread's last swc_winograd2x2_conv / _conv_bf16 / _conv_epilogue / _conv_bf16in / _conv_bf16in_ws call got ("" before the
- * first): "sync" (any shape and alignment), "ring32" / "ring16" (64x64 tiles, 32- / 16-channel steps),
+/* Diagnostic with no counterpart in the reference: the name of the convolution kernel that the calling
+ * thread's last swc_winograd2x2_conv / _conv_bf16 / _conv_epilogue / _conv_bf16in / _conv_bf16in_ws call launched ("" before the
+ * first): over fp32 planes "sync" (any shape and alignment), "ring32" / "ring16" (64x64 tiles, 32- / 16-channel steps),
  * "tall16" / "short16" (row groups of up to 112 / 32 rows, dealt evenly over the CUs), "wide48" (48 rows x 128
  * columns per workgroup, left-over rows as extra tiles split along the channels; C % 64 == 0, K % 128 == 0),
- * "wide48x64" (the same with 64 columns per workgroup; K % 64 == 0); for
+ * "wide48x64" (the same with 64 columns per workgroup; K % 64 == 0), or a form of swc_winograd2x2_conv_last_form(); for
  * bf16-stored operands "stored-ring3" / "stored-ring4" (64x64 tiles, 3- / 4-deep copy ring) / "stored-split"
  * (small grids: the 16 positions of a tile split over two groups of waves, whose partial sums are added at the
  * end) / "stored-split4" (smaller grids still: 32-row tiles, four groups of waves) / "stored-tall" (128x64
  * tiles for C = 64, 128, 256 or 512 on grids that fill the device) / "stored-spread" (the same tiles, four workgroups
- * each, on grids far too small for it; swc_winograd2x2_conv_bf16in_ws with a scratch buffer only).  For fp32 planes it names what the
- * shape rule assigns to one workgroup per tile; swc_winograd2x2_conv_last_form() says whether that ran or a form that
- * splits tiles further.  Which one runs
+ * each, on grids far too small for it; swc_winograd2x2_conv_bf16in_ws with a scratch buffer only).  Which one runs
  * depends only on the shapes, pointer alignment, whether a scratch buffer was passed, and the device's CU count and
  * L2 size; all give the same results to within the order of the fp32 summations ("wide48", "stored-tall" and
  * "stored-spread" also add the nine terms of an output in another order than the rest: 1e-6 relative, exact on
  * integer-valued data). */
 SWC_API const char *swc_winograd2x2_conv_last_kernel(void);
-/* Diagnostic with no counterpart in the reference: how that call ran over fp32 planes: "whole" (the tiling of
- * swc_winograd2x2_conv_last_kernel(), one workgroup per tile), or, on grids that leave most of the device idle that
+/* Diagnostic with no counterpart in the reference: how that call ran: "whole" (one workgroup per tile of one of the kernels
+ * above; bf16-stored operands always do), or over fp32 planes, on grids that leave most of the device idle that
  * way, "direct16x16" / "direct16x32" / "direct16x64" / "direct32x64": sixteen waves per workgroup, one per position,
  * each with the named tile of rows x columns (C % 4 == 0); or, with bf16 operands, "split32" / "split48" / "split64": tiles
  * of that many rows x 64 columns, the positions split over eight waves. */

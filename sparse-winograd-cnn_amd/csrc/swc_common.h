@@ -10,11 +10,9 @@ namespace swc {
 // Records a failed HIP call for swc_last_hip_error() and maps it to SWC_ERR_HIP.
 int note_hip_error(hipError_t e);
 
-// Records which convolution kernel a call chose, for swc_winograd2x2_conv_last_kernel().
-void note_conv_kernel(const char *name);
-
-// Records in which form it ran, for swc_winograd2x2_conv_last_form().
-void note_conv_form(const char *name);
+// Records which convolution kernel a call launches, for swc_winograd2x2_conv_last_kernel(), and in which form over fp32
+// planes, for swc_winograd2x2_conv_last_form().
+void note_conv_kernel(const char *name, const char *form = "whole");
 
 // The tiling set with swc_winograd2x2_conv_force_tiling() on this host thread, or nullptr.
 const char *forced_conv_tiling();

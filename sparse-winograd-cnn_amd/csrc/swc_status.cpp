@@ -14,9 +14,11 @@ thread_local char g_forced_tiling[16] = "";
 
 const char *forced_conv_tiling() { return g_forced_tiling[0] != '\0' ? g_forced_tiling : nullptr; }
 
-void note_conv_kernel(const char *name) { g_conv_kernel = name; }
-
-void note_conv_form(const char *name) { g_conv_form = name; }
+void note_conv_kernel(const char *name, const char *form)
+{
+    g_conv_kernel = name;
+    g_conv_form = form;
+}
 
 int note_hip_error(hipError_t e)
 {

@@ -76,22 +76,21 @@ int conv_entry(const float *Input, const float *Weight, float *Output, int C, in
     // two tiles in flight to cover the memory latency); fp32 picks among all of them.
     TilingChoice pick = {ring_eligible<Tile32>(Input, Weight, C, K, true) ? TILING_RING32 : TILING_SYNC, Tile32::BM};
     if (!BF16) pick = choose_tiling(Input, Weight, M, C, K, true, true);
-    note_conv_kernel(tiling_name(pick.tiling));
     double direct_us, split_us = 1e30;
     const DirectForm direct = choose_direct(Input, Weight, M, C, K, pick.tiling != TILING_SYNC, BF16, &direct_us);
     const SplitForm split = BF16 ? choose_split(Input, Weight, Output, ep.residual, M, C, K, &split_us) : SPLIT_NONE;
-    // The bf16-operand ring takes 6 us + 9 per 64 channels at best (one tile per CU); below 64 channels that is less than
+    // The bf16-operand ring takes 6 us + 9 per 64 channels at best (one tile per CU), which at 32 channels is as little as
     // the split forms' 6.5 to 8.5 + 4.1 to 5.  A direct form is offered only where it takes less than the ring.
     const double ring_us = pick.tiling == TILING_SYNC ? 1e30 : 6.0 + 9.0 * C / 64;
     if (split != SPLIT_NONE && split_us < direct_us && split_us < ring_us) {
-        note_conv_form(kSplitNames[split]);
+        note_conv_kernel(kSplitNames[split], kSplitNames[split]);
         return launch_split(split, Input, Weight, Output, M, C, K, nW, ep.scale, ep.shift, ep.residual, ep.residual_relu, s);
     }
     if (direct != DIRECT_NONE) {
-        note_conv_form(kDirectNames[direct]);
+        note_conv_kernel(kDirectNames[direct], kDirectNames[direct]);
         return launch_direct(direct, BF16, Input, Weight, Output, M, C, K, nW, ep.scale, ep.shift, ep.residual, ep.residual_relu, s);
     }
-    note_conv_form("whole");
+    note_conv_kernel(tiling_name(pick.tiling));
     switch (pick.tiling) {
         case TILING_WIDE48:
         case TILING_WIDE48X64:

@@ -50,7 +50,7 @@ def test_direct_forms(oracle, forced, form, shape, precision):
     dev = lambda a: torch.from_numpy(a).cuda()
     assert forced.swc_winograd2x2_conv_force_tiling(form.encode()) == 0
     got = winograd2x2_conv(dev(ti), dev(w), precision=precision).cpu().numpy()
-    assert forced.swc_winograd2x2_conv_last_form().decode() == form
+    assert forced.swc_winograd2x2_conv_last_form().decode() == forced.swc_winograd2x2_conv_last_kernel().decode() == form
     exact = winograd2x2_conv(dev(tii), dev(wi), precision=precision).cpu().numpy()
     ep = winograd2x2_conv(dev(ti), dev(w), precision=precision, scale=dev(scale), shift=dev(shift), residual=dev(res),
                           residual_relu=True).cpu().numpy()
@@ -97,3 +97,12 @@ def test_odd_columns_and_unaligned_weights_take_single_columns(oracle, forced):
         want = oracle.conv(ti, w, acc64=True)
         err = np.abs(tiles_of(got, 5, 9).astype(np.float64) - tiles_of(want, 5, 9))
         assert (err <= bound(ti, w)[:, None, :] + 2.0 ** -24 * np.abs(tiles_of(want, 5, 9))).all()
+
+
+def test_the_form_is_that_of_the_last_call(forced):
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv
+    ti, w = torch.zeros((16, 1, 8, 8, 64), device="cuda"), torch.zeros((16, 64, 64), device="cuda")
+    winograd2x2_conv(ti, w)
+    assert forced.swc_winograd2x2_conv_last_form() == forced.swc_winograd2x2_conv_last_kernel() == b"direct16x16"
+    winograd2x2_conv(ti.bfloat16(), w)
+    assert forced.swc_winograd2x2_conv_last_form() == b"whole" and forced.swc_winograd2x2_conv_last_kernel().startswith(b"stored-")

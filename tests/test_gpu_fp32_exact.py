@@ -13,9 +13,7 @@ SHAPES = [((1, 8, 8, 64, 64), "direct16x16"), ((16, 7, 7, 256, 256), "direct16x6
 
 def ran():
     import swc_hip
-    L = swc_hip.lib()
-    form = L.swc_winograd2x2_conv_last_form().decode()
-    return L.swc_winograd2x2_conv_last_kernel().decode() if form == "whole" else form
+    return swc_hip.lib().swc_winograd2x2_conv_last_kernel().decode()
 
 
 def conv(ti, w):

@@ -96,16 +96,22 @@ CONV_SHAPES = [
     (8, 7, 7, 256, 256),   # config 4a
     (8, 4, 4, 512, 512),   # config 4b
     (1, 2, 2, 1028, 12),
-    # shapes that steer the launcher onto each of its kernels and their ragged edges
-    (2, 3, 5, 64, 100),    # copy-ring kernel, 32-channel steps: rows and columns beyond the last tile
-    (1, 5, 7, 48, 20),     # copy-ring kernel, 16-channel steps (C % 32 != 0), K below one tile
-    (3, 7, 7, 32, 64),     # a single 32-channel step per position
+    # small grids (a wave per position) with ragged edges
+    (2, 3, 5, 64, 100),    # rows and columns beyond the last tile
+    (1, 5, 7, 48, 20),     # C % 32 != 0, K below one tile
+    (3, 7, 7, 32, 64),     # C below a block of 64 indices
     (2, 3, 3, 96, 132),    # K = 2 tiles + 4 columns
     (1, 1, 1, 32, 4),      # one tile row, one column group
-    (5, 9, 11, 160, 72),   # M = 495 (ragged last tile), C = 5 steps
-    (8, 9, 9, 128, 72),    # short row groups (16x16 MFMAs), ragged rows and columns
+    (5, 9, 11, 160, 72),   # M = 495 (ragged last tile)
+    (8, 9, 9, 128, 72),    # ragged rows and columns
+    # grids beyond the small forms: shapes that steer the launcher onto each of its other kernels
     (63, 14, 14, 128, 120),  # tall row groups of 97 rows, last one 29; K = 2 tiles - 8 columns
     (32, 28, 28, 64, 64),  # tall row groups, one 64-channel reduction in two steps
+    (18, 19, 24, 32, 32),  # copy ring, a single 32-channel step per position
+    (14, 31, 22, 48, 36),  # copy ring, 16-channel steps (C % 32 != 0), K below one tile
+    (41, 18, 12, 64, 32),  # short row groups (16x16 MFMAs), the last one ragged
+    (15, 12, 23, 64, 384),  # 48-row x 128-column groups
+    (15, 7, 10, 64, 512),  # 48-row x 64-column groups
 ]
 
 
@@ -134,19 +140,17 @@ def test_conv_fp32_matches_oracle(oracle, dev, shape):
 
 
 def test_conv_shapes_reach_every_kernel(dev):
-    # The launcher picks a kernel from the shapes alone; the parity shapes above must cover all five.
+    # The launcher picks a kernel from the shapes alone; the parity shapes above must cover all of them.
     import swc_hip
     _, conv = ops()
     seen = set()
-    # the last two: benchmark config 3, checked in full below, and config 4a's geometry (one 48-row x 64-column
-    # workgroup per CU of an MI355X), checked in full in test_gpu_cfg4_full.py
-    for shape in CONV_SHAPES + [(64, 14, 14, 128, 128), (64, 7, 7, 256, 256)]:
+    for shape in CONV_SHAPES:
         B, nH, nW, C, K = shape
         conv(torch.zeros((16, B, nH, nW, C), device=dev), torch.zeros((16, C, K), device=dev))
         seen.add(swc_hip.lib().swc_winograd2x2_conv_last_kernel().decode())
-    assert seen >= {"sync", "ring32", "ring16", "tall16", "short16", "wide48"}, seen
-    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
-        assert "wide48x64" in seen, seen
+    assert seen >= {"sync", "direct16x16"}, seen
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:   # where a grid is small depends on the CUs
+        assert seen >= {"ring32", "ring16", "tall16", "short16", "wide48", "wide48x64", "direct16x32", "direct16x64"}, seen
 
 
 @pytest.mark.parametrize("tiling", ["ring32", "ring16", "tall16", "short16", "sync"])
@@ -168,7 +172,10 @@ def test_conv_fp32_under_every_tiling(oracle, dev, shape, tiling):
     finally:
         assert L.swc_winograd2x2_conv_force_tiling(None) == 0
     conv(gpu(ti, dev), gpu(w, dev))
-    assert L.swc_winograd2x2_conv_last_kernel().decode() in ("ring32", "ring16", "tall16", "short16")
+    B, nH, nW, C, K = shape
+    small = -(-B * nH * nW // 32) * -(-K // 64) <= torch.cuda.get_device_properties(dev).multi_processor_count
+    assert L.swc_winograd2x2_conv_last_kernel().decode().startswith("direct") if small else \
+        L.swc_winograd2x2_conv_last_kernel().decode() in ("ring32", "ring16", "tall16", "short16")
 
 
 # wide48 takes C % 64 == 0 and K % 128 == 0.  The shapes cover its two ways of dealing out the rows: levelled row
