@@ -124,15 +124,29 @@ def stem_conv_pool(image, w):
     return out
 
 
+def _observed(conv):
+    """Whether somebody sees or replaces the call of ``conv``: hooks on it or on every module, a forward of its own, a
+    dispatch mode."""
+    every = torch.nn.modules.module
+    own = vars(conv)
+    return (conv._forward_hooks or conv._forward_pre_hooks or every._global_forward_hooks or every._global_forward_pre_hooks
+            or "forward" in own or "_conv_forward" in own or own.get("_compiled_call_impl") is not None
+            or torch._C._len_torch_dispatch_stack() > 0)
+
+
 def _is_stem(conv, image):
     """Whether ``stem_conv_pool`` computes what calling ``conv`` (padded SAME) and pooling does: the layer as the model
-    builds it, nothing hooked onto it, fp32 on one GPU."""
+    builds it, nothing watching its call, fp32 on one GPU, an image of the sizes the kernel takes."""
+    if not (type(conv) is torch.nn.Conv2d and type(image) is torch.Tensor) or _observed(conv):
+        return False
     w = conv.weight
-    return (type(conv) is torch.nn.Conv2d and w.shape == (64, 3, 7, 7) and conv.bias is None
-            and conv.stride == (2, 2) and conv.padding == (0, 0) and conv.dilation == (1, 1) and conv.groups == 1
-            and not (conv._forward_hooks or conv._forward_pre_hooks) and not torch.is_autocast_enabled()
-            and type(image) is torch.Tensor and image.is_cuda and image.device == w.device and image.dim() == 4
-            and image.shape[3] == 3 and image.dtype == torch.float32 and w.dtype == torch.float32 and image.numel() > 0)
+    if not (w.shape == (64, 3, 7, 7) and conv.bias is None and conv.stride == (2, 2) and conv.padding == (0, 0)
+            and conv.dilation == (1, 1) and conv.groups == 1 and not torch.is_autocast_enabled()
+            and image.is_cuda and image.device == w.device and image.dim() == 4 and image.shape[3] == 3
+            and image.dtype == torch.float32 and w.dtype == torch.float32 and not (image.is_neg() or w.is_neg())):
+        return False
+    B, H, W, _ = image.shape
+    return image.numel() > 0 and max(H, W) < 1 << 20 and H * W < 1 << 29 and B * -(-H // 28) * -(-W // 28) < 1 << 31
 
 
 def _to_nhwc(x):   # NCHW tensor in channels_last memory -> contiguous [B,H,W,C] view

@@ -116,3 +116,44 @@ def test_the_model_takes_it_and_the_library_path_agrees():
     plain = model(image)
     assert seen and torch.equal(strided, fused)
     assert (fused - plain).norm() <= 2e-6 * plain.norm()     # two fp32 sums of 147 products, through eight units
+
+
+def test_whoever_watches_or_replaces_conv1_still_does():
+    import resnet18_var
+    from torch.utils.flop_counter import FlopCounterMode
+    torch.manual_seed(3)
+    model = resnet18_var.ResNet18Var().cuda()
+    image = torch.randn((1, 32, 32, 3), device="cuda")
+    seen = []
+    watch = lambda m, i, *o: seen.append(m)   # noqa: E731
+    for register in (torch.nn.modules.module.register_module_forward_hook, torch.nn.modules.module.register_module_forward_pre_hook,
+                     model.conv1.register_forward_hook, model.conv1.register_forward_pre_hook):
+        handle = register(watch)
+        model(image)
+        handle.remove()
+        assert model.conv1 in seen, register
+        del seen[:]
+    own = model.conv1.forward
+    model.conv1.forward = lambda x: (seen.append(model.conv1), own(x))[1]
+    model(image)
+    assert seen
+    del model.conv1.forward
+    counter = FlopCounterMode(display=False)
+    with counter:
+        model(image)
+    assert counter.get_total_flops() >= 2 * 16 * 16 * 147 * 64
+    assert resnet18_var._is_stem(model.conv1, image)
+
+
+def test_images_the_kernel_does_not_take_go_to_the_layers():
+    import resnet18_var
+    import swc_hip
+    model = resnet18_var.ResNet18Var().cuda()
+    w = model.conv1.weight
+    for H, W in ((1 << 20, 1), (1, 1 << 20)):
+        image = torch.zeros((1, H, W, 3), device="cuda")
+        assert not resnet18_var._is_stem(model.conv1, image)
+        with pytest.raises(swc_hip.SwcError):
+            resnet18_var.stem_conv_pool(image, w)
+    image = torch.complex(torch.zeros(1, 32, 32, 3), torch.randn(1, 32, 32, 3)).cuda().conj().imag   # negated lazily
+    assert image.is_neg() and not resnet18_var._is_stem(model.conv1, image)
