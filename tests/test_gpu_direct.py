@@ -54,6 +54,14 @@ def test_direct_forms(oracle, forced, form, shape, precision):
     exact = winograd2x2_conv(dev(tii), dev(wi), precision=precision).cpu().numpy()
     ep = winograd2x2_conv(dev(ti), dev(w), precision=precision, scale=dev(scale), shift=dev(shift), residual=dev(res),
                           residual_relu=True).cpu().numpy()
+    buf = dev(res)
+    winograd2x2_conv(dev(ti), dev(w), precision=precision, out=buf, residual=buf)   # residual aliasing the output
+    off = torch.zeros(2 * res.size + 2, device="cuda")                              # output and residual 4 bytes past a line
+    out, shifted = off[1:1 + res.size].view(res.shape), off[1 + res.size:1 + 2 * res.size].view(res.shape)
+    shifted.copy_(dev(res))
+    winograd2x2_conv(dev(ti), dev(w), precision=precision, out=out, residual=shifted)
+    assert forced.swc_winograd2x2_conv_last_form().decode() == form
+    assert np.array_equal(buf.cpu().numpy(), got + res) and np.array_equal(out.cpu().numpy(), got + res)
     if precision == "bf16":
         ti, w = oracle.round_bf16(ti), oracle.round_bf16(w)
     want = oracle.conv(ti, w, acc64=True)

@@ -69,3 +69,20 @@ def test_forced_on_fp32_operands_they_are_refused(forced):  # noqa: F811
     assert forced.swc_winograd2x2_conv_force_tiling(b"split64") == 0
     winograd2x2_conv(ti, w)
     assert forced.swc_winograd2x2_conv_last_form() == b"whole" and forced.swc_winograd2x2_conv_last_kernel() == b"sync"
+
+
+def test_unaligned_output_or_residual_takes_another_kernel(forced):  # noqa: F811
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv
+    gen = torch.Generator(device="cuda").manual_seed(77)
+    ti, w = torch.randn((16, 16, 7, 7, 512), device="cuda", generator=gen), torch.randn((16, 512, 512), device="cuda", generator=gen)
+    want = winograd2x2_conv(ti, w, precision="bf16")
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert forced.swc_winograd2x2_conv_last_form() == b"split32"
+    n = want.numel()
+    off = torch.zeros(2 * n + 2, device="cuda")
+    out, res = off[1:1 + n].view(want.shape), off[1 + n:1 + 2 * n].view(want.shape)
+    for kw in ({"out": out}, {"residual": res}):
+        got = winograd2x2_conv(ti, w, precision="bf16", **kw)
+        assert not forced.swc_winograd2x2_conv_last_form().startswith(b"split")
+        # fp32 sums of the same 512 products and nine terms in another order
+        assert (got - want).norm() <= 1e-5 * want.norm()
