@@ -77,7 +77,7 @@ int conv_entry(const float *Input, const float *Weight, float *Output, int C, in
     TilingChoice pick = {ring_eligible<Tile32>(Input, Weight, C, K, true) ? TILING_RING32 : TILING_SYNC, Tile32::BM};
     if (!BF16) pick = choose_tiling(Input, Weight, M, C, K, true, true);
     double direct_us, split_us = 1e30;
-    const DirectForm direct = choose_direct(Input, Weight, M, C, K, pick.tiling != TILING_SYNC, BF16, &direct_us);
+    const DirectForm direct = choose_direct(Input, Weight, M, C, K, pick.tiling != TILING_SYNC, pick.tiling == TILING_SHORT16, BF16, &direct_us);
     const SplitForm split = BF16 ? choose_split(Input, Weight, Output, ep.residual, M, C, K, &split_us) : SPLIT_NONE;
     // The bf16-operand ring takes 6 us + 9 per 64 channels at best (one tile per CU), which at 32 channels is as little as
     // the split forms' 6.5 to 8.5 + 4.1 to 5.  A direct form is offered only where it takes less than the ring.

@@ -47,10 +47,13 @@ static bool direct_eligible(const void *TI, size_t M, int C, int K)
 // 32x64 (with bf16 operands 3 + 2.3, 3.2 + 3.5, 3.6 + 3.6, 5 + 5.2), so the smallest tile that needs one round wins.
 // The ring kernels take 4.3 + 8.9 us per 64 channels at best (bf16 6 + 9) and hold that up to one 64x64 tile per CU:
 // beyond one round of 32x64 tiles they are as fast or faster (784x64->64: 13.4 -> 5.7 us; 49x512->512: 75.6 -> 22.3;
-// 784x256->256: 41.6 -> 24.8; 1024x512->512: 77.6 -> 73.0; 6272x64->64: 14.2 against 14.7).  Where only the
+// 784x256->256: 41.6 -> 24.8; 1024x512->512: 76.3 -> 74.8).  short16 deals out the same 32x64 tiles at four waves each and
+// two or three to a CU; below 256 channels it is the faster one (1024 to 8192 rows, 64 channels: 13.3 to 14.8 us against
+// 14.5 to 15.9; 128: 22.5 to 24.2 against 22.7 to 25.2; 192: 32.0 against 32.5; 256: 41.0 against 40.8), while ring32, which takes
+// the other channel counts, is not (96 channels: 31 against 20).  Where only the
 // synchronous kernel could run (44 us for 104x72->48, 6.6 here) every round is worth it, except that single columns
 // (K % 4 != 0 or W unaligned) come in 16x16 tiles only.
-DirectForm choose_direct(const void *TI, const void *Wt, size_t M, int C, int K, bool ring, bool bf16, double *us)
+DirectForm choose_direct(const void *TI, const void *Wt, size_t M, int C, int K, bool ring, bool short16, bool bf16, double *us)
 {
     *us = 1e30;
     if (!direct_eligible(TI, M, C, K)) return DIRECT_NONE;
@@ -71,6 +74,7 @@ DirectForm choose_direct(const void *TI, const void *Wt, size_t M, int C, int K,
         const size_t wgs = (M + kForms[i].rows - 1) / kForms[i].rows * ((K + kForms[i].cols - 1) / kForms[i].cols);
         const size_t rounds = (wgs + cus - 1) / cus;
         if (rounds > (ring ? 1 : wide ? ~size_t(0) : 4)) continue;
+        if (i == DIRECT_32X64 && short16 && C < 256) continue;
         const double this_us = rounds * (kForms[i].base[bf16] + kForms[i].per64[bf16] * C / 64);
         if (this_us < *us) {
             *us = this_us;

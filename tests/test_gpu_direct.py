@@ -76,6 +76,8 @@ def test_direct_forms(oracle, forced, form, shape, precision):
     ((5, 14, 16, 96, 72), "fp32", "direct16x32"),     # 350 tiles of 16x16, 210 of 16x32
     ((16, 7, 7, 256, 256), "fp32", "direct16x64"),
     ((16, 7, 7, 512, 512), "fp32", "direct32x64"),    # 200 tiles of 32x64
+    ((16, 14, 14, 128, 128), "fp32", "whole"),        # 196, but short16 is faster below 256 channels
+    ((16, 14, 14, 96, 128), "fp32", "direct32x64"),   # and takes multiples of 64 only
     ((64, 28, 28, 64, 64), "fp32", "whole"),          # 1568 of them
     ((16, 7, 7, 512, 512), "bf16", "split32"),
     ((64, 7, 7, 256, 256), "bf16", "split64"),        # 196 tiles of 64x64

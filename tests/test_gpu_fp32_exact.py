@@ -6,8 +6,8 @@ import torch
 pytestmark = pytest.mark.gpu
 
 # (B, nH, nW, C, K) and what runs on 256 CUs
-SHAPES = [((1, 8, 8, 64, 64), "direct16x16"), ((16, 7, 7, 256, 256), "direct16x64"), ((16, 14, 14, 128, 128), "direct32x64"),
-          ((40, 14, 14, 96, 128), "ring32"), ((64, 14, 14, 48, 64), "ring16"), ((32, 28, 28, 64, 64), "tall16"),
+SHAPES = [((1, 8, 8, 64, 64), "direct16x16"), ((16, 7, 7, 256, 256), "direct16x64"), ((16, 7, 7, 512, 512), "direct32x64"),
+          ((16, 14, 14, 128, 128), "short16"), ((40, 14, 14, 96, 128), "ring32"), ((64, 14, 14, 48, 64), "ring16"), ((32, 28, 28, 64, 64), "tall16"),
           ((64, 14, 14, 128, 128), "wide48"), ((64, 7, 7, 256, 256), "wide48x64"), ((2, 4, 4, 5, 7), "sync")]
 
 
