@@ -236,7 +236,8 @@ SWEEP_SHAPES = [(("N%d %dx%d %d->%d" % (n, hw, hw, c, k)), n, hw, c, k)
     ("N4 56x56 256->64", 4, 56, 256, 64), ("N100 10x10 320->160", 100, 10, 320, 160),
     ("N24 28x28 96->192", 24, 28, 96, 192), ("N12 14x14 1024->256", 12, 14, 1024, 256), ("N200 8x8 64->320", 200, 8, 64, 320),
     ("N2 224x224 32->64", 2, 224, 32, 64), ("N64 12x12 384->384", 64, 12, 384, 384)]
-TILINGS = ("ring32", "ring16", "tall16", "short16", "wide48", "wide48x64", "direct16x16", "direct16x32", "direct16x64", "direct32x64")
+TILINGS = ("ring32", "ring16", "tall16", "short16", "wide48", "wide48x64", "direct16x16", "direct16x32", "direct16x64", "direct32x64",
+           "split32", "split48", "split64", "split64+32", "split64+48")
 
 
 def bench_sweep(args, torch, dev):
@@ -552,8 +553,11 @@ def main():
     gbs_imtrans = imtrans_bytes / (ms_imtrans * 1e-3) / 1e9
     gbs_conv = conv_bytes / (ms_conv * 1e-3) / 1e9
     if args.precision == "fp32":
-        # fp32 MFMA bounds the contraction (arithmetic intensity 51 flop/B at conv3, ridge 19.7)
-        conv_roofline = {"kernel": "winograd2x2_conv (16 GEMMs + fused A^T m A), fp32 MFMA, tiling %s" % conv_ran(L), "bound": "mfma",
+        # fp32 MFMA bounds the contraction (arithmetic intensity 51 flop/B at conv3, ridge 19.7); the split forms take six
+        # bf16 products for one fp32 product and are held against the same peak
+        ran = conv_ran(L)
+        conv_roofline = {"kernel": "winograd2x2_conv (16 GEMMs + fused A^T m A), fp32 %s %s"
+                                   % ("in bf16 pieces," if ran.startswith("split") else "MFMA, tiling", ran), "bound": "mfma",
                          "achieved": round(tf_conv, 2), "peak": FP32_MFMA_PEAK_TF, "unit": "TFLOP/s",
                          "frac": round(tf_conv / FP32_MFMA_PEAK_TF, 4)}
     else:

@@ -60,8 +60,11 @@ SWC_API const char *swc_winograd2x2_conv_last_kernel(void);
 /* Diagnostic with no counterpart in the reference: how that call ran: "whole" (one workgroup per tile of one of the kernels
  * above; bf16-stored operands always do), or over fp32 planes, on grids that leave most of the device idle that
  * way, "direct16x16" / "direct16x32" / "direct16x64" / "direct32x64": sixteen waves per workgroup, one per position,
- * each with the named tile of rows x columns (C % 4 == 0); or, with bf16 operands, "split32" / "split48" / "split64": tiles
- * of that many rows x 64 columns, the positions split over eight waves. */
+ * each with the named tile of rows x columns (C % 4 == 0); or "split32" / "split48" / "split64" / "split64+32" /
+ * "split64+48" (whole rounds of 64-row tiles, the rest in lower ones): tiles of that many rows x 64 columns, the positions
+ * split over eight waves, on the 16-bit matrix instructions: fp32 operands in three bf16 pieces each, which hold all their
+ * bits (nearer to float64 than the fp32 instructions; a tile with operands above 2^30 or sums below 2^-75 is multiplied
+ * with those, operands below 2^-134 count as zero), or bf16 operands. */
 SWC_API const char *swc_winograd2x2_conv_last_form(void);
 /* Diagnostic with no counterpart in the reference, for benchmarks and tests that compare the tilings: makes
  * the calling thread's later swc_winograd2x2_conv calls

@@ -76,15 +76,19 @@ int conv_entry(const float *Input, const float *Weight, float *Output, int C, in
     // two tiles in flight to cover the memory latency); fp32 picks among all of them.
     TilingChoice pick = {ring_eligible<Tile32>(Input, Weight, C, K, true) ? TILING_RING32 : TILING_SYNC, Tile32::BM};
     if (!BF16) pick = choose_tiling(Input, Weight, M, C, K, true, true);
-    double direct_us, split_us = 1e30;
+    double direct_us;
     const DirectForm direct = choose_direct(Input, Weight, M, C, K, pick.tiling != TILING_SYNC, pick.tiling == TILING_SHORT16, BF16, &direct_us);
-    const SplitForm split = BF16 ? choose_split(Input, Weight, Output, ep.residual, M, C, K, &split_us) : SPLIT_NONE;
-    // The bf16-operand ring takes 6 us + 9 per 64 channels at best (one tile per CU), which at 32 channels is as little as
-    // the split forms' 6.5 to 8.5 + 4.1 to 5.  A direct form is offered only where it takes less than the ring.
-    const double ring_us = pick.tiling == TILING_SYNC ? 1e30 : 6.0 + 9.0 * C / 64;
-    if (split != SPLIT_NONE && split_us < direct_us && split_us < ring_us) {
-        note_conv_kernel(kSplitNames[split], kSplitNames[split]);
-        return launch_split(split, Input, Weight, Output, M, C, K, nW, ep.scale, ep.shift, ep.residual, ep.residual_relu, s);
+    const SplitChoice split = choose_split(Input, Weight, Output, ep.residual, M, C, K, BF16);
+    // What the ring and wide kernels take.  fp32: 6 us + 3.75 per unit of their cost and 64 channels; over 230 shapes the
+    // measured time was 0.95 to 1.4 times that (median 1.1), with the wide tilings 0.88 to 1.08, which therefore count for a
+    // tenth less.  bf16 operands: 6 us + 9 per 64 channels at best (one tile per CU), at 32 channels as little as the split
+    // forms' 6.5 to 8.5 + 4.1 to 5.  A direct form is offered only where it takes less.
+    const double per64 = static_cast<double>(C) / 64;
+    const double scale = pick.tiling == TILING_WIDE48 || pick.tiling == TILING_WIDE48X64 ? 0.9 : 1.0;
+    const double whole_us = pick.tiling == TILING_SYNC ? 1e30 : BF16 ? 6.0 + 9.0 * per64 : scale * (6.0 + 3.75 * pick.cost * per64);
+    if (split.form != SPLIT_NONE && split.us < direct_us && split.us < whole_us) {
+        note_conv_kernel(kSplitNames[split.form], kSplitNames[split.form]);
+        return launch_split(split, BF16, Input, Weight, Output, M, C, K, nW, ep.scale, ep.shift, ep.residual, ep.residual_relu, s);
     }
     if (direct != DIRECT_NONE) {
         note_conv_kernel(kDirectNames[direct], kDirectNames[direct]);

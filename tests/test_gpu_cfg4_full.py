@@ -43,10 +43,9 @@ def test_config4_full_size(oracle, layer):
     assert got.shape == want.shape == (N, 2 * nT, 2 * nT, K)
     assert rel_max(got, want) <= TOL and rel_l1(got, want) <= TOL
     if cus == 256:
-        # the tiling follows from the CU count: on an MI355X 32-row x 64-column tiles of sixteen waves make one round over
-        # the CUs at config 4b; at config 4a one 48-row x 64-column workgroup per CU does (64 of them carry one of the
-        # 16 tiles of the 64 left-over rows)
-        assert L.swc_winograd2x2_conv_last_kernel() == (b"wide48x64" if name == "4a" else b"direct32x64")
+        # the tiling follows from the CU count: on an MI355X 64-row x 64-column tiles make one round over the CUs at
+        # config 4a, 32-row ones at config 4b
+        assert L.swc_winograd2x2_conv_last_kernel() == (b"split64" if name == "4a" else b"split32")
 
     # bf16 operands, fp32 planes: against the oracle fed the same rounded operands
     want16 = oracle.conv(oracle.round_bf16(ti_want), oracle.round_bf16(w), acc64=True)

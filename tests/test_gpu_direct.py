@@ -75,10 +75,13 @@ def test_direct_forms(oracle, forced, form, shape, precision):
     ((1, 8, 8, 64, 64), "fp32", "direct16x16"),       # 16 tiles of 16x16
     ((5, 14, 16, 96, 72), "fp32", "direct16x32"),     # 350 tiles of 16x16, 210 of 16x32
     ((16, 7, 7, 256, 256), "fp32", "direct16x64"),
-    ((16, 7, 7, 512, 512), "fp32", "direct32x64"),    # 200 tiles of 32x64
-    ((16, 14, 14, 128, 128), "fp32", "whole"),        # 196, but short16 is faster below 256 channels
-    ((16, 14, 14, 96, 128), "fp32", "direct32x64"),   # and takes multiples of 64 only
-    ((64, 28, 28, 64, 64), "fp32", "whole"),          # 1568 of them
+    ((63, 14, 14, 36, 120), "fp32", "direct32x64"),   # below 64 channels
+    ((16, 7, 7, 512, 512), "fp32", "split32"),        # 200 tiles of 32x64
+    ((64, 14, 14, 128, 64), "fp32", "split64"),       # 196 tiles of 64x64
+    ((128, 7, 7, 256, 256), "fp32", "split64+48"),    # 392: one round, the rest in 184 lower ones
+    ((49, 30, 27, 96, 36), "fp32", "split64+32"),     # 621: two rounds, and 6922 rows in lower tiles
+    ((64, 14, 14, 128, 128), "fp32", "whole"),        # 392 too, but 128 channels: wide48 is as fast
+    ((64, 28, 28, 64, 64), "fp32", "whole"),          # 64 channels and more than a round
     ((16, 7, 7, 512, 512), "bf16", "split32"),
     ((64, 7, 7, 256, 256), "bf16", "split64"),        # 196 tiles of 64x64
     ((64, 14, 14, 128, 128), "bf16", "whole"),        # 392
@@ -89,7 +92,7 @@ def test_the_launcher_picks_the_smallest_tile_that_needs_one_round(forced, shape
     if torch.cuda.get_device_properties(0).multi_processor_count != 256:
         pytest.skip("the picks are those of 256 CUs")
     B, nH, nW, C, K = shape
-    winograd2x2_conv(torch.zeros((16, B, nH, nW, C), device="cuda"), torch.zeros((16, C, K), device="cuda"), precision=precision)
+    winograd2x2_conv(torch.ones((16, B, nH, nW, C), device="cuda"), torch.ones((16, C, K), device="cuda"), precision=precision)
     assert forced.swc_winograd2x2_conv_last_form().decode() == want
 
 

@@ -6,9 +6,11 @@ import torch
 pytestmark = pytest.mark.gpu
 
 # (B, nH, nW, C, K) and what runs on 256 CUs
-SHAPES = [((1, 8, 8, 64, 64), "direct16x16"), ((16, 7, 7, 256, 256), "direct16x64"), ((16, 7, 7, 512, 512), "direct32x64"),
-          ((16, 14, 14, 128, 128), "short16"), ((40, 14, 14, 96, 128), "ring32"), ((64, 14, 14, 48, 64), "ring16"), ((32, 28, 28, 64, 64), "tall16"),
-          ((64, 14, 14, 128, 128), "wide48"), ((64, 7, 7, 256, 256), "wide48x64"), ((2, 4, 4, 5, 7), "sync")]
+SHAPES = [((1, 8, 8, 64, 64), "direct16x16"), ((16, 7, 7, 256, 256), "direct16x64"), ((63, 14, 14, 36, 120), "direct32x64"),
+          ((18, 19, 24, 32, 32), "ring32"), ((64, 14, 14, 48, 64), "ring16"), ((32, 28, 28, 64, 64), "tall16"),
+          ((96, 22, 8, 64, 32), "short16"), ((15, 12, 23, 64, 384), "wide48"), ((64, 14, 14, 64, 64), "wide48x64"),
+          ((16, 7, 7, 512, 512), "split32"), ((41, 18, 12, 64, 32), "split48"), ((64, 7, 7, 256, 256), "split64"),
+          ((49, 30, 27, 96, 36), "split64+32"), ((128, 7, 7, 256, 256), "split64+48"), ((2, 4, 4, 5, 7), "sync")]
 
 
 def ran():
@@ -25,7 +27,8 @@ def conv(ti, w):
 @pytest.mark.parametrize("positive", [False, True])
 def test_scaling_by_powers_of_two_commutes(shape, kernel, positive):
     """Rows of TI and columns of W down to 2^-50 of the others beside them, and channels whose activations and weights
-    compensate each other: each product and sum is the unscaled one times a power of two, so nothing may round differently."""
+    compensate each other: each product and sum is the unscaled one times a power of two, so nothing may round differently.
+    (Over 2^30 the split forms multiply with the fp32 instructions, whose sums are those of the direct form.)"""
     B, nH, nW, C, K = shape
     gen = torch.Generator(device="cuda").manual_seed(75)
     ti = torch.randn((16, B, nH, nW, C), device="cuda", generator=gen)
@@ -43,9 +46,20 @@ def test_scaling_by_powers_of_two_commutes(shape, kernel, positive):
     by_rows = torch.equal(conv(ti * rows.reshape(1, B, nH, nW, 1), w), plain * by_pixel)
     cols = pick(K).float()
     by_columns = torch.equal(conv(ti, w * cols), plain * cols)
-    channels = (2.0 ** (torch.arange(C, device="cuda") * 7 % 81 - 40).double()).float()
+    wide = torch.arange(C, device="cuda") * 7 % 81 - 40
+    channels = (2.0 ** (wide / 2).round().double()).float()
     by_channels = torch.equal(conv(ti * channels, w / channels.reshape(C, 1)), plain)
-    assert by_rows and by_columns and by_channels, (by_rows, by_columns, by_channels)
+    channels = (2.0 ** wide.double()).float()
+    far = conv(ti * channels, w / channels.reshape(C, 1))
+    if got_kernel.startswith("split"):
+        import swc_hip
+        assert swc_hip.lib().swc_winograd2x2_conv_force_tiling(b"direct32x64") == 0
+        try:
+            plain = conv(ti, w)
+        finally:
+            assert swc_hip.lib().swc_winograd2x2_conv_force_tiling(None) == 0
+    by_channels_far = torch.equal(far, plain)
+    assert by_rows and by_columns and by_channels and by_channels_far, (by_rows, by_columns, by_channels, by_channels_far)
     if torch.cuda.get_device_properties(0).multi_processor_count == 256:
         assert got_kernel == kernel
 

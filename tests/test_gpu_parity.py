@@ -105,13 +105,14 @@ CONV_SHAPES = [
     (5, 9, 11, 160, 72),   # M = 495 (ragged last tile)
     (8, 9, 9, 128, 72),    # ragged rows and columns
     # grids beyond the small forms: shapes that steer the launcher onto each of its other kernels
-    (63, 14, 14, 128, 120),  # tall row groups of 97 rows, last one 29; K = 2 tiles - 8 columns
+    (63, 14, 14, 128, 120),  # 64-row tiles and 48-row ones behind them; K = 2 tiles - 8 columns
     (32, 28, 28, 64, 64),  # tall row groups, one 64-channel reduction in two steps
     (18, 19, 24, 32, 32),  # copy ring, a single 32-channel step per position
     (14, 31, 22, 48, 36),  # copy ring, 16-channel steps (C % 32 != 0), K below one tile
-    (41, 18, 12, 64, 32),  # short row groups (16x16 MFMAs), the last one ragged
+    (70, 20, 6, 64, 72),   # short row groups (16x16 MFMAs), ragged rows and columns
     (15, 12, 23, 64, 384),  # 48-row x 128-column groups
-    (15, 7, 10, 64, 512),  # 48-row x 64-column groups
+    (64, 14, 14, 64, 64),  # 48-row x 64-column groups
+    (41, 18, 12, 64, 32),  # 48-row tiles, positions split over eight waves
 ]
 
 
@@ -150,7 +151,8 @@ def test_conv_shapes_reach_every_kernel(dev):
         seen.add(swc_hip.lib().swc_winograd2x2_conv_last_kernel().decode())
     assert seen >= {"sync", "direct16x16"}, seen
     if torch.cuda.get_device_properties(dev).multi_processor_count == 256:   # where a grid is small depends on the CUs
-        assert seen >= {"ring32", "ring16", "tall16", "short16", "wide48", "wide48x64", "direct16x32", "direct16x64"}, seen
+        assert seen >= {"ring32", "ring16", "tall16", "short16", "wide48", "wide48x64", "direct16x32", "direct16x64",
+                        "split48", "split64+48"}, seen
 
 
 @pytest.mark.parametrize("tiling", ["ring32", "ring16", "tall16", "short16", "sync"])
@@ -174,8 +176,8 @@ def test_conv_fp32_under_every_tiling(oracle, dev, shape, tiling):
     conv(gpu(ti, dev), gpu(w, dev))
     B, nH, nW, C, K = shape
     small = -(-B * nH * nW // 32) * -(-K // 64) <= torch.cuda.get_device_properties(dev).multi_processor_count
-    assert L.swc_winograd2x2_conv_last_kernel().decode().startswith("direct") if small else \
-        L.swc_winograd2x2_conv_last_kernel().decode() in ("ring32", "ring16", "tall16", "short16")
+    picked = L.swc_winograd2x2_conv_last_kernel().decode()
+    assert picked.startswith(("direct", "split")) if small else picked in ("ring32", "ring16", "tall16", "short16", "split64", "split64+48")
 
 
 # wide48 takes C % 64 == 0 and K % 128 == 0.  The shapes cover its two ways of dealing out the rows: levelled row
