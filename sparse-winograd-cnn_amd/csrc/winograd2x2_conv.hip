@@ -81,10 +81,11 @@ int conv_entry(const float *Input, const float *Weight, float *Output, int C, in
     const SplitChoice split = choose_split(Input, Weight, Output, ep.residual, M, C, K, BF16);
     // What the ring and wide kernels take.  fp32: 6 us + 3.75 per unit of their cost and 64 channels; over 230 shapes the
     // measured time was 0.95 to 1.4 times that (median 1.1), with the wide tilings 0.88 to 1.08, which therefore count for a
-    // tenth less.  bf16 operands: 6 us + 9 per 64 channels at best (one tile per CU), at 32 channels as little as the split
+    // tenth less, and up to 128 channels, where several rounds of a split form take up to 6 % longer than they are taken to
+    // (39572x128->64 101.5 us against 95.6), for 15 %.  bf16 operands: 6 us + 9 per 64 channels at best (one tile per CU), at 32 channels as little as the split
     // forms' 6.5 to 8.5 + 4.1 to 5.  A direct form is offered only where it takes less.
     const double per64 = static_cast<double>(C) / 64;
-    const double scale = pick.tiling == TILING_WIDE48 || pick.tiling == TILING_WIDE48X64 ? 0.9 : 1.0;
+    const double scale = pick.tiling != TILING_WIDE48 && pick.tiling != TILING_WIDE48X64 ? 1.0 : C > 128 ? 0.9 : 0.85;
     const double whole_us = pick.tiling == TILING_SYNC ? 1e30 : BF16 ? 6.0 + 9.0 * per64 : scale * (6.0 + 3.75 * pick.cost * per64);
     if (split.form != SPLIT_NONE && split.us < direct_us && split.us < whole_us) {
         note_conv_kernel(kSplitNames[split.form], kSplitNames[split.form]);

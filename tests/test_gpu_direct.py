@@ -77,7 +77,7 @@ def test_direct_forms(oracle, forced, form, shape, precision):
     ((16, 7, 7, 256, 256), "fp32", "direct16x64"),
     ((63, 14, 14, 36, 120), "fp32", "direct32x64"),   # below 64 channels
     ((16, 7, 7, 512, 512), "fp32", "split32"),        # 200 tiles of 32x64
-    ((64, 14, 14, 128, 64), "fp32", "split64"),       # 196 tiles of 64x64
+    ((64, 7, 7, 256, 256), "fp32", "split64"),        # 196 tiles of 64x64
     ((128, 7, 7, 256, 256), "fp32", "split64+48"),    # 392: one round, the rest in 184 lower ones
     ((49, 30, 27, 96, 36), "fp32", "split64+32"),     # 621: two rounds, and 6922 rows in lower tiles
     ((64, 14, 14, 128, 128), "fp32", "whole"),        # 392 too, but 128 channels: wide48 is as fast
