@@ -2,6 +2,11 @@
 // P_i [M,K] = TI_i [M,C] . W_i [C,K] on the matrix cores, with the output transform
 // Y = A^T p A folded into the same kernel.
 //
+// This file holds the entry points, the choice of a kernel and the launches of the ring kernels, which are what the next
+// paragraph describes.  Small grids run with a wave per position (winograd2x2_conv_direct.hip), grids of one round of
+// workgroups or of many channels with two positions per wave and fp32 operands in three bf16 pieces
+// (winograd2x2_conv_split.hip), the rest with fp32 matrix instructions here and in winograd2x2_conv_wide*.hip.
+//
 // Stands in for Winograd2x2ConvComputeLauncher of the reference
 // (winograd2x2_cublas/winograd2x2_conv/winograd2x2_conv_cuda.cu.cc:65-93): the `assign`
 // pointer-table kernel (:55-61), cublasSgemmBatched (:80-85) and the Output_transform
