@@ -58,8 +58,8 @@ SWC_API const char *swc_version(void);
  * integer-valued data). */
 SWC_API const char *swc_winograd2x2_conv_last_kernel(void);
 /* Diagnostic with no counterpart in the reference: how that call ran: "whole" (one workgroup per tile of one of the kernels
- * above; bf16-stored operands always do), or over fp32 planes, on grids that leave most of the device idle that
- * way, "direct16x16" / "direct16x32" / "direct16x64" / "direct32x64": sixteen waves per workgroup, one per position,
+ * above; bf16-stored operands always do), or over fp32 planes "direct16x16" / "direct16x32" / "direct16x64" / "direct32x64"
+ * (grids that would leave most of the device idle): sixteen waves per workgroup, one per position,
  * each with the named tile of rows x columns (C % 4 == 0); or "split32" / "split48" / "split64" / "split64+32" /
  * "split64+48" (whole rounds of 64-row tiles, the rest in lower ones): tiles of that many rows x 64 columns, the positions
  * split over eight waves, on the 16-bit matrix instructions: fp32 operands in three bf16 pieces each, which hold all their
