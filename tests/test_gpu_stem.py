@@ -58,6 +58,23 @@ def test_values_that_do_not_split():
     assert ((got - want).abs() <= 147 * 2.0 ** -24 * expected_magnitude(image[1:], w)[..., 3]).all()
 
 
+def test_spreads_beyond_the_exponents_that_pieces_are_shifted_by():
+    """Within a channel's weights beyond 2^80, within a tile beyond 2^138: fp32 vector arithmetic, each pixel as good as alone."""
+    import resnet18_var
+    gen = torch.Generator().manual_seed(85)
+    image, w = torch.randn((1, 64, 64, 3), generator=gen), torch.randn((64, 3, 7, 7), generator=gen) * 0.1
+    bound = 2 * (147 + 4) * 2.0 ** -24
+    spread = w.clone()
+    spread[7, :, :3] *= 1e-28
+    wide = image.clone()
+    wide[0, :20] *= 1e22
+    wide[0, 30:] *= 1e-22
+    for im, wt in ((image, spread), (wide, w), (wide, spread)):
+        got = resnet18_var.stem_conv_pool(im.cuda(), wt.cuda()).cpu()
+        want = expected(im.double(), wt.double())
+        assert ((got - want).abs() <= bound * expected_magnitude(im, wt)).all()
+
+
 @pytest.mark.parametrize("bright", [24, 28, 34, 46, 60, 100])
 @pytest.mark.parametrize("positive", [False, True])
 def test_a_pixel_changes_only_what_sees_it(bright, positive):
