@@ -27,6 +27,8 @@ import swc_hip  # noqa: E402
 from winograd_conv import WinogradConv  # noqa: E402
 from winograd_imtrans import WinogradImTrans  # noqa: E402
 
+_native = swc_hip.native()
+
 # (unit name, C_in of the first conv, C_out, has 1x1 shortcut conv, max-pool after the unit)
 UNITS = (
     ("2a", 64, 64, True, False), ("2b", 64, 64, False, True),
@@ -61,12 +63,12 @@ def _max_pool_same(x):
 
 def _bn_affine(bn):
     """Inference-mode BatchNorm2d as y = x*scale + shift; cached until a parameter or statistic changes."""
-    tensors = (bn.weight, bn.bias, bn.running_mean, bn.running_var)
-    key = tuple((t._version, t.data_ptr()) for t in tensors)
-    cached = getattr(bn, "_swc_affine", None)
+    weight, bias, mean, var = bn.weight, bn.bias, bn.running_mean, bn.running_var
+    key = _native.key(weight, bias, mean, var)
+    cached = bn.__dict__.get("_swc_affine")
     if cached is None or cached[0] != key:
-        scale = (bn.weight * torch.rsqrt(bn.running_var + bn.eps)).detach()
-        cached = (key, scale.contiguous(), (bn.bias - bn.running_mean * scale).detach().contiguous())
+        scale = (weight * torch.rsqrt(var + bn.eps)).detach()
+        cached = (key, scale.contiguous(), (bias - mean * scale).detach().contiguous())
         bn._swc_affine = cached
     return cached[1], cached[2]
 
@@ -75,10 +77,11 @@ def _conv_bn_folded(conv, bn):
     """A bias-free conv followed by an inference-mode BatchNorm as one conv: weights scaled per output
     channel, the shift as bias.  Cached until the weights or the BatchNorm change."""
     scale, shift = _bn_affine(bn)
-    key = (conv.weight._version, conv.weight.data_ptr(), bn._swc_affine[0])
-    cached = getattr(conv, "_swc_folded", None)
+    weight = conv.weight
+    key = (_native.key(weight), bn._swc_affine[0])
+    cached = conv.__dict__.get("_swc_folded")
     if cached is None or cached[0] != key:
-        cached = (key, (conv.weight * scale.view(-1, 1, 1, 1)).detach(), shift)
+        cached = (key, (weight * scale.view(-1, 1, 1, 1)).detach(), shift)
         conv._swc_folded = cached
     return cached[1], cached[2]
 
@@ -91,7 +94,7 @@ def _shortcut_folded(conv, bn, bn_out):
     w1, b1 = _conv_bn_folded(conv, bn)
     scale, shift = _bn_affine(bn_out)
     key = (conv._swc_folded[0], bn_out._swc_affine[0])
-    cached = getattr(conv, "_swc_shortcut", None)
+    cached = conv.__dict__.get("_swc_shortcut")
     if cached is None or cached[0] != key:
         cached = (key, w1.view(w1.shape[0], w1.shape[1]).contiguous(), scale, (shift + b1).contiguous())
         conv._swc_shortcut = cached
@@ -101,6 +104,9 @@ def _shortcut_folded(conv, bn, bn_out):
 def pointwise_conv(x, w):
     """x [B,H,W,C] NHWC, w [K,C] -> [B,H,W,K]: a 1x1 convolution.  On the GPU it runs on the library's kernel
     (``swc_winograd2x2_pointwise_conv``) where that takes the shape (C % 32 == 0), else as a matrix product."""
+    out = _native.pointwise(x, w)
+    if out is not None:
+        return out
     B, H, W, C = x.shape
     if x.is_cuda and x.dtype == torch.float32 and w.dtype == torch.float32 and x.is_contiguous() and w.is_contiguous():
         out = torch.empty((B, H, W, w.shape[0]), dtype=torch.float32, device=x.device)

@@ -3,11 +3,13 @@
 There is no fallback: if the library has not been built, loading raises.
 """
 import ctypes
+import importlib.util
 import os
 import subprocess
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libwinograd2x2_hip.so")
+NATIVE_PATH = os.path.join(_HERE, "_swc_torch.so")
 CSRC = os.path.join(_HERE, "csrc")
 
 SWC_OK = 0
@@ -44,10 +46,27 @@ CXX_SYMBOLS = (
 )
 
 _lib = None
+_native = None
+
+
+def native():
+    """The native host side of the ops (csrc/swc_torch.cpp)."""
+    global _native
+    if _native is None:
+        lib()
+        import torch  # noqa: F401  (its libraries are what the module is linked against)
+
+        if not os.path.exists(NATIVE_PATH):
+            raise ImportError("%s is missing: build it with `make -C %s` (or __graft_entry__.build())" % (NATIVE_PATH, CSRC))
+        spec = importlib.util.spec_from_file_location("_swc_torch", NATIVE_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _native = module
+    return _native
 
 
 def build():
-    """Compile the library for gfx950 with hipcc (works without a GPU)."""
+    """Compile the library for gfx950 with hipcc and the ops' host side (works without a GPU)."""
     subprocess.check_call(["make", "-s", "-C", CSRC, "-j8"])
     return LIB_PATH
 

@@ -14,6 +14,8 @@ import torch
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import swc_hip  # noqa: E402
 
+_native = swc_hip.native()   # the plain case in one call; None back from it where the case is another
+
 PRECISIONS = {"fp32": 0, "bf16": 1}
 
 
@@ -46,6 +48,10 @@ def _plan(i_shape, w_shape):
 def _forward(I, W, precision, out, scale=None, shift=None, residual=None, residual_relu=False):
     if precision not in PRECISIONS:
         raise ValueError("precision must be one of %s" % sorted(PRECISIONS))
+    if out is None:
+        result = _native.conv(I, W, precision == "bf16", scale, shift, residual, residual_relu)
+        if result is not None:
+            return result
     I = swc_hip.require_cuda_f32(I, "I", 5)
     W = swc_hip.require_cuda_f32(W, "W", 3)
     if W.device != I.device:
@@ -98,6 +104,10 @@ def winograd2x2_weights_bf16(W):
 
 def _forward_bf16_stored(I, W, out, scale, shift, residual, residual_relu=False, workspace=True):
     """I [16,B,nH,nW,C] bfloat16; W [16,C,K] float32 or prepared [16,K,C] bfloat16."""
+    if out is None:
+        result = _native.conv_stored(I, W, scale, shift, residual, residual_relu, workspace)
+        if result is not None:
+            return result
     I = swc_hip.require_cuda_f32(I, "I", 5, torch.bfloat16)
     if not isinstance(W, torch.Tensor) or W.dim() != 3:
         raise ValueError("W must be a rank-3 tensor")
@@ -151,6 +161,9 @@ def winograd2x2_conv_grad_shape(i_shape, w_shape, g_shape):
 def winograd2x2_conv_grad(i1, i2, grad):
     """(I [16,B,nH,nW,C], W [16,C,K], grad [B,2nH,2nW,K]) -> (dI, dW), as the reference's
     winograd2x2_conv_grad (winograd2x2_conv.py:16-17).  fp32 throughout."""
+    result = _native.conv_grad(i1, i2, grad)
+    if result is not None:
+        return result
     I = swc_hip.require_cuda_f32(i1, "i1", 5)
     W = swc_hip.require_cuda_f32(i2, "i2", 3)
     grad = swc_hip.require_cuda_f32(grad, "grad", 4)
@@ -200,7 +213,8 @@ def winograd2x2_conv(I, W, precision="fp32", out=None, scale=None, shift=None, r
     ``precision="bf16"`` rounds both GEMM operands to bf16 (fp32 accumulate).  Differentiable
     through ``winograd2x2_conv_grad`` when an input requires grad.
     """
-    needs_grad = torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in (I, W))
+    needs_grad = torch.is_grad_enabled() and ((isinstance(I, torch.Tensor) and I.requires_grad) or
+                                              (isinstance(W, torch.Tensor) and W.requires_grad))
     if isinstance(I, torch.Tensor) and I.dtype == torch.bfloat16:
         if needs_grad:
             raise NotImplementedError("the bf16-stored variant is forward only")

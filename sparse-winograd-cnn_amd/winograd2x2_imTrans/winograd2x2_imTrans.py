@@ -13,6 +13,8 @@ import torch
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import swc_hip  # noqa: E402
 
+_native = swc_hip.native()   # the plain case in one call; None back from it where the case is another
+
 
 def winograd2x2_imTrans_shape(shape):
     """[B,H,W,C] -> [16,B,(H+1)/2,(W+1)/2,C] (winograd2x2_imTrans.py:20-27), computed by the C++ host wrapper."""
@@ -39,6 +41,10 @@ def _plan(shape):
 
 
 def _forward(I, relu, out, scale=None, shift=None, out_dtype=torch.float32):
+    if out is None and (out_dtype is torch.float32 or out_dtype is torch.bfloat16):
+        result = _native.imtrans(I, relu, scale, shift, out_dtype is torch.bfloat16)
+        if result is not None:
+            return result
     I = swc_hip.require_cuda_f32(I, "I", 4)
     shape, i_dims, o_dims = _plan(I.shape)
     if (scale is None) != (shift is None):
@@ -82,6 +88,10 @@ def winograd2x2_imTrans_grad(grad, H=None, W=None, relu_output=None, relu_input=
     it, which reads a quarter of the bytes) is given.  ``grad`` is left untouched (the reference
     overwrites it).
     """
+    if relu_output is None and type(H) is int and type(W) is int:
+        result = _native.imtrans_grad(grad, H, W, relu_input)
+        if result is not None:
+            return result
     grad = swc_hip.require_cuda_f32(grad, "grad", 5)
     if grad.shape[0] != 16:
         raise ValueError("grad must have shape [16,B,nH,nW,C]")

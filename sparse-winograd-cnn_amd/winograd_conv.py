@@ -6,7 +6,10 @@ import sys
 import torch
 
 sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+import swc_hip  # noqa: E402
 import winograd2x2_conv.winograd2x2_conv  # noqa: E402
+
+_native = swc_hip.native()
 
 __all__ = ["WinogradConv"]
 
@@ -60,8 +63,7 @@ class WinogradConv(torch.nn.Module):
 
     def _weight_key(self):
         # In-place writes bump _version; a replaced or moved tensor changes data_ptr / device.
-        w, m = self.W, self.mask
-        return (w._version, w.data_ptr(), w.device, None if m is None else (m._version, m.data_ptr()))
+        return _native.key(self.W, self.mask)
 
     def bf16_weight(self):
         """W*mask as the [16,K,C] bfloat16 tensor the bf16-stored kernel reads; cached like masked_weight()."""
@@ -75,12 +77,13 @@ class WinogradConv(torch.nn.Module):
     def masked_weight(self):
         """W*mask without autograd history, recomputed only when W or mask changed since the last call (a write
         through ``.data`` is not such a change: see refresh())."""
-        if self.mask is None:
-            return self.W.detach()   # shares W's version counter: a write to what is handed out is noticed
-        key = self._weight_key()
+        W, mask = self.W, self.mask
+        if mask is None:
+            return W.detach()   # shares W's version counter: a write to what is handed out is noticed
+        key = _native.key(W, mask)
         cached = self._masked
         if cached is None or cached[0] != key:
-            cached = (key, (self.W.detach() * self.mask).contiguous())
+            cached = (key, (W.detach() * mask).contiguous())
             self._masked = cached
         return cached[1]
 
@@ -94,6 +97,4 @@ class WinogradConv(torch.nn.Module):
         else:
             w = self.masked_weight()
         scale, shift = affine if affine is not None else (None, None)
-        return winograd2x2_conv.winograd2x2_conv.winograd2x2_conv(x, w, precision=self.precision, scale=scale,
-                                                                  shift=shift, residual=residual,
-                                                                  residual_relu=residual_relu)
+        return winograd2x2_conv.winograd2x2_conv.winograd2x2_conv(x, w, self.precision, None, scale, shift, residual, residual_relu)

@@ -29,14 +29,11 @@ def WinogradImTrans(x, nl=identity, affine=None, out_dtype=torch.float32):
     transform kernel; any other callable is applied to the op's result.
     """
     op = winograd2x2_imTrans.winograd2x2_imTrans.winograd2x2_imTrans
-    if affine is not None or out_dtype != torch.float32:
-        scale, shift = affine if affine is not None else (None, None)
-        base = op
-        op = lambda t, relu=False: base(t, relu=relu, scale=scale, shift=shift, out_dtype=out_dtype)  # noqa: E731
+    scale, shift = affine if affine is not None else (None, None)
+    if nl is _RELUS[0] or nl == "relu" or nl is _RELUS[1] or isinstance(nl, torch.nn.ReLU):
+        return op(x, True, None, scale, shift, out_dtype)
     if nl is None or nl is identity or nl == "identity":
-        return op(x)
-    if nl == "relu" or isinstance(nl, torch.nn.ReLU) or any(nl is f for f in _RELUS):
-        return op(x, relu=True)
+        return op(x, False, None, scale, shift, out_dtype)
     if not callable(nl):
         raise TypeError("nl must be callable, 'identity' or 'relu'")
-    return nl(op(x))
+    return nl(op(x, False, None, scale, shift, out_dtype))

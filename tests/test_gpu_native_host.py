@@ -1,0 +1,114 @@
+"""The native host side of the Python ops: the same values as the general path, which everything that is not a plain call takes."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def operands(C=64, K=72, relu=False):
+    gen = torch.Generator(device="cuda").manual_seed(91)
+    rand = lambda *s: torch.randn(s, device="cuda", generator=gen)   # noqa: E731
+    return {"x": rand(2, 7, 10, C), "ti": rand(16, 2, 4, 5, C), "w": rand(16, C, K), "a": rand(C), "b": rand(C), "scale": rand(K), "shift": rand(K),
+            "res": rand(2, 8, 10, K)}
+
+
+def calls(o, **kw):
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv, winograd2x2_weights_bf16
+    from winograd2x2_imTrans.winograd2x2_imTrans import winograd2x2_imTrans
+    yield "transform", lambda **k: winograd2x2_imTrans(o["x"], **k), (16, 2, 4, 5, 64)
+    yield "transform, relu, affine", lambda **k: winograd2x2_imTrans(o["x"], relu=True, scale=o["a"], shift=o["b"], **k), (16, 2, 4, 5, 64)
+    yield "transform, bf16", lambda **k: winograd2x2_imTrans(o["x"], relu=True, out_dtype=torch.bfloat16, **k), (16, 2, 4, 5, 64)
+    for precision in ("fp32", "bf16"):
+        yield "conv " + precision, lambda **k: winograd2x2_conv(o["ti"], o["w"], precision=precision, **k), (2, 8, 10, 72)
+        yield "conv epilogue " + precision, lambda **k: winograd2x2_conv(o["ti"], o["w"], precision=precision, scale=o["scale"], shift=o["shift"],
+                                                                         residual=o["res"], residual_relu=True, **k), (2, 8, 10, 72)
+    yield "stored", lambda **k: winograd2x2_conv(o["ti"].bfloat16(), winograd2x2_weights_bf16(o["w"]), residual=o["res"], **k), (2, 8, 10, 72)
+
+
+def test_plain_calls_and_calls_with_out_agree():
+    o = operands()
+    for name, call, shape in calls(o):
+        got = call()
+        assert got.shape == shape and not got.requires_grad, name
+        assert torch.equal(got, call(out=torch.empty_like(got))), name
+
+
+def test_what_is_not_plain_takes_the_general_path():
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv
+    from winograd2x2_imTrans.winograd2x2_imTrans import winograd2x2_imTrans
+
+    class Count(TorchDispatchMode):
+        seen = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            Count.seen += 1
+            return func(*args, **(kwargs or {}))
+
+    class Sub(torch.Tensor):
+        pass
+
+    o = operands()
+    plain = winograd2x2_conv(winograd2x2_imTrans(o["x"]), o["w"])
+    with Count():
+        watched = winograd2x2_conv(winograd2x2_imTrans(o["x"]), o["w"])
+    assert Count.seen >= 2 and torch.equal(watched, plain)
+    strided = torch.empty((2, 10, 7, 64), device="cuda").transpose(1, 2).copy_(o["x"])
+    assert torch.equal(winograd2x2_conv(winograd2x2_imTrans(strided), o["w"].transpose(1, 2).contiguous().transpose(1, 2)), plain)
+    assert torch.equal(winograd2x2_conv(winograd2x2_imTrans(o["x"].as_subclass(Sub)), o["w"]), plain)
+    x, w = o["x"].clone().requires_grad_(), o["w"].clone().requires_grad_()
+    y = winograd2x2_conv(winograd2x2_imTrans(x), w)
+    assert torch.equal(y, plain) and y.requires_grad
+    with torch.no_grad():
+        assert not winograd2x2_conv(winograd2x2_imTrans(x), w).requires_grad
+    with torch.inference_mode():
+        assert torch.equal(winograd2x2_conv(winograd2x2_imTrans(o["x"]), o["w"]), plain)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        other = winograd2x2_conv(winograd2x2_imTrans(o["x"]), o["w"])
+    side.synchronize()
+    assert torch.equal(other, plain)
+    for bad in (o["x"].double(), o["x"].cpu(), o["x"][0], "x"):
+        with pytest.raises((TypeError, ValueError, RuntimeError)):
+            winograd2x2_imTrans(bad)
+    for bad in (o["w"][:, :60], o["w"][:15], o["w"].half(), o["w"].cpu(), None):
+        with pytest.raises((TypeError, ValueError, RuntimeError)):
+            winograd2x2_conv(o["ti"], bad)
+    for bad in ({"scale": o["scale"]}, {"scale": o["scale"][:5], "shift": o["shift"]}, {"residual": o["res"][:1]}, {"residual_relu": True}):
+        with pytest.raises((TypeError, ValueError)):
+            winograd2x2_conv(o["ti"], o["w"], **bad)
+    with pytest.raises(Exception):
+        torch.func.vmap(lambda t: winograd2x2_imTrans(t))(o["x"].unsqueeze(0))
+
+
+def test_gradients_through_both_paths():
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv_grad
+    from winograd2x2_imTrans.winograd2x2_imTrans import winograd2x2_imTrans_grad
+    o = operands()
+    g = torch.randn((2, 8, 10, 72), device="cuda")
+    strided = g.transpose(1, 2).contiguous().transpose(1, 2)      # not contiguous
+    for a, b in zip(winograd2x2_conv_grad(o["ti"], o["w"], g), winograd2x2_conv_grad(o["ti"], o["w"], strided)):
+        assert torch.equal(a, b)
+    strided = o["ti"].transpose(1, 2).contiguous().transpose(1, 2)
+    for relu_input in (None, o["x"]):
+        assert torch.equal(winograd2x2_imTrans_grad(o["ti"], 7, 10, relu_input=relu_input),
+                           winograd2x2_imTrans_grad(strided, 7, 10, relu_input=relu_input))
+    for bad in (g[:1], g[:, :6], g[..., :70]):
+        with pytest.raises(Exception):
+            winograd2x2_conv_grad(o["ti"], o["w"], bad)
+    with pytest.raises(ValueError):
+        winograd2x2_imTrans_grad(o["ti"], 9, 10)
+
+
+def test_key_tells_writes_and_replacements():
+    import swc_hip
+    key = swc_hip.native().key
+    w, m = torch.zeros(4, device="cuda"), torch.ones(4, device="cuda")
+    k = key(w, m)
+    assert key(w, m) == k and key(w.detach(), m) == k
+    assert key(w, None) != k and key(w, m.clone()) != k and key(m, w) != k
+    w.add_(1)
+    assert key(w, m) != k
+    with pytest.raises(TypeError):
+        key(1)
