@@ -64,7 +64,8 @@ SWC_API const char *swc_winograd2x2_conv_last_kernel(void);
  * "split64+48" (whole rounds of 64-row tiles, the rest in lower ones): tiles of that many rows x 64 columns, the positions
  * split over eight waves, on the 16-bit matrix instructions: fp32 operands in three bf16 pieces each, which hold all their
  * bits (nearer to float64 than the fp32 instructions; a tile with operands above 2^30 or sums below 2^-75 is multiplied
- * with those, operands below 2^-134 count as zero), or bf16 operands. */
+ * with those, operands below 2^-134 count as zero), or bf16 operands; or "pieces32" / "pieces64" / "pieces64+32": the same
+ * with fp32 weights that were taken apart beforehand (swc_winograd2x2_conv_prepared). */
 SWC_API const char *swc_winograd2x2_conv_last_form(void);
 /* Diagnostic with no counterpart in the reference, for benchmarks and tests that compare the tilings: makes
  * the calling thread's later swc_winograd2x2_conv calls
@@ -148,6 +149,24 @@ SWC_API int swc_winograd2x2_conv_epilogue(const float *Input, const float *Weigh
                                   const float *Scale, const float *Shift, const float *Residual, int residual_relu,
                                   int C, int B, int nH, int nW, int K, int pad_h, int pad_w,
                                   int precision, swc_stream_t stream);
+
+/*
+ * The fp32 convolution on weights that were taken apart beforehand.  No counterpart in the reference.
+ * swc_winograd2x2_weight_pieces writes what the matrix instructions read: every weight as three bf16 values whose sum it is,
+ * 6 bytes where it has 4, padded to 32 indices and 64 columns (device memory, 16-byte aligned,
+ * swc_winograd2x2_weight_pieces_bytes of it; 0 of them: too large).  Done once per weight update, like
+ * swc_winograd2x2_weights_bf16.
+ * swc_winograd2x2_conv_prepared is swc_winograd2x2_conv_epilogue with precision 0; Pieces are Weight's, or NULL, and are used
+ * where that is the faster way and the operands are aligned; results agree to fp32 rounding.
+ * swc_winograd2x2_conv_pieces_gain says for a shape on the current device whether it is: 0 no, 1 yes, 2 also if the pieces
+ * have to be made for this call alone.
+ */
+SWC_API size_t swc_winograd2x2_weight_pieces_bytes(int C, int K);
+SWC_API int swc_winograd2x2_weight_pieces(const float *Weight, void *Pieces, int C, int K, swc_stream_t stream);
+SWC_API int swc_winograd2x2_conv_prepared(const float *Input, const float *Weight, const void *Pieces, float *Output,
+                                          const float *Scale, const float *Shift, const float *Residual, int residual_relu,
+                                          int C, int B, int nH, int nW, int K, int pad_h, int pad_w, swc_stream_t stream);
+SWC_API int swc_winograd2x2_conv_pieces_gain(int C, int B, int nH, int nW, int K);
 
 /*
  * Same contract as swc_winograd2x2_conv, with both GEMM operands rounded to bf16

@@ -55,7 +55,7 @@ extern "C" int swc_winograd2x2_conv_force_tiling(const char *name)
         return SWC_OK;
     }
     for (const char *known : {"sync", "ring32", "ring16", "tall16", "short16", "wide48", "wide48x64", "direct16x16", "direct16x32", "direct16x64",
-                              "direct32x64", "split32", "split48", "split64", "split64+32", "split64+48"}) {
+                              "direct32x64", "split32", "split48", "split64", "split64+32", "split64+48", "pieces32", "pieces64", "pieces64+32"}) {
         if (std::strcmp(name, known) == 0) {
             std::strcpy(swc::g_forced_tiling, known);
             return SWC_OK;

@@ -141,10 +141,10 @@ PyObject *imtrans(PyObject *, PyObject *const *args, Py_ssize_t count)
     END_HANDLE_TH_ERRORS
 }
 
-// conv(I, W, bf16 operands, scale, shift, residual, residual_relu)
+// conv(I, W, bf16 operands, scale, shift, residual, residual_relu, pieces)
 PyObject *conv(PyObject *, PyObject *const *args, Py_ssize_t count)
 {
-    SWC_ARGS(7)
+    SWC_ARGS(8)
     const at::Tensor *I = plain(args[0], at::kFloat, 5), *W = plain(args[1], at::kFloat, 3);
     if (I == nullptr || W == nullptr || watched() || records(*I) || records(*W) || I->device() != W->device()) return none();
     const int64_t B = I->size(1), nH = I->size(2), nW = I->size(3), C = I->size(4), K = W->size(2);
@@ -153,18 +153,48 @@ PyObject *conv(PyObject *, PyObject *const *args, Py_ssize_t count)
     bool ok = bf16 >= 0 && residual_relu >= 0 && (args[3] == Py_None) == (args[4] == Py_None) && !(residual_relu && args[5] == Py_None);
     const float *scale = optional(args[3], *I, {K}, &ok), *shift = optional(args[4], *I, {K}, &ok),
                 *residual = optional(args[5], *I, {B, 2 * nH, 2 * nW, K}, &ok);
+    const bool for_this_call = args[7] == Py_True;
+    at::Tensor pieces;
+    if (ok && args[7] != Py_None && !for_this_call) {
+        const at::Tensor *p = plain(args[7], at::kByte, 1);
+        if (p == nullptr || bf16 || p->device() != I->device() ||
+            static_cast<size_t>(p->size(0)) != swc_winograd2x2_weight_pieces_bytes(as_int(C), as_int(K)))
+            return none();
+        pieces = *p;
+    }
     if (!ok) return none();
     at::Tensor out;
-    int st;
+    int st = SWC_OK;
     {
         NoGil nogil;
         const c10::DeviceGuard guard(I->device());
         const swc_stream_t stream = stream_of(*I);
         out = make(*I, {B, 2 * nH, 2 * nW, K});
-        st = swc_winograd2x2_conv_epilogue(floats(*I), floats(*W), floats_of(out), scale, shift, residual, residual_relu, as_int(C), as_int(B),
-                                           as_int(nH), as_int(nW), as_int(K), 1, 1, bf16, stream);
+        if (for_this_call && !bf16 && swc_winograd2x2_conv_pieces_gain(as_int(C), as_int(B), as_int(nH), as_int(nW), as_int(K)) == 2) {
+            pieces = make(*I, {static_cast<int64_t>(swc_winograd2x2_weight_pieces_bytes(as_int(C), as_int(K)))}, at::kByte);
+            st = swc_winograd2x2_weight_pieces(floats(*W), pieces.mutable_data_ptr(), as_int(C), as_int(K), stream);
+        }
+        if (st == SWC_OK && pieces.defined())
+            st = swc_winograd2x2_conv_prepared(floats(*I), floats(*W), pieces.const_data_ptr(), floats_of(out), scale, shift, residual, residual_relu,
+                                               as_int(C), as_int(B), as_int(nH), as_int(nW), as_int(K), 1, 1, stream);
+        else if (st == SWC_OK)
+            st = swc_winograd2x2_conv_epilogue(floats(*I), floats(*W), floats_of(out), scale, shift, residual, residual_relu, as_int(C), as_int(B),
+                                               as_int(nH), as_int(nW), as_int(K), 1, 1, bf16, stream);
     }
     return st == SWC_OK ? THPVariable_Wrap(std::move(out)) : none();
+    END_HANDLE_TH_ERRORS
+}
+
+// pieces_gain(I, K): swc_winograd2x2_conv_pieces_gain for I [16,B,nH,nW,C], 0 where that is not I's shape
+PyObject *pieces_gain(PyObject *, PyObject *const *args, Py_ssize_t count)
+{
+    SWC_ARGS(2)
+    const long K = PyLong_AsLong(args[1]);
+    if (K == -1 && PyErr_Occurred()) return nullptr;
+    const at::Tensor *I = plain(args[0], at::kFloat, 5);
+    if (I == nullptr || I->size(0) != 16 || !fits(I->sizes()) || !fits({K})) return PyLong_FromLong(0);
+    const c10::DeviceGuard guard(I->device());
+    return PyLong_FromLong(swc_winograd2x2_conv_pieces_gain(as_int(I->size(4)), as_int(I->size(1)), as_int(I->size(2)), as_int(I->size(3)), as_int(K)));
     END_HANDLE_TH_ERRORS
 }
 
@@ -285,6 +315,7 @@ PyMethodDef method(const char *name, Fast f) { return {name, reinterpret_cast<Py
 PyMethodDef methods[] = {method("key", key),
                          method("imtrans", imtrans),
                          method("conv", conv),
+                         method("pieces_gain", pieces_gain),
                          method("conv_stored", conv_stored),
                          method("conv_grad", conv_grad),
                          method("imtrans_grad", imtrans_grad),

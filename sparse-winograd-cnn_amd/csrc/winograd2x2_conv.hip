@@ -66,9 +66,50 @@ int launch_async(const float *TI, const float *Wt, float *Out, size_t M, int C, 
     return check_launch();
 }
 
+// What a call is to run, and what that is taken to last in us.
+struct ConvChoice {
+    TilingChoice whole;
+    double whole_us = 1e30, wide_scale = 1.0;
+    DirectForm direct = DIRECT_NONE;
+    double direct_us = 1e30;
+    SplitChoice split;
+    bool split_wins() const { return split.form != SPLIT_NONE && split.us < direct_us && split.us < whole_us; }
+};
+
+template <bool BF16>
+ConvChoice choose_conv(const void *Input, const void *Weight, const void *Output, const void *residual, size_t M, int C, int K)
+{
+    ConvChoice choice;
+    // The bf16-operand variant has one tiling (ring32, 3-deep: its step is 8x shorter than the fp32 one and needs
+    // two tiles in flight to cover the memory latency); fp32 picks among all of them.
+    TilingChoice &pick = choice.whole;
+    pick = {ring_eligible<Tile32>(Input, Weight, C, K, true) ? TILING_RING32 : TILING_SYNC, Tile32::BM};
+    if (!BF16) pick = choose_tiling(Input, Weight, M, C, K, true, true);
+    choice.direct = choose_direct(Input, Weight, M, C, K, pick.tiling != TILING_SYNC, pick.tiling == TILING_SHORT16, BF16, &choice.direct_us);
+    choice.split = choose_split(Input, Weight, Output, residual, M, C, K, BF16);
+    // What the ring and wide kernels take.  fp32: 6 us + 3.75 per unit of their cost and 64 channels; over 230 shapes the
+    // measured time was 0.95 to 1.4 times that (median 1.1), with the wide tilings 0.88 to 1.08, which therefore count for a
+    // tenth less, and up to 128 channels, where several rounds of a split form take up to 6 % longer than they are taken to
+    // (39572x128->64 101.5 us against 95.6), for 15 %.  bf16 operands: 6 us + 9 per 64 channels at best (one tile per CU), at 32 channels as little as the split
+    // forms' 6.5 to 8.5 + 4.1 to 5.  A direct form is offered only where it takes less.
+    const double per64 = static_cast<double>(C) / 64;
+    const double scale = pick.tiling != TILING_WIDE48 && pick.tiling != TILING_WIDE48X64 ? 1.0 : C > 128 ? 0.9 : 0.85;
+    choice.wide_scale = scale;
+    if (pick.tiling != TILING_SYNC) choice.whole_us = BF16 ? 6.0 + 9.0 * per64 : scale * (6.0 + 3.75 * pick.cost * per64);
+    return choice;
+}
+
+// What weights in pieces are taken to save, in us, with 3 % for what the estimates are off by.
+double pieces_gain(const PiecesChoice &pieces, const ConvChoice &choice)
+{
+    if (pieces.form == PIECES_NONE) return -1e30;
+    if (forced_conv_tiling() != nullptr) return 1e30;
+    return 0.97 * (choice.split_wins() ? choice.split.us : choice.direct != DIRECT_NONE ? choice.direct_us : choice.whole_us / choice.wide_scale) - pieces.us;
+}
+
 template <bool BF16>
 int conv_entry(const float *Input, const float *Weight, float *Output, int C, int B, int nH, int nW, int K,
-               int pad_h, int pad_w, const ConvEpilogue &ep, swc_stream_t stream)
+               int pad_h, int pad_w, const ConvEpilogue &ep, swc_stream_t stream, const void *weight_pieces = nullptr)
 {
     if (Input == nullptr || Weight == nullptr || Output == nullptr) return SWC_ERR_NULL_POINTER;
     if ((ep.scale == nullptr) != (ep.shift == nullptr)) return SWC_ERR_NULL_POINTER;
@@ -77,28 +118,23 @@ int conv_entry(const float *Input, const float *Weight, float *Output, int C, in
     const size_t M = static_cast<size_t>(B) * nH * nW;
     if (M >= (1ull << 31)) return SWC_ERR_BAD_DIMS;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    // The bf16-operand variant has one tiling (ring32, 3-deep: its step is 8x shorter than the fp32 one and needs
-    // two tiles in flight to cover the memory latency); fp32 picks among all of them.
-    TilingChoice pick = {ring_eligible<Tile32>(Input, Weight, C, K, true) ? TILING_RING32 : TILING_SYNC, Tile32::BM};
-    if (!BF16) pick = choose_tiling(Input, Weight, M, C, K, true, true);
-    double direct_us;
-    const DirectForm direct = choose_direct(Input, Weight, M, C, K, pick.tiling != TILING_SYNC, pick.tiling == TILING_SHORT16, BF16, &direct_us);
-    const SplitChoice split = choose_split(Input, Weight, Output, ep.residual, M, C, K, BF16);
-    // What the ring and wide kernels take.  fp32: 6 us + 3.75 per unit of their cost and 64 channels; over 230 shapes the
-    // measured time was 0.95 to 1.4 times that (median 1.1), with the wide tilings 0.88 to 1.08, which therefore count for a
-    // tenth less, and up to 128 channels, where several rounds of a split form take up to 6 % longer than they are taken to
-    // (39572x128->64 101.5 us against 95.6), for 15 %.  bf16 operands: 6 us + 9 per 64 channels at best (one tile per CU), at 32 channels as little as the split
-    // forms' 6.5 to 8.5 + 4.1 to 5.  A direct form is offered only where it takes less.
-    const double per64 = static_cast<double>(C) / 64;
-    const double scale = pick.tiling != TILING_WIDE48 && pick.tiling != TILING_WIDE48X64 ? 1.0 : C > 128 ? 0.9 : 0.85;
-    const double whole_us = pick.tiling == TILING_SYNC ? 1e30 : BF16 ? 6.0 + 9.0 * per64 : scale * (6.0 + 3.75 * pick.cost * per64);
-    if (split.form != SPLIT_NONE && split.us < direct_us && split.us < whole_us) {
+    const ConvChoice choice = choose_conv<BF16>(Input, Weight, Output, ep.residual, M, C, K);
+    if (weight_pieces != nullptr) {
+        const PiecesChoice pieces = choose_pieces(Input, Weight, weight_pieces, Output, ep.residual, M, C, K);
+        if (pieces_gain(pieces, choice) > 0) {
+            note_conv_kernel(kPiecesNames[pieces.form], kPiecesNames[pieces.form]);
+            return launch_pieces(pieces, Input, Weight, weight_pieces, Output, M, C, K, nW, ep.scale, ep.shift, ep.residual, ep.residual_relu, s);
+        }
+    }
+    const TilingChoice &pick = choice.whole;
+    if (choice.split_wins()) {
+        const SplitChoice &split = choice.split;
         note_conv_kernel(kSplitNames[split.form], kSplitNames[split.form]);
         return launch_split(split, BF16, Input, Weight, Output, M, C, K, nW, ep.scale, ep.shift, ep.residual, ep.residual_relu, s);
     }
-    if (direct != DIRECT_NONE) {
-        note_conv_kernel(kDirectNames[direct], kDirectNames[direct]);
-        return launch_direct(direct, BF16, Input, Weight, Output, M, C, K, nW, ep.scale, ep.shift, ep.residual, ep.residual_relu, s);
+    if (choice.direct != DIRECT_NONE) {
+        note_conv_kernel(kDirectNames[choice.direct], kDirectNames[choice.direct]);
+        return launch_direct(choice.direct, BF16, Input, Weight, Output, M, C, K, nW, ep.scale, ep.shift, ep.residual, ep.residual_relu, s);
     }
     note_conv_kernel(tiling_name(pick.tiling));
     switch (pick.tiling) {
@@ -147,6 +183,30 @@ extern "C" int swc_winograd2x2_conv_epilogue(const float *Input, const float *We
     if (precision == 0) return swc::conv_entry<false>(Input, Weight, Output, C, B, nH, nW, K, pad_h, pad_w, ep, stream);
     if (precision == 1) return swc::conv_entry<true>(Input, Weight, Output, C, B, nH, nW, K, pad_h, pad_w, ep, stream);
     return SWC_ERR_BAD_DIMS;
+}
+
+extern "C" int swc_winograd2x2_conv_prepared(const float *Input, const float *Weight, const void *Pieces, float *Output, const float *Scale,
+                                             const float *Shift, const float *Residual, int residual_relu, int C, int B, int nH,
+                                             int nW, int K, int pad_h, int pad_w, swc_stream_t stream)
+{
+    swc::ConvEpilogue ep;
+    ep.scale = Scale;
+    ep.shift = Shift;
+    ep.residual = Residual;
+    ep.residual_relu = residual_relu != 0;
+    return swc::conv_entry<false>(Input, Weight, Output, C, B, nH, nW, K, pad_h, pad_w, ep, stream, Pieces);
+}
+
+extern "C" int swc_winograd2x2_conv_pieces_gain(int C, int B, int nH, int nW, int K)
+{
+    using namespace swc;
+    if (C <= 0 || B <= 0 || nH <= 0 || nW <= 0 || K <= 0) return 0;
+    const size_t M = static_cast<size_t>(B) * nH * nW;
+    if (M >= (1ull << 31)) return 0;
+    const ConvChoice choice = choose_conv<false>(nullptr, nullptr, nullptr, nullptr, M, C, K);
+    const PiecesChoice pieces = choose_pieces(nullptr, nullptr, nullptr, nullptr, nullptr, M, C, K);
+    const double gain = pieces_gain(pieces, choice);
+    return gain > 2.5 + 1.2 / (1 << 20) * 16 * C * K ? 2 : gain > 0 ? 1 : 0;
 }
 
 extern "C" int swc_winograd2x2_weights_bf16(const float *Weight, unsigned short *Weight16t, int C, int K,

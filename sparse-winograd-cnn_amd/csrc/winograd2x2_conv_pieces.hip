@@ -1,0 +1,134 @@
+// Launches of the convolution with weights in pieces (winograd2x2_conv_pieces_kernel.h) and of the kernel that makes those.  Part
+// of what stands in for Winograd2x2ConvComputeLauncher (winograd2x2_cublas/winograd2x2_conv/winograd2x2_conv_cuda.cu.cc:65-93).
+#include "winograd2x2_conv_pieces_kernel.h"
+#include "winograd2x2_conv_launch.h"
+
+namespace swc {
+namespace {
+
+template <typename Main, typename Tail = Main>
+int launch_as(const float *TI, const float *Wt, const void *Wp, float *Out, size_t M, int C, int K, int nW, size_t main_m, const ConvEpilogue &ep,
+              hipStream_t stream)
+{
+    struct Tag {};
+    const int st = raise_lds_limit<Tag>(reinterpret_cast<const void *>(conv_pieces_kernel<Main, Tail>), Main::LDS_BYTES);
+    if (st != SWC_OK) return st;
+    static_assert(Main::LDS_BYTES >= Tail::LDS_BYTES, "the launch asks for the main tiles' LDS");
+    const size_t tiles_n = (static_cast<size_t>(K) + Main::WN - 1) / Main::WN, cus = device_cus();
+    size_t tail_m = 0;
+    if (std::is_same<Main, Tail>::value)
+        main_m = (M + Main::WM - 1) / Main::WM;
+    else
+        tail_m = (M - main_m * Main::WM + Tail::WM - 1) / Tail::WM;   // main_m * WM <= M
+    if ((main_m + tail_m) * tiles_n >= (1ull << 31)) return SWC_ERR_BAD_DIMS;
+    const size_t main_wgs = main_m * tiles_n < cus ? main_m * tiles_n : cus;
+    conv_pieces_kernel<Main, Tail><<<dim3(static_cast<unsigned>(main_wgs + tail_m * tiles_n)), dim3(Main::NT), Main::LDS_BYTES, stream>>>(
+        TI, Wt, static_cast<const char *>(Wp), Out, static_cast<unsigned>(M), C, K, nW, static_cast<unsigned>(main_m),
+        static_cast<unsigned>(main_wgs), static_cast<unsigned>(tail_m), static_cast<unsigned>(tiles_n), ep);
+    return check_launch();
+}
+
+constexpr size_t kInfinityCacheBytes = 256u << 20;
+
+size_t steps_of(int C) { return (static_cast<size_t>(C) + 31) / 32; }
+size_t groups_of(int K) { return (static_cast<size_t>(K) + 63) / 64; }
+
+// Bytes of the pieces of W [16,C,K]; 0 where the offsets within a position's 64 columns would not fit 31 bits.
+size_t pieces_bytes(int C, int K)
+{
+    if (C <= 0 || K <= 0 || C > (1 << 17) || steps_of(C) * groups_of(K) >= (1ull << 27)) return 0;
+    return 16 * groups_of(K) * steps_of(C) * (4 * kPieces * 1024 + sizeof(float));
+}
+
+// 16-byte loads of TI and the pieces, 32-bit byte offsets into a position's planes and 31-bit ones into the output; W itself is
+// read where the fp32 instructions take over.
+bool pieces_eligible(const void *TI, const void *Wt, const void *Wp, const void *Out, const void *residual, size_t M, int C, int K)
+{
+    return C % 4 == 0 && K % 4 == 0 && aligned16(TI) && aligned16(Wt) && aligned16(Wp) && aligned16(Out) && aligned16(residual) &&
+           pieces_bytes(C, K) != 0 && M * static_cast<size_t>(C) < (1ull << 29) && static_cast<size_t>(C + 128) * K < (1ull << 29) &&
+           M * 16 * static_cast<size_t>(K) < (1ull << 31);
+}
+
+}  // namespace
+
+// A workgroup fills a CU, so a launch takes rounds of tiles over the CUs.  Measured per round, 64-row tiles: 8 us + 8.25 per 64
+// channels, 1 us more in all; 32-row tiles: 2.5 + 5.9, and 2.5 + 0.4 more in all.  Where 64-row tiles make more than a round, whole
+// rounds of them and the rest in one round of 32-row ones, 5 + 6.9.  Against what runs on W itself:
+//   14x14x256 -> 256, batch 64    split64       57.5 us   pieces64      43.5 us
+//   7x7x512 -> 512, batch 64      split32       66.5      pieces32      55.4 (58.5)
+//   14x14x256 -> 256, batch 128   split64+48    97.5      pieces64      81.7
+//   28x28x128 -> 128, batch 64    wide48        55.0      not taken: pieces64 takes 49.0, and 63 behind the transform
+//   14x14x512 -> 512, batch 128   split64+32   337        pieces64+32  295.7
+//   784x256 -> 256                direct16x64   24.5      not taken: pieces32 takes 29.3
+//   56x56x64 -> 64, batch 64      tall16        74.6      not taken: pieces64 takes 71.4
+// Over 209 random shapes the choice made here was 5 % faster on the geometric mean where the best of all is 6 %.  Left out: fewer than
+// 64 channels (10000x32->48 14.7 us against 15.6, 3456x48->512 34 against 42), and planes that exceed the Infinity Cache and are
+// read by one column of tiles, which last as long as their bytes take (21756x320->64 129 us against 143.5, 14175x512->64 124 against 129).
+PiecesChoice choose_pieces(const void *TI, const void *Wt, const void *Wp, const void *Out, const void *residual, size_t M, int C, int K)
+{
+    PiecesChoice best;
+    if (!pieces_eligible(TI, Wt, Wp, Out, residual, M, C, K)) return best;
+    if (const char *f = forced_conv_tiling()) {
+        for (int i = PIECES_32; i < PIECES_FORMS; ++i)
+            if (std::string_view(f) == kPiecesNames[i]) best = {static_cast<PiecesForm>(i), M / 128, 0.0};
+        return best;
+    }
+    const size_t cus = device_cus(), tiles_n = groups_of(K);
+    if (C < 64 || (tiles_n == 1 && M * C * 64 > kInfinityCacheBytes)) return best;
+    const double c = static_cast<double>(C) / 64;
+    auto rounds_of = [&](size_t rows, size_t high) { return static_cast<double>(((rows + high - 1) / high * tiles_n + cus - 1) / cus); };
+    auto us64 = [&](double rounds) { return 1.0 + rounds * (8.0 + 8.25 * c); };
+    const double us32 = 2.5 + 0.4 * c + rounds_of(M, 32) * (2.5 + 5.9 * c);
+    best = {PIECES_64, 0, us64(rounds_of(M, 64))};
+    if (us32 < best.us) best = {PIECES_32, 0, us32};
+    const size_t whole = M / 64 * tiles_n / cus, main_m = whole * cus / tiles_n;
+    if (whole > 0 && main_m * 64 < M) {
+        const double us = us64(static_cast<double>(whole)) + rounds_of(M - main_m * 64, 32) * (5.0 + 6.9 * c);
+        if (us < best.us) best = {PIECES_64_32, main_m, us};
+    }
+    // The above holds for planes that the Infinity Cache has; behind the transform that wrote them larger ones come from memory, a half step
+    // ahead only: 0.12 us for every MB beyond 50 (behind the transform 28x28x128 at batch 64 takes 63 us, wide48 62; 14x14x512 at batch 128 328, split64+32 346).
+    const double mb = static_cast<double>(M) * C * 64 / 1e6;
+    if (mb > 50) best.us += 0.12 * (mb - 50);
+    return best;
+}
+
+int launch_pieces(const PiecesChoice &pick, const float *TI, const float *Wt, const void *Wp, float *Out, size_t M, int C, int K, int nW,
+                  const float *scale, const float *shift, const float *residual, int residual_relu, hipStream_t s)
+{
+    ConvEpilogue ep;
+    ep.scale = scale;
+    ep.shift = shift;
+    ep.residual = residual;
+    ep.residual_relu = residual_relu;
+    const bool ragged = C % 16 != 0, deep = steps_of(C) % 2 == 0 && !ragged;
+    switch (pick.form) {
+        case PIECES_64:
+            return ragged ? launch_as<PiecesCfg<2, 2, true>>(TI, Wt, Wp, Out, M, C, K, nW, 0, ep, s)
+                          : launch_as<PiecesCfg<2, 2, false>>(TI, Wt, Wp, Out, M, C, K, nW, 0, ep, s);
+        case PIECES_32:
+            return ragged ? launch_as<PiecesCfg<1, 2, true>>(TI, Wt, Wp, Out, M, C, K, nW, 0, ep, s)
+                   : deep ? launch_as<PiecesCfg<1, 4, false>>(TI, Wt, Wp, Out, M, C, K, nW, 0, ep, s)
+                          : launch_as<PiecesCfg<1, 2, false>>(TI, Wt, Wp, Out, M, C, K, nW, 0, ep, s);
+        case PIECES_64_32:
+            return ragged ? launch_as<PiecesCfg<2, 2, true>, PiecesCfg<1, 2, true>>(TI, Wt, Wp, Out, M, C, K, nW, pick.main_m, ep, s)
+                          : launch_as<PiecesCfg<2, 2, false>, PiecesCfg<1, 2, false>>(TI, Wt, Wp, Out, M, C, K, nW, pick.main_m, ep, s);
+        default: return SWC_ERR_UNSUPPORTED;
+    }
+}
+
+}  // namespace swc
+
+extern "C" size_t swc_winograd2x2_weight_pieces_bytes(int C, int K) { return swc::pieces_bytes(C, K); }
+
+extern "C" int swc_winograd2x2_weight_pieces(const float *Weight, void *Pieces, int C, int K, swc_stream_t stream)
+{
+    using namespace swc;
+    if (Weight == nullptr || Pieces == nullptr) return SWC_ERR_NULL_POINTER;
+    if (C <= 0 || K <= 0 || pieces_bytes(C, K) == 0) return SWC_ERR_BAD_DIMS;
+    if (!aligned16(Pieces)) return SWC_ERR_UNSUPPORTED;
+    const unsigned groups = static_cast<unsigned>(groups_of(K)), steps = static_cast<unsigned>(steps_of(C));
+    weight_pieces_kernel<<<dim3(16 * groups * steps), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(Weight, static_cast<char *>(Pieces), C,
+                                                                                                        K, groups, steps);
+    return check_launch();
+}

@@ -45,11 +45,11 @@ def _plan(i_shape, w_shape):
     return plan
 
 
-def _forward(I, W, precision, out, scale=None, shift=None, residual=None, residual_relu=False):
+def _forward(I, W, precision, out, scale=None, shift=None, residual=None, residual_relu=False, pieces=None):
     if precision not in PRECISIONS:
         raise ValueError("precision must be one of %s" % sorted(PRECISIONS))
     if out is None:
-        result = _native.conv(I, W, precision == "bf16", scale, shift, residual, residual_relu)
+        result = _native.conv(I, W, precision == "bf16", scale, shift, residual, residual_relu, pieces)
         if result is not None:
             return result
     I = swc_hip.require_cuda_f32(I, "I", 5)
@@ -75,8 +75,17 @@ def _forward(I, W, precision, out, scale=None, shift=None, residual=None, residu
         if tuple(residual.shape) != shape:
             raise ValueError("residual must have the output's shape %s" % (shape,))
     with swc_hip.on_device(I.device) as stream:
-        if epilogue:
-            _, B, nH, nW, C = I.shape
+        _, B, nH, nW, C = I.shape
+        if pieces is True:
+            pieces = None
+            if precision == "fp32" and swc_hip.lib().swc_winograd2x2_conv_pieces_gain(C, B, nH, nW, shape[3]) == 2:
+                pieces = winograd2x2_weight_pieces(W)
+        if pieces is not None:
+            st = swc_hip.lib().swc_winograd2x2_conv_prepared(
+                I.data_ptr(), W.data_ptr(), pieces.data_ptr(), out.data_ptr(), None if scale is None else scale.data_ptr(),
+                None if shift is None else shift.data_ptr(), None if residual is None else residual.data_ptr(),
+                int(bool(residual_relu)), C, B, nH, nW, shape[3], 1, 1, stream)
+        elif epilogue:
             st = swc_hip.lib().swc_winograd2x2_conv_epilogue(
                 I.data_ptr(), W.data_ptr(), out.data_ptr(), None if scale is None else scale.data_ptr(),
                 None if shift is None else shift.data_ptr(), None if residual is None else residual.data_ptr(),
@@ -86,6 +95,22 @@ def _forward(I, W, precision, out, scale=None, shift=None, residual=None, residu
                 I.data_ptr(), 5, i_dims, W.data_ptr(), 3, w_dims, out.data_ptr(), 4, o_dims, PRECISIONS[precision],
                 stream)
     swc_hip.check(st, "winograd2x2_conv")
+    return out
+
+
+def winograd2x2_weight_pieces(W):
+    """W [16,C,K] float32 -> the bytes ``winograd2x2_conv(..., pieces=...)`` multiplies with: every weight as three bfloat16
+    values whose sum it is.  Prepare once per weight update."""
+    W = swc_hip.require_cuda_f32(W, "W", 3)
+    if W.shape[0] != 16:
+        raise ValueError("W must have shape [16,C,K]")
+    n = swc_hip.lib().swc_winograd2x2_weight_pieces_bytes(W.shape[1], W.shape[2])
+    if n == 0:
+        raise ValueError("W of shape %s is empty or too large to be taken apart" % (tuple(W.shape),))
+    out = torch.empty(n, dtype=torch.uint8, device=W.device)
+    with swc_hip.on_device(W.device) as stream:
+        st = swc_hip.lib().swc_winograd2x2_weight_pieces(W.data_ptr(), out.data_ptr(), W.shape[1], W.shape[2], stream)
+    swc_hip.check(st, "winograd2x2_weight_pieces")
     return out
 
 
@@ -184,19 +209,19 @@ class _ConvFunction(torch.autograd.Function):
     whatever the forward's GEMM precision was."""
 
     @staticmethod
-    def forward(ctx, I, W, precision):
+    def forward(ctx, I, W, precision, pieces):
         ctx.save_for_backward(I, W)
-        return _forward(I, W, precision, None)
+        return _forward(I, W, precision, None, pieces=pieces)
 
     @staticmethod
     def backward(ctx, grad):
         I, W = ctx.saved_tensors
         dI, dW = winograd2x2_conv_grad(I, W, grad.contiguous())
-        return dI, dW, None
+        return dI, dW, None, None
 
 
 def winograd2x2_conv(I, W, precision="fp32", out=None, scale=None, shift=None, residual=None, residual_relu=False,
-                     workspace=True):
+                     workspace=True, pieces=None):
     """I: [16,B,nH,nW,C], W: [16,C,K], float32 on the GPU -> [B,2nH,2nW,K] (uncropped).
 
     A bfloat16 ``I`` (from ``winograd2x2_imTrans(..., out_dtype=torch.bfloat16)``) takes the bf16-stored
@@ -210,6 +235,9 @@ def winograd2x2_conv(I, W, precision="fp32", out=None, scale=None, shift=None, r
     The bf16-stored kernel gets a temporary of the size its launcher asks for (most shapes: none), as the
     reference's op allocates its launcher's (winograd2x2_conv_op.cc:57-60); ``workspace=False`` calls it without.
 
+    ``pieces`` (fp32 only): what ``winograd2x2_weight_pieces`` made of this W, which is then multiplied with where that is
+    the faster way, or True: made here where even that is faster.  The same result to fp32 rounding.
+
     ``precision="bf16"`` rounds both GEMM operands to bf16 (fp32 accumulate).  Differentiable
     through ``winograd2x2_conv_grad`` when an input requires grad.
     """
@@ -221,13 +249,19 @@ def winograd2x2_conv(I, W, precision="fp32", out=None, scale=None, shift=None, r
         return _forward_bf16_stored(I, W, out, scale, shift, residual, residual_relu, workspace)
     if residual_relu and residual is None:
         raise ValueError("residual_relu needs a residual")
+    if pieces is not None and pieces is not True:
+        if precision != "fp32":
+            raise ValueError("pieces are fp32 weights'")
+        if not isinstance(W, torch.Tensor) or W.dim() != 3 or pieces.dtype != torch.uint8 or pieces.device != W.device or \
+                not pieces.is_contiguous() or pieces.numel() != swc_hip.lib().swc_winograd2x2_weight_pieces_bytes(*W.shape[1:]):
+            raise ValueError("pieces must be what winograd2x2_weight_pieces made of W")
     if (scale is not None or residual is not None) and needs_grad:
         raise NotImplementedError("the scale/shift/residual epilogue is forward only")
     if needs_grad:
         if out is not None:
             raise NotImplementedError("out= is forward only: the result written there would carry no gradient")
-        return _ConvFunction.apply(I, W, precision)
-    return _forward(I, W, precision, out, scale, shift, residual, residual_relu)
+        return _ConvFunction.apply(I, W, precision, pieces)
+    return _forward(I, W, precision, out, scale, shift, residual, residual_relu, pieces)
 
 
 def winograd2x2_relu_conv(X, W, relu=True, out=None):

@@ -50,9 +50,10 @@ class WinogradConv(torch.nn.Module):
         self.register_buffer("mask", mask)
         self._masked = None
         self._bf16 = None
+        self._pieces = None
 
     def refresh(self):
-        """Drop the cached W*mask and its bf16 copy.  Not needed after in-place updates of W or mask made on
+        """Drop the cached W*mask, its bf16 copy and its pieces.  Not needed after in-place updates of W or mask made on
         the tensors themselves or on ``detach()``ed views of them (optimizer steps, ``load_state_dict``,
         ``with torch.no_grad(): W.mul_(m)``): the caches are keyed on the tensors' version counters and storage,
         so those are noticed by themselves.  Needed after a write through ``.data`` (``layer.W.data.mul_(m)``,
@@ -60,6 +61,7 @@ class WinogradConv(torch.nn.Module):
         no trace on W."""
         self._masked = None
         self._bf16 = None
+        self._pieces = None
 
     def _weight_key(self):
         # In-place writes bump _version; a replaced or moved tensor changes data_ptr / device.
@@ -72,6 +74,15 @@ class WinogradConv(torch.nn.Module):
         if cached is None or cached[0] != key:
             cached = (key, winograd2x2_conv.winograd2x2_conv.winograd2x2_weights_bf16(self.masked_weight()))
             self._bf16 = cached
+        return cached[1]
+
+    def weight_pieces(self):
+        """W*mask taken apart for the fp32 convolution; cached like masked_weight()."""
+        key = self._weight_key()
+        cached = self._pieces
+        if cached is None or cached[0] != key:
+            cached = (key, winograd2x2_conv.winograd2x2_conv.winograd2x2_weight_pieces(self.masked_weight()))
+            self._pieces = cached
         return cached[1]
 
     def masked_weight(self):
@@ -90,11 +101,19 @@ class WinogradConv(torch.nn.Module):
     def forward(self, x, affine=None, residual=None, residual_relu=False):
         """``affine=(scale, shift)`` and ``residual`` (forward only) are applied to the result inside
         the kernel: ``conv*scale + shift + residual`` (``+ relu(residual)`` with ``residual_relu``)."""
+        pieces = None
         if x.dtype == torch.bfloat16:      # bf16-stored activations: forward only
             w = self.bf16_weight()
         elif torch.is_grad_enabled() and self.W.requires_grad:
             w = self.W if self.mask is None else self.W * self.mask
+            pieces = True
         else:
             w = self.masked_weight()
+            if self.precision == "fp32":
+                # the cached pieces where W*mask is cached too, pieces made for this call where W itself is used
+                if self.mask is None:
+                    pieces = True
+                elif _native.pieces_gain(x, self.out_channel) and x.device == w.device and x.shape[4] == w.shape[1]:
+                    pieces = self.weight_pieces()
         scale, shift = affine if affine is not None else (None, None)
-        return winograd2x2_conv.winograd2x2_conv.winograd2x2_conv(x, w, self.precision, None, scale, shift, residual, residual_relu)
+        return winograd2x2_conv.winograd2x2_conv.winograd2x2_conv(x, w, self.precision, None, scale, shift, residual, residual_relu, True, pieces)

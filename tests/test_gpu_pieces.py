@@ -1,0 +1,181 @@
+"""The fp32 convolution on weights that were taken apart beforehand: each tile height forced at the edges of its tiles and steps,
+its error against float64 beside the fp32 instructions', the operands that those multiply instead, and the layer that keeps the
+pieces."""
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_direct import bound, forced, tiles_of  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+FORMS = ["pieces32", "pieces64", "pieces64+32"]
+# "pieces64+32" forced takes half of the whole 64-row tiles and leaves the rest to 32-row ones.
+# (B, nH, nW, C, K): M = 1, 17, 33, 65, 130, 255 rows; C below, at and past 16, 32 and 64 indices; K below, at and past 64, and more
+# than four columns of tiles; the last one has more tiles than a GPU has CUs
+SHAPES = [(1, 1, 1, 4, 4), (1, 1, 17, 36, 20), (3, 1, 11, 64, 68), (1, 5, 13, 16, 64), (2, 5, 13, 160, 36), (1, 15, 17, 128, 132),
+          (1, 7, 10, 96, 328), (1, 13, 15, 20, 64), (6, 40, 70, 64, 40)]
+
+
+def dev(a):
+    return torch.from_numpy(a).cuda()
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("shape", SHAPES)
+def test_pieces_forms(oracle, forced, form, shape):  # noqa: F811
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv, winograd2x2_weight_pieces
+    B, nH, nW, C, K = shape
+    rng = np.random.default_rng(81)
+    ti = np.maximum(rng.standard_normal((16, B, nH, nW, C)), 0).astype(np.float32)
+    w = (rng.standard_normal((16, C, K)) * 0.05).astype(np.float32)
+    tii = rng.integers(-4, 5, size=ti.shape).astype(np.float32)
+    wi = rng.integers(-4, 5, size=w.shape).astype(np.float32)
+    scale, shift = rng.standard_normal(K).astype(np.float32), rng.standard_normal(K).astype(np.float32)
+    res = rng.standard_normal((B, 2 * nH, 2 * nW, K)).astype(np.float32)
+    pieces, pieces_i = winograd2x2_weight_pieces(dev(w)), winograd2x2_weight_pieces(dev(wi))
+    assert forced.swc_winograd2x2_conv_force_tiling(form.encode()) == 0
+    got = winograd2x2_conv(dev(ti), dev(w), pieces=pieces).cpu().numpy()
+    assert forced.swc_winograd2x2_conv_last_form().decode() == form
+    exact = winograd2x2_conv(dev(tii), dev(wi), pieces=pieces_i).cpu().numpy()
+    ep = winograd2x2_conv(dev(ti), dev(w), scale=dev(scale), shift=dev(shift), residual=dev(res), residual_relu=True, pieces=pieces).cpu().numpy()
+    buf = dev(res)
+    winograd2x2_conv(dev(ti), dev(w), out=buf, residual=buf, pieces=pieces)   # residual aliasing the output
+    want = oracle.conv(ti, w, acc64=True)
+    err = np.abs(tiles_of(got, nH, nW).astype(np.float64) - tiles_of(want, nH, nW))
+    # the fp32 instructions' bound, and one more rounding a product for the products of pieces that are left out
+    more = 1 + 1 / (w.shape[1] + 8)
+    assert (err <= more * bound(ti, w)[:, None, :] + 2.0 ** -24 * np.abs(tiles_of(want, nH, nW))).all()
+    assert np.array_equal(exact, oracle.conv(tii, wi))
+    assert np.array_equal(ep, oracle.affine(got, scale, shift) + np.maximum(res, 0))
+    assert np.array_equal(buf.cpu().numpy(), got + res)
+
+
+@pytest.mark.parametrize("C", [64, 72, 256, 512])
+@pytest.mark.parametrize("density", [0.1, 0.3, 1.0])
+@pytest.mark.parametrize("magnitude", [(1.0, 0.05), (1e-6, 1e-5), (3e4, 20.0)])
+def test_no_further_from_float64_than_in_one_kernel(forced, C, density, magnitude):  # noqa: F811
+    """Against the forms that take the weights apart themselves and the fp32 instructions."""
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv, winograd2x2_weight_pieces
+    gen = torch.Generator(device="cuda").manual_seed(82)
+    ti = torch.randn((16, 4, 16, 16, C), device="cuda", generator=gen).relu_() * magnitude[0]
+    w = torch.randn((16, C, 128), device="cuda", generator=gen)
+    w *= magnitude[1] * (w.abs() >= w.abs().flatten()[::7].quantile(1 - density))     # the largest are kept
+    p = torch.bmm(ti.reshape(16, -1, C).double(), w.double()).reshape(4, 4, -1, 128)
+    rows = torch.stack([p[0] + p[1] + p[2], p[1] - p[2] - p[3]])
+    want = torch.stack([rows[:, 0] + rows[:, 1] + rows[:, 2], rows[:, 1] - rows[:, 2] - rows[:, 3]], 1)   # [dy,dx,M,K]
+    want = want.reshape(2, 2, 4, 16, 16, 128).permute(2, 3, 0, 4, 1, 5).reshape(4, 32, 32, 128)
+    pieces = winograd2x2_weight_pieces(w)
+    errors = {}
+    for form in FORMS + ["direct16x64", "split64"]:
+        assert forced.swc_winograd2x2_conv_force_tiling(form.encode()) == 0
+        errors[form] = ((winograd2x2_conv(ti, w, pieces=pieces).double() - want).norm() / want.norm()).item()
+        assert forced.swc_winograd2x2_conv_last_form().decode() == form
+    # with few products (64 channels at 10 %) the outputs' own nine-term sums make most of either's error: equal to 1 %
+    assert all(errors[f] <= 1.01 * min(errors["direct16x64"], errors["split64"]) for f in FORMS), errors
+
+
+@pytest.mark.parametrize("name", ["infinite", "nan", "late outlier", "large weights", "large activations", "tiny", "infinite weight"])
+def test_operands_left_to_the_fp32_instructions(forced, name):  # noqa: F811
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv, winograd2x2_weight_pieces
+    gen = torch.Generator(device="cuda").manual_seed(83)
+    ti = torch.randn((16, 1, 8, 12, 96), device="cuda", generator=gen).relu_()
+    w = torch.randn((16, 96, 64), device="cuda", generator=gen) * 0.05
+    if name == "infinite":
+        ti[3, 0, 2, 5, 40] = float("inf")
+    elif name == "infinite weight":
+        w[9, 70, 11] = float("-inf")
+    elif name == "nan":
+        ti[5, 0, 7, 7, 95] = float("nan")
+    elif name == "late outlier":
+        ti[:, :, :, :, 64:] *= 1e12
+    elif name == "large weights":
+        w, ti = w * 1e34, ti * 1e-34
+    elif name == "large activations":
+        w, ti = w * 1e-34, ti * 1e34
+    elif name == "tiny":
+        w, ti = w * 1e-10, ti * 1e-20
+    pieces = winograd2x2_weight_pieces(w)
+    assert forced.swc_winograd2x2_conv_force_tiling(b"direct32x64") == 0
+    want = winograd2x2_conv(ti, w)
+    finite = torch.isfinite(want)
+    for form in FORMS:
+        assert forced.swc_winograd2x2_conv_force_tiling(form.encode()) == 0
+        got = winograd2x2_conv(ti, w, pieces=pieces)
+        assert torch.equal(torch.isnan(got), torch.isnan(want)), form
+        assert torch.equal(got[torch.isinf(want)], want[torch.isinf(want)]), form
+        # sums of 96 products and nine terms in another order
+        assert (got[finite].double() - want[finite]).norm() <= 1e-5 * want[finite].double().norm(), form
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_scaling_by_powers_of_two_commutes(forced, form):  # noqa: F811
+    """Rows, columns and channels scaled against each other down to 2^-50: nothing may round differently."""
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv, winograd2x2_weight_pieces
+    gen = torch.Generator(device="cuda").manual_seed(84)
+    ti = torch.randn((16, 2, 9, 8, 96), device="cuda", generator=gen).relu_()
+    w = torch.randn((16, 96, 72), device="cuda", generator=gen)
+    assert forced.swc_winograd2x2_conv_force_tiling(form.encode()) == 0
+    run = lambda a, b: winograd2x2_conv(a, b, pieces=winograd2x2_weight_pieces(b))   # noqa: E731
+    plain = run(ti, w)
+    powers = torch.tensor([0, 0, -24, 0, -28, -34, 0, -44, -46, 0, -50], device="cuda")
+    pick = lambda n: (2.0 ** powers[torch.arange(n, device="cuda") % len(powers)].double()).float()   # noqa: E731
+    rows, cols = pick(144), pick(72)
+    by_pixel = rows.reshape(2, 9, 1, 8, 1, 1).expand(2, 9, 2, 8, 2, 1).reshape(2, 18, 16, 1)
+    assert torch.equal(run(ti * rows.reshape(1, 2, 9, 8, 1), w), plain * by_pixel)
+    assert torch.equal(run(ti, w * cols), plain * cols)
+    channels = (2.0 ** ((torch.arange(96, device="cuda") * 7 % 41 - 20).double())).float()
+    assert torch.equal(run(ti * channels, w / channels.reshape(96, 1)), plain)
+
+
+@pytest.mark.parametrize("masked", [False, True])
+def test_layer_follows_its_weights(oracle, masked):
+    """The layer's pieces are those of the weights it has at the call: written in place, replaced, masked anew; with gradients
+    and without."""
+    import swc_hip
+    from winograd_conv import WinogradConv
+    gen = torch.Generator(device="cuda").manual_seed(85)
+    B, n, C = 64, 7, 256
+    ti = torch.randn((16, B, n, n, C), device="cuda", generator=gen).relu_()
+    w = torch.randn((16, C, C), device="cuda", generator=gen) * 0.05
+    mask = (torch.rand((16, C, C), device="cuda", generator=gen) < 0.3).float() if masked else None
+    layer = WinogradConv(C, C, mask=mask, W_init=w, device="cuda")
+
+    def check():
+        m = layer.W.detach().double() if layer.mask is None else layer.W.detach().double() * layer.mask
+        p = torch.bmm(ti.reshape(16, -1, C).double(), m).reshape(4, 4, -1, C)
+        r = torch.stack([p[0] + p[1] + p[2], p[1] - p[2] - p[3]])
+        want = torch.stack([r[:, 0] + r[:, 1] + r[:, 2], r[:, 1] - r[:, 2] - r[:, 3]], 1).reshape(2, 2, B, n, n, C)
+        want = want.permute(2, 3, 0, 4, 1, 5).reshape(B, 2 * n, 2 * n, C)
+        for grad in (False, True):
+            with torch.set_grad_enabled(grad):
+                y = layer(ti)
+            if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+                assert swc_hip.lib().swc_winograd2x2_conv_last_form() == b"pieces64"
+            assert (y.detach().double() - want).norm() <= 1e-6 * want.norm()
+
+    check()
+    with torch.no_grad():
+        layer.W.mul_(-1.5)
+    check()
+    if masked:
+        layer.mask.copy_(1 - layer.mask)
+        check()
+    else:
+        layer.W.data.mul_(0.5)      # no trace on W: nothing may be kept of it
+        check()
+    layer.W = torch.nn.Parameter(torch.randn((16, C, C), device="cuda", generator=gen))
+    check()
+    layer.load_state_dict({k: v.flip(1) for k, v in layer.state_dict().items()})
+    check()
+
+
+def test_pieces_that_are_not_the_weights_are_refused():
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv, winograd2x2_weight_pieces
+    ti, w = torch.zeros((16, 1, 2, 2, 64), device="cuda"), torch.zeros((16, 64, 64), device="cuda")
+    pieces = winograd2x2_weight_pieces(w)
+    for bad in (pieces[:-16], pieces.view(torch.int8), pieces.cpu()):
+        with pytest.raises(ValueError):
+            winograd2x2_conv(ti, w, pieces=bad)
+    with pytest.raises(ValueError):
+        winograd2x2_conv(ti, w, precision="bf16", pieces=pieces)
