@@ -25,10 +25,12 @@ int launch_form(DirectForm form, const float *TI, const float *Wt, float *Out, s
                 hipStream_t s)
 {
     switch (form) {
-        case DIRECT_16X16: return launch_as<DirectCfg<1, 1, 16, BF16>>(TI, Wt, Out, M, C, K, nW, ep, s);
-        case DIRECT_16X32: return launch_as<DirectCfg<1, 2, 8, BF16>>(TI, Wt, Out, M, C, K, nW, ep, s);
-        case DIRECT_16X64: return launch_as<DirectCfg<1, 4, 8, BF16>>(TI, Wt, Out, M, C, K, nW, ep, s);
-        case DIRECT_32X64: return launch_as<DirectCfg<2, 4, BF16 ? 8 : 4, BF16, BF16 ? 1 : 2>>(TI, Wt, Out, M, C, K, nW, ep, s);
+        case DIRECT_16X16:   // the only form that takes single columns
+            return K % 4 == 0 && aligned16(Wt) ? launch_as<DirectCfg<1, 1, 8, BF16, 3, true>>(TI, Wt, Out, M, C, K, nW, ep, s)
+                                               : launch_as<DirectCfg<1, 1, 16, BF16>>(TI, Wt, Out, M, C, K, nW, ep, s);
+        case DIRECT_16X32: return launch_as<DirectCfg<1, 2, 8, BF16, 3, true>>(TI, Wt, Out, M, C, K, nW, ep, s);
+        case DIRECT_16X64: return launch_as<DirectCfg<1, 4, 8, BF16, 2, true>>(TI, Wt, Out, M, C, K, nW, ep, s);
+        case DIRECT_32X64: return launch_as<DirectCfg<2, 4, BF16 ? 8 : 4, BF16, BF16 ? 1 : 2, !BF16>>(TI, Wt, Out, M, C, K, nW, ep, s);
         default: return SWC_ERR_UNSUPPORTED;
     }
 }
@@ -43,11 +45,13 @@ static bool direct_eligible(const void *TI, size_t M, int C, int K)
 }
 
 // A workgroup fills a CU (sixteen waves of up to 128 registers), so a launch takes whole rounds over the CUs.  Measured
-// per round, fp32: 3.2 us + 2.4 per 64 channels for 16x16 tiles, 3.4 + 3.6 for 16x32, 4 + 4.8 for 16x64, 6 + 8.2 for
-// 32x64 (with bf16 operands 3 + 2.3, 3.2 + 3.5, 3.6 + 3.6, 5 + 5.2), so the smallest tile that needs one round wins.
+// per round, fp32: 3.1 us + 1.45 per 64 channels for 16x16 tiles, 3.5 + 2.5 for 16x32, 4.2 + 4.2 for 16x64, 5.5 + 7.6 for
+// 32x64 (with bf16 operands 3 + 1.4, 3.2 + 1.95, 3.6 + 2.25, 5 + 5.2), so the smallest tile that needs one round wins.
+// With a row of TI and a column of W per lane the first three were 3.2 + 2.4, 3.4 + 3.6 and 4 + 4.8 (49x512->512 22.9 -> 14.8 us,
+// 196x512->512 34.1 -> 25.5, 784x64->64 5.7 -> 4.65), and blocks of 64 indices instead of 32 spill at three in flight (21.4).
 // The ring kernels take 4.3 + 8.9 us per 64 channels at best (bf16 6 + 9) and hold that up to one 64x64 tile per CU:
-// beyond one round of 32x64 tiles they are as fast or faster (784x64->64: 13.4 -> 5.7 us; 49x512->512: 75.6 -> 22.3;
-// 784x256->256: 41.6 -> 24.8; 1024x512->512: 76.3 -> 74.8).  short16 deals out the same 32x64 tiles at four waves each and
+// beyond one round of 32x64 tiles they are as fast or faster (784x64->64: 13.4 -> 5.7 us; 49x512->512: 75.6 -> 14.8;
+// 784x256->256: 41.6 -> 21.4; 1024x512->512: 76.3 -> 68).  short16 deals out the same 32x64 tiles at four waves each and
 // two or three to a CU; below 256 channels it is the faster one (1024 to 8192 rows, 64 channels: 13.3 to 14.8 us against
 // 14.5 to 15.9; 128: 22.5 to 24.2 against 22.7 to 25.2; 192: 32.0 against 32.5; 256: 41.0 against 40.8), while ring32, which takes
 // the other channel counts, is not (96 channels: 31 against 20).  Where only the
@@ -67,7 +71,7 @@ DirectForm choose_direct(const void *TI, const void *Wt, size_t M, int C, int K,
         return DIRECT_NONE;
     }
     static constexpr struct { size_t rows, cols; double base[2], per64[2]; } kForms[DIRECT_FORMS] = {
-        {}, {16, 16, {3.2, 3.0}, {2.4, 2.3}}, {16, 32, {3.4, 3.2}, {3.6, 3.5}}, {16, 64, {4.0, 3.6}, {4.8, 3.6}}, {32, 64, {6.0, 5.0}, {8.2, 5.2}}};
+        {}, {16, 16, {3.1, 3.0}, {1.45, 1.4}}, {16, 32, {3.5, 3.2}, {2.5, 1.95}}, {16, 64, {4.2, 3.6}, {4.2, 2.25}}, {32, 64, {5.5, 5.0}, {7.6, 5.2}}};
     const size_t cus = device_cus();
     DirectForm best = DIRECT_NONE;
     for (int i = DIRECT_16X16; i <= (wide ? DIRECT_32X64 : DIRECT_16X16); ++i) {

@@ -21,18 +21,22 @@ namespace {
 // 4*lg .. 4*lg+3 of every group of 16, as in the 16x16 ring tilings (the fp32 results are theirs bit for bit): one
 // 16-byte load of its row of TI and four loads of its TN neighbouring columns of W per group, KB = 4*KL indices at a
 // time.  Which columns a tile holds is free: tile tn takes columns TN*li + tn, so that one load of TN floats feeds TN
-// tiles.  A CU answers about one load instruction in 17 clocks whatever its width, which is what bounds the narrow
-// tiles.
-template <int TM_, int TN_, int KL_, bool BF16_, int NBUF_ = 2>
+// tiles.  Where TI and W allow 16-byte loads (TURN) a load takes whole rows instead, 32 indices x 8 rows of TI (16 x 16 with blocks of
+// 16 indices), 16 indices x 16 columns or 8 x 32 of W, and the wave turns them round in its own LDS: a load costs the L1 an
+// access for every 64 bytes that neighbouring lanes share, and one for every lane where they share none, which held a 16x16 tile
+// to 2.4 us per 64 indices.
+template <int TM_, int TN_, int KL_, bool BF16_, int NBUF_ = 2, bool TURN_ = false>
 struct DirectCfg {
     static constexpr int TM = TM_, TN = TN_, KL = KL_;
     static constexpr int NBUF = NBUF_;             // blocks of operands in flight
-    static constexpr bool BF16 = BF16_;
+    static constexpr bool BF16 = BF16_, TURN = TURN_;
     static constexpr int KB = 4 * KL;              // reduction indices per block
     static constexpr int WM = 16 * TM, WN = 16 * TN;
     static constexpr int E = WM * WN;              // elements of a product tile
     static constexpr int NT = 1024;
-    static constexpr int LDS_BYTES = 16 * E * 4;   // the product tiles of the sixteen positions
+    static constexpr bool TURN_W = TURN && TN <= 2;          // wider tiles load 16 bytes a lane as it is
+    static constexpr int STAGE = !TURN ? 0 : TURN_W && WN > WM ? KB * WN : KB * WM;   // floats a wave turns its operands round in
+    static constexpr int LDS_BYTES = 16 * (E + STAGE) * 4;   // the product tiles of the sixteen positions
     static_assert(KL % 8 == 0 || (KL == 4 && !BF16), "a bf16 MFMA takes eight indices per lane");
     static_assert(LDS_BYTES <= 160 * 1024, "a CU has 160 KiB of LDS");
 };
@@ -44,7 +48,7 @@ __global__ __launch_bounds__(Cfg::NT) void conv_direct_kernel(const float *__res
                                                               ConvEpilogue ep)
 {
     constexpr int TM = Cfg::TM, TN = Cfg::TN, KL = Cfg::KL, KB = Cfg::KB, E = Cfg::E, WN = Cfg::WN;
-    extern __shared__ __attribute__((aligned(16))) float P[];   // [16][E]
+    extern __shared__ __attribute__((aligned(16))) float P[];   // [16][E] and the staging blocks
 
     const unsigned lid = xcd_swizzle(blockIdx.x, gridDim.x);
     // Consecutive workgroups share an XCD's L2: let them share whichever operand is the larger one.
@@ -56,13 +60,19 @@ __global__ __launch_bounds__(Cfg::NT) void conv_direct_kernel(const float *__res
     const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
 
     // Rows and columns beyond the edge repeat the last one: what they produce is not stored.
-    unsigned a_off[TM], b_off;   // bytes
+    constexpr int LPR = KB >= 32 ? 8 : 4, NA = Cfg::TURN ? LPR / 4 : 1;   // TURN: lanes to a row, loads for 16 rows
+    unsigned a_off[TM][NA], b_off;   // bytes
 #pragma unroll
-    for (int tm = 0; tm < TM; ++tm) {
-        const unsigned row = m0 + tm * 16 + li;
-        a_off[tm] = ((row < M ? row : M - 1) * static_cast<unsigned>(C) + lg * 4) * 4u;
-    }
-    {
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+        for (int h = 0; h < NA; ++h) {
+            const unsigned row = m0 + tm * 16 + (Cfg::TURN ? 8 * h + lane / LPR : li);
+            a_off[tm][h] = ((row < M ? row : M - 1) * static_cast<unsigned>(C) + (Cfg::TURN ? lane % LPR : lg) * 4) * 4u;
+        }
+    if constexpr (Cfg::TURN_W) {   // lane: index lane / (4*TN) of the load's, columns 4 * (lane % (4*TN)) .. + 3
+        const int n = n0 + lane % (4 * TN) * 4;
+        b_off = (static_cast<unsigned>(lane / (4 * TN)) * K + (n + 4 <= K ? n : K - 4)) * 4u;   // K % 4 == 0
+    } else {
         const int n = n0 + TN * li;
         b_off = (static_cast<unsigned>(lg * 4) * K + (n + TN <= K ? n : K - TN)) * 4u;   // K % TN == 0
     }
@@ -72,9 +82,10 @@ __global__ __launch_bounds__(Cfg::NT) void conv_direct_kernel(const float *__res
     const __amdgpu_buffer_rsrc_t b_desc = make_rsrc(Wt + static_cast<size_t>(pos) * C * K, static_cast<unsigned>(C) * K * 4u);
 
     typedef float BVec __attribute__((ext_vector_type(TN)));
+    constexpr int KR = 16 / TN, NR = KB / KR;   // TURN: indices to a load, loads to a block
     struct Frag {
         float4 a[TM][KL / 4];
-        BVec b[KL];
+        typename std::conditional<Cfg::TURN_W, floatx4[NR], BVec[KL]>::type b;
     };
     auto load = [&](Frag &f, int k0) __attribute__((always_inline)) {
         const bool whole = k0 + KB <= C;     // uniform; else the last block: indices beyond C are zero on both sides
@@ -82,9 +93,20 @@ __global__ __launch_bounds__(Cfg::NT) void conv_direct_kernel(const float *__res
 #pragma unroll
         for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
-            for (int j = 0; j < KL / 4; ++j)
+            for (int j = 0; j < KL / 4; ++j) {
+                // TURN: load j holds rows 8*(j % NA) .. of indices 4*LPR*(j / NA) ..
+                const int at = Cfg::TURN ? j / NA * 4 * LPR : 16 * j;
+                const bool in = whole || (Cfg::TURN ? at + lane % LPR * 4 < C - k0 : at < left);
                 f.a[tm][j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                            a_desc, static_cast<int>(whole || 16 * j < left ? a_off[tm] : kOutOfRange), (k0 + 16 * j) * 4, 0));
+                                                            a_desc, static_cast<int>(in ? a_off[tm][j % NA] : kOutOfRange), (k0 + at) * 4, 0));
+            }
+        if constexpr (Cfg::TURN_W) {
+#pragma unroll
+            for (int i = 0; i < NR; ++i)
+                f.b[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                         b_desc, static_cast<int>(whole || KR * i + lane / (4 * TN) < C - k0 ? b_off : kOutOfRange),
+                                                         (k0 + KR * i) * K * 4, 0));
+        } else
 #pragma unroll
         for (int t = 0; t < KL; ++t) {
             const int j = t / 4, voff = static_cast<int>(whole || 16 * j < left ? b_off : kOutOfRange), soff = (k0 + 16 * j + t % 4) * K * 4;
@@ -105,7 +127,58 @@ __global__ __launch_bounds__(Cfg::NT) void conv_direct_kernel(const float *__res
             for (int r = 0; r < 4; ++r) acc[tm][tn][r] = 0.f;
 
     auto at4 = [](const float4 &v, int q) __attribute__((always_inline)) { return q == 0 ? v.x : q == 1 ? v.y : q == 2 ? v.z : v.w; };
-    auto multiply = [&](const Frag &f) __attribute__((always_inline)) {
+    // Index 16*j + 4*g + t of a block lies in row 16*j + 4*t + g of the staging block: what the four lane groups read at a time is
+    // then side by side.
+    float *const stage = P + 16 * E + pos * Cfg::STAGE;
+    auto multiply = [&](const Frag &raw) __attribute__((always_inline)) {
+        struct {
+            float4 a[TM][KL / 4];
+            BVec b[KL];
+        } f;
+        if constexpr (Cfg::TURN) {   // 16-byte chunk c of row r of 16 rows x 4*LPR indices in slot c ^ (r % 8), c ^ (r / 2 % 4) with four
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+                for (int j = 0; j < KL / 4; ++j) {
+                    const int r = 8 * (j % NA) + lane / LPR, c = lane % LPR;
+                    *reinterpret_cast<float4 *>(stage + (tm * KB + j / NA * 4 * LPR) * 16 + r * 4 * LPR + (c ^ (LPR == 8 ? r % 8 : r / 2 % 4)) * 4) =
+                        raw.a[tm][j];
+                }
+            asm volatile("" ::: "memory");   // other lanes' values are read back; a wave's LDS operations are executed in order
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+                for (int j = 0; j < KL / 4; ++j) {
+                    const int c = j % NA * 4 + lg;
+                    f.a[tm][j] = *reinterpret_cast<const float4 *>(stage + (tm * KB + j / NA * 4 * LPR) * 16 + li * 4 * LPR +
+                                                                   (c ^ (LPR == 8 ? li % 8 : li / 2 % 4)) * 4);
+                }
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+        } else {
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+                for (int j = 0; j < KL / 4; ++j) f.a[tm][j] = raw.a[tm][j];
+        }
+        if constexpr (Cfg::TURN_W) {
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                const int k = KR * i + lane / (4 * TN), row = k / 16 * 16 + k % 4 * 4 + k / 4 % 4;
+                *reinterpret_cast<floatx4 *>(stage + row * WN + lane % (4 * TN) * 4) = raw.b[i];
+            }
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int t = 0; t < KL; ++t)
+                f.b[t] = *reinterpret_cast<const BVec *>(stage + (t / 4 * 16 + t % 4 * 4 + lg) * WN + TN * li);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+        } else {
+#pragma unroll
+            for (int t = 0; t < KL; ++t) f.b[t] = raw.b[t];
+        }
         if constexpr (Cfg::BF16) {
 #pragma unroll
             for (int g = 0; g < KL / 8; ++g) {
@@ -138,19 +211,20 @@ __global__ __launch_bounds__(Cfg::NT) void conv_direct_kernel(const float *__res
         }
     };
 
-    if constexpr (Cfg::NBUF == 2) {
-        Frag f0, f1;
-        load(f0, 0);
-        for (int k0 = 0;;) {
-            if (k0 + KB < C) load(f1, k0 + KB);
-            multiply(f0);
-            k0 += KB;
-            if (k0 >= C) break;
-            if (k0 + KB < C) load(f0, k0 + KB);
-            multiply(f1);
-            k0 += KB;
-            if (k0 >= C) break;
-        }
+    if constexpr (Cfg::NBUF > 1) {
+        constexpr int N = Cfg::NBUF;
+        Frag f[N];
+#pragma unroll
+        for (int i = 0; i + 1 < N; ++i)
+            if (i * KB < C) load(f[i], i * KB);
+        for (int k0 = 0; k0 < C;)
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                if (k0 + (N - 1) * KB < C) load(f[(i + N - 1) % N], k0 + (N - 1) * KB);
+                multiply(f[i]);
+                k0 += KB;
+                if (k0 >= C) break;
+            }
     } else {
         for (int k0 = 0; k0 < C; k0 += KB) {
             Frag f;
