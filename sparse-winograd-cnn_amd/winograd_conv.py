@@ -33,6 +33,8 @@ class WinogradConv(torch.nn.Module):
     W is a trainable parameter; gradients come from ``winograd2x2_conv_grad``.
     """
 
+    _pieces = None   # also for a layer that was pickled without it
+
     def __init__(self, in_channel, out_channel, mask=None, W_init=None, precision="fp32", device=None):
         super().__init__()
         self.in_channel, self.out_channel, self.precision = int(in_channel), int(out_channel), precision
@@ -50,7 +52,6 @@ class WinogradConv(torch.nn.Module):
         self.register_buffer("mask", mask)
         self._masked = None
         self._bf16 = None
-        self._pieces = None
 
     def refresh(self):
         """Drop the cached W*mask, its bf16 copy and its pieces.  Not needed after in-place updates of W or mask made on

@@ -254,3 +254,14 @@ def test_static_entry_bounds_its_size_one_factor_at_a_time():
         assert L.swc_winograd2x2_conv_grad_static(p, p, p, p, p, C, B, H, W, K, 1, 1, None) == swc_hip.SWC_ERR_TOO_LARGE, dims
         if dims[1] > 2:   # and the allocating entry refuses what no buffer could hold (the last case is valid there)
             assert L.swc_winograd2x2_conv_grad(p, p, p, p, p, p, None, C, B, H, W, K, 1, 1, None) == swc_hip.SWC_ERR_BAD_DIMS, dims
+
+
+def test_a_layer_pickled_without_pieces_still_works():
+    from winograd_conv import WinogradConv
+    layer = WinogradConv(8, 8)
+    state = dict(layer.__getstate__() if hasattr(layer, "__getstate__") else layer.__dict__)
+    state.pop("_pieces", None)
+    old = WinogradConv.__new__(WinogradConv)
+    old.__setstate__(state)
+    assert old._pieces is None
+    old.refresh()
