@@ -288,22 +288,30 @@ PyObject *imtrans_grad(PyObject *, PyObject *const *args, Py_ssize_t count)
     END_HANDLE_TH_ERRORS
 }
 
-// pointwise(x [B,H,W,C], w [K,C])
+// pointwise(x [B,H,W,C], w [K,C], relu, scale, shift)
 PyObject *pointwise(PyObject *, PyObject *const *args, Py_ssize_t count)
 {
-    SWC_ARGS(2)
+    SWC_ARGS(5)
     const at::Tensor *x = plain(args[0], at::kFloat, 4), *w = plain(args[1], at::kFloat, 2);
     if (x == nullptr || w == nullptr || watched() || records(*x) || records(*w) || x->device() != w->device() || w->size(1) != x->size(3) ||
         !fits(x->sizes()) || !fits(w->sizes()))
         return none();
+    const int relu = PyObject_IsTrue(args[2]);
+    bool ok = relu >= 0 && (args[3] == Py_None) == (args[4] == Py_None) && (relu || args[3] == Py_None);
+    const float *scale = optional(args[3], *x, {x->size(3)}, &ok), *shift = optional(args[4], *x, {x->size(3)}, &ok);
+    if (!ok) return none();
     at::Tensor out;
     int st;
     {
         NoGil nogil;
         const c10::DeviceGuard guard(x->device());
         out = make(*x, {x->size(0), x->size(1), x->size(2), w->size(0)});
-        st = swc_winograd2x2_pointwise_conv(floats(*x), floats(*w), floats_of(out), as_int(x->size(3)), x->size(0) * x->size(1) * x->size(2),
-                                            as_int(w->size(0)), stream_of(*x));
+        const int64_t rows = x->size(0) * x->size(1) * x->size(2);
+        if (relu)
+            st = swc_winograd2x2_relu_pointwise_conv(floats(*x), scale, shift, floats(*w), floats_of(out), as_int(x->size(3)), rows,
+                                                     as_int(w->size(0)), stream_of(*x));
+        else
+            st = swc_winograd2x2_pointwise_conv(floats(*x), floats(*w), floats_of(out), as_int(x->size(3)), rows, as_int(w->size(0)), stream_of(*x));
     }
     return st == SWC_OK ? THPVariable_Wrap(std::move(out)) : none();
     END_HANDLE_TH_ERRORS

@@ -520,7 +520,11 @@ constexpr int async_lds_bytes()
 // NPOS: how many of the 16 positions (planes of TI, Wt and, in dgrad mode, Out) the call walks, starting at the
 // planes the three pointers point to.  The forward fold needs all 16; the products of the data gradient are
 // independent, so its launcher may deal groups of positions to different workgroups.
-template <typename Cfg, int NSTAGE, bool BF16, int MODE, int NPOS = 16>
+// ACT (dgrad mode): what A's values go through between LDS and the matrix instruction.  RING_RELU: relu(a), with NaN kept;
+// RING_AFFINE_RELU: relu(a*ep.scale[r] + ep.shift[r]) by reduction index r, both vectors kept in LDS behind the ring (2*R floats).
+// One to three vector instructions per 64-cycle matrix instruction, which hides them.
+enum RingAct { RING_PLAIN = 0, RING_RELU = 1, RING_AFFINE_RELU = 2 };
+template <typename Cfg, int NSTAGE, bool BF16, int MODE, int NPOS = 16, int ACT = RING_PLAIN>
 __device__ __forceinline__ void conv_ring_body(const float *__restrict__ TI, const float *__restrict__ Wt,
                                                float *__restrict__ Out, size_t M, int R, int N, int nW, const size_t m0,
                                                const int n0, const unsigned rows_valid, const int wm0, const int wn0,
@@ -553,6 +557,7 @@ __device__ __forceinline__ void conv_ring_body(const float *__restrict__ TI, con
     static_assert((BM * CH) % 64 == 0 && (BK * BN / 4) % 64 == 0, "tiles are whole wave-wide copies");
     static_assert((NSTAGE - 2) * LPS + (DGRAD ? TM * TN * Cfg::REGS : 0) < 64, "vmcnt range");
     static_assert(!DGRAD || NSTAGE <= 3, "the wait below allows for the stores of one earlier step");
+    static_assert(ACT == RING_PLAIN || (DGRAD && NPOS == 1), "one plane's operand");
     static_assert(NPOS == 16 || (DGRAD && NPOS >= 1 && 16 % NPOS == 0), "the output transform folds all 16 positions");
 
     static_assert(NSTAGE * STAGE_FLOATS * 4 == async_lds_bytes<Cfg, NSTAGE, MODE>(), "launcher and kernel agree on the LDS size");
@@ -666,7 +671,18 @@ __device__ __forceinline__ void conv_ring_body(const float *__restrict__ TI, con
         float4 a[KH][TM];
         float b[DGRAD ? 1 : KH][4][TN];
         float4 bq[DGRAD ? KH : 1][TN];
+        float4 scale[ACT == RING_AFFINE_RELU ? KH : 1], shift[ACT == RING_AFFINE_RELU ? KH : 1];
     };
+    // Affine form: this lane's first reduction index of a step, as an offset into smem, for the step whose fragments are read next.
+    constexpr int AFFINE = NSTAGE * STAGE_FLOATS;
+    int affine_at = AFFINE + 4 * lg;
+    if constexpr (ACT == RING_AFFINE_RELU) {
+        for (int r = tid; r < R; r += NT) {
+            smem[AFFINE + r] = ep.scale[r];
+            smem[AFFINE + R + r] = ep.shift[r];
+        }
+        __syncthreads();
+    }
     constexpr int NUB = DGRAD ? TN : 2 * TN;    // B read units per group: b128 reads, or b32 pairs
     constexpr int NU = KH * (TM + NUB);         // read units per half
     // MFMAs per half: fp32 32x32x2 reduces 2 indices each, bf16 32x32x16 all 16 of a half at once.
@@ -701,6 +717,12 @@ __device__ __forceinline__ void conv_ring_body(const float *__restrict__ TI, con
         const int k8 = h * KH + k8l;
         if (v < TM) {
             F.a[k8l][v] = reinterpret_cast<const float4 *>(smem)[st / 4 + a_off[k8][v]];
+            if constexpr (ACT == RING_AFFINE_RELU) {
+                if (v == 0) {
+                    F.scale[k8l] = *reinterpret_cast<const float4 *>(smem + affine_at + KG * k8);
+                    F.shift[k8l] = *reinterpret_cast<const float4 *>(smem + affine_at + KG * k8 + R);
+                }
+            }
         } else if constexpr (DGRAD) {
             F.bq[k8l][v - TM] = reinterpret_cast<const float4 *>(smem)[st / 4 + bq_off[k8][v - TM]];
         } else {
@@ -823,7 +845,13 @@ __device__ __forceinline__ void conv_ring_body(const float *__restrict__ TI, con
             } else {
                 const int tn = i % TN, tm = (i / TN) % TM, t = (i / (TN * TM)) % 4, k8l = i / (TN * TM * 4);
                 const float4 a4 = F.a[k8l][tm];
-                const float av = t == 0 ? a4.x : t == 1 ? a4.y : t == 2 ? a4.z : a4.w;
+                float av = t == 0 ? a4.x : t == 1 ? a4.y : t == 2 ? a4.z : a4.w;
+                if constexpr (ACT == RING_AFFINE_RELU) {
+                    const float4 sc = F.scale[k8l], sh = F.shift[k8l];
+                    av = t == 0 ? __builtin_fmaf(av, sc.x, sh.x) : t == 1 ? __builtin_fmaf(av, sc.y, sh.y)
+                       : t == 2 ? __builtin_fmaf(av, sc.z, sh.z) : __builtin_fmaf(av, sc.w, sh.w);
+                }
+                if constexpr (ACT != RING_PLAIN) av = av < 0.0f ? 0.0f : av;
                 float bv;
                 if constexpr (DGRAD) {
                     const float4 b4 = F.bq[k8l][tn];
@@ -853,6 +881,10 @@ __device__ __forceinline__ void conv_ring_body(const float *__restrict__ TI, con
                     if (finish_slot(e) == i) finish_unit(Pprev, done_pos, e);
             }
             __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (ACT == RING_AFFINE_RELU) {   // F1 of the next step; behind the last one it reads the first again
+            affine_at += BK;
+            if (affine_at >= AFFINE + R) affine_at -= R;
         }
 #pragma unroll
         for (int i = 0; i < NM; ++i) {

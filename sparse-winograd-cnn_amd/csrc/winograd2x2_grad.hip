@@ -696,29 +696,66 @@ int imtrans_grad_entry(const float *TransIm_grad, const float *relu_mask_source,
 }  // namespace
 }  // namespace swc
 
-// Out [M][K] = Input [M][C] . Weight [K][C]^T: a 1x1 convolution over NHWC pixels.  It is one position of the data
-// gradient's product with the roles renamed, so it runs on the same kernel, one plane per workgroup.
-extern "C" int swc_winograd2x2_pointwise_conv(const float *Input, const float *Weight, float *Output, int C, long long M,
-                                              int K, swc_stream_t stream)
+// Out [M][K] = act(Input [M][C]) . Weight [K][C]^T: a 1x1 convolution over NHWC pixels.  It is one position of the data
+// gradient's product with the roles renamed, so it runs on the same kernel body, one plane per workgroup.  Bound by memory
+// (56x56x64 -> 64 at batch 128: 205 MB); the ReLU or BatchNorm + ReLU in front of the model's shortcuts goes onto the operand on its
+// way from LDS, where it costs nothing beside the matrix instructions, instead of passes of its own over the input.
+namespace swc {
+namespace {
+template <typename Cfg, int NSTAGE, int ACT>
+__global__ __launch_bounds__(Cfg::NT) __attribute__((amdgpu_waves_per_eu(Cfg::OCC, Cfg::OCC))) void pointwise_conv_kernel(
+    const float *__restrict__ X, const float *__restrict__ Wt, float *__restrict__ Out, size_t M, int C, int K, unsigned tiles_n, ConvEpilogue in)
 {
-    using namespace swc;
+    const unsigned tile = xcd_swizzle(blockIdx.x, gridDim.x);
+    const size_t m0 = static_cast<size_t>(tile / tiles_n) * Cfg::BM;
+    const int n0 = static_cast<int>(tile % tiles_n) * Cfg::BN;
+    const unsigned rows_valid = static_cast<unsigned>(M - m0 < Cfg::BM ? M - m0 : Cfg::BM);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm0 = (wave / Cfg::WGN) * Cfg::WM, wn0 = (wave % Cfg::WGN) * Cfg::WN;
+    conv_ring_body<Cfg, NSTAGE, false, RING_DGRAD, 1, ACT>(X, Wt, Out, M, C, K, 0, m0, n0, rows_valid, wm0, wn0, in);
+}
+
+template <int ACT>
+int pointwise_entry(const float *Input, const float *Scale, const float *Shift, const float *Weight, float *Output, int C, long long M, int K,
+                    swc_stream_t stream)
+{
     if (Input == nullptr || Weight == nullptr || Output == nullptr) return SWC_ERR_NULL_POINTER;
     if (C <= 0 || K <= 0 || M <= 0 || M >= (1ll << 31)) return SWC_ERR_BAD_DIMS;
-    // reduction over C in whole 32-index steps, 16-byte copies, 32-bit offsets within a tile's rows and the weights
-    if (static_cast<size_t>(DgradTile::BM) * K >= (1ull << 30) || static_cast<size_t>(C) * K >= (1ull << 30) ||
-        !ring_eligible<DgradTile>(Input, Weight, C, K, false))
-        return SWC_ERR_UNSUPPORTED;
     constexpr int kStages = 2;
-    constexpr int lds_bytes = async_lds_bytes<DgradTile, kStages, RING_DGRAD>();
+    constexpr int ring_bytes = async_lds_bytes<DgradTile, kStages, RING_DGRAD>();
+    // reduction over C in whole 32-index steps, 16-byte copies, 32-bit offsets within a tile's rows and the weights; scale and shift
+    // in what 64 KiB of LDS leave
+    if (static_cast<size_t>(DgradTile::BM) * K >= (1ull << 30) || static_cast<size_t>(C) * K >= (1ull << 30) ||
+        !ring_eligible<DgradTile>(Input, Weight, C, K, false) || (ACT == RING_AFFINE_RELU && C > (64 * 1024 - ring_bytes) / 8))
+        return SWC_ERR_UNSUPPORTED;
     const size_t rows = static_cast<size_t>(M);
     const size_t tiles_m = (rows + DgradTile::BM - 1) / DgradTile::BM;
     const size_t tiles_n = (static_cast<size_t>(K) + DgradTile::BN - 1) / DgradTile::BN;
     if (tiles_m * tiles_n >= (1ull << 31)) return SWC_ERR_BAD_DIMS;
-    conv_dgrad_async_kernel<DgradTile, kStages, 1>
+    ConvEpilogue in;
+    in.scale = Scale;
+    in.shift = Shift;
+    const int lds_bytes = ring_bytes + (ACT == RING_AFFINE_RELU ? 8 * C : 0);
+    pointwise_conv_kernel<DgradTile, kStages, ACT>
         <<<dim3(static_cast<unsigned>(tiles_m * tiles_n)), dim3(DgradTile::NT), lds_bytes, static_cast<hipStream_t>(stream)>>>(
-            Input, Weight, Output, rows, K, C, static_cast<unsigned>(tiles_m), static_cast<unsigned>(tiles_n),
-            static_cast<unsigned>(DgradTile::BM));
+            Input, Weight, Output, rows, C, K, static_cast<unsigned>(tiles_n), in);
     return check_launch();
+}
+}  // namespace
+}  // namespace swc
+
+extern "C" int swc_winograd2x2_pointwise_conv(const float *Input, const float *Weight, float *Output, int C, long long M,
+                                              int K, swc_stream_t stream)
+{
+    return swc::pointwise_entry<swc::RING_PLAIN>(Input, nullptr, nullptr, Weight, Output, C, M, K, stream);
+}
+
+extern "C" int swc_winograd2x2_relu_pointwise_conv(const float *Input, const float *Scale, const float *Shift, const float *Weight,
+                                                   float *Output, int C, long long M, int K, swc_stream_t stream)
+{
+    if ((Scale == nullptr) != (Shift == nullptr)) return SWC_ERR_NULL_POINTER;
+    return Scale != nullptr ? swc::pointwise_entry<swc::RING_AFFINE_RELU>(Input, Scale, Shift, Weight, Output, C, M, K, stream)
+                            : swc::pointwise_entry<swc::RING_RELU>(Input, nullptr, nullptr, Weight, Output, C, M, K, stream);
 }
 
 extern "C" int swc_winograd2x2_imtrans_grad(const float *TransIm_grad, const float *relu_mask_source, float *Input_grad,

@@ -104,7 +104,7 @@ def _shortcut_folded(conv, bn, bn_out):
 def pointwise_conv(x, w):
     """x [B,H,W,C] NHWC, w [K,C] -> [B,H,W,K]: a 1x1 convolution.  On the GPU it runs on the library's kernel
     (``swc_winograd2x2_pointwise_conv``) where that takes the shape (C % 32 == 0), else as a matrix product."""
-    out = _native.pointwise(x, w)
+    out = _native.pointwise(x, w, False, None, None)
     if out is not None:
         return out
     B, H, W, C = x.shape
@@ -117,6 +117,16 @@ def pointwise_conv(x, w):
             swc_hip.check(st, "pointwise_conv")
             return out
     return torch.mm(x.reshape(-1, C), w.t()).view(B, H, W, w.shape[0])
+
+
+def relu_pointwise_conv(x, w, affine=None):
+    """``pointwise_conv`` of relu(x), or of relu(x*scale + shift) with ``affine`` = (scale, shift) by channel, x [B,H,W,C] NHWC: applied
+    as the kernel reads x, and where that does not take the call as passes of their own."""
+    scale, shift = affine if affine is not None else (None, None)
+    out = _native.pointwise(x, w, True, scale, shift)
+    if out is not None:
+        return out
+    return pointwise_conv(torch.relu(x) if affine is None else torch.addcmul(shift, x, scale).relu_(), w)
 
 
 def stem_conv_pool(image, w):
@@ -201,19 +211,12 @@ class WinogradUnit(torch.nn.Module):
     def forward(self, x):
         out_affine = None
         if self.shortcut:
-            if self.bn_pre is not None and self.fold_bn:
-                # BNReLU as x*scale + shift and an in-place ReLU: two elementwise passes instead of the library
-                # BatchNorm's slower one plus a ReLU that allocates
-                a, b = _bn_affine(self.bn_pre)
-                s = torch.addcmul(b.view(1, -1, 1, 1), x, a.view(1, -1, 1, 1)).relu_()
-            else:
-                s = torch.relu(self.bn_pre(x)) if self.bn_pre is not None else torch.relu(x)
             if self.fold_bn:
                 w1, scale, shift = _shortcut_folded(self.conv1, self.bn1, self.bn2c)
-                sc = pointwise_conv(_to_nhwc(s), w1)
+                sc = relu_pointwise_conv(_to_nhwc(x), w1, _bn_affine(self.bn_pre) if self.bn_pre is not None else None)
                 out_affine = (scale, shift)
             else:
-                sc = self.bn1(self.conv1(s))
+                sc = self.bn1(self.conv1(torch.relu(self.bn_pre(x)) if self.bn_pre is not None else torch.relu(x)))
         elif self.fold_bn:
             sc = _to_nhwc(x)   # the identity shortcut relu(x): its ReLU is applied where the kernel reads it
         else:

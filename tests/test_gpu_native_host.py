@@ -112,3 +112,28 @@ def test_key_tells_writes_and_replacements():
     assert key(w, m) != k
     with pytest.raises(TypeError):
         key(1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("affine", [False, True])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 32, 1), (2, 7, 9, 64, 64), (1, 8, 8, 96, 65), (3, 5, 13, 128, 200), (1, 3, 3, 48, 20), (1, 2, 3, 4128, 8)])
+def test_relu_pointwise_conv(shape, affine):
+    # Tiles of 64 rows and columns and steps of 32 channels: below, at and beyond each; 48 channels, and 4128 with an affine, take
+    # passes of their own.  Whole numbers up to 8*32*4128 < 2^24 are exact in any order of the sums.
+    import resnet18_var
+    B, H, W, C, K = shape
+    gen = torch.Generator().manual_seed(5)
+    x, w = (torch.randint(-4, 5, s, generator=gen).float() for s in ((B, H, W, C), (K, C)))
+    a, b = (torch.randint(-2, 3, (C,), generator=gen).float() for _ in range(2))
+    dev = torch.device("cuda:0")
+    got = resnet18_var.relu_pointwise_conv(x.to(dev), w.to(dev), (a.to(dev), b.to(dev)) if affine else None).cpu()
+    act = torch.relu(x.double() * a + b) if affine else torch.relu(x.double())
+    assert torch.equal(got.double(), act @ w.double().t())
+    # an infinity or NaN reaches its own pixel's sums and no other's
+    for bad in (float("nan"), float("inf"), float("-inf")):
+        y = x.clone()
+        y[0, 0, 0, C // 2] = bad
+        w1, a1, b1 = torch.ones_like(w), torch.ones_like(a), torch.zeros_like(b)
+        got = resnet18_var.relu_pointwise_conv(y.to(dev), w1.to(dev), (a1.to(dev), b1.to(dev)) if affine else None).cpu()
+        want = torch.relu(y) @ w1.t()
+        assert torch.equal(torch.nan_to_num(got, 7.5, 9.5, 1.5), torch.nan_to_num(want, 7.5, 9.5, 1.5))
