@@ -308,6 +308,15 @@ SWC_API int swc_winograd2x2_relu_pointwise_conv(const float *Input, const float 
                                                 float *Output, int C, long long M, int K, swc_stream_t stream);
 
 /*
+ * 3x3 stride-2 max-pool over NHWC pixels with TensorFlow's SAME padding, Output [B,ceil(H/2),ceil(W/2),C], and the mean over all pixels of
+ * relu(Input), Output [B,C]: the model's pools (imagenet-resnet-transWino-prune.py:115 and behind stages 2 and 3) and its last layer before the
+ * classifier.  NaN propagates in both.  C % 4 == 0 and 16-byte aligned operands, below 2^31 groups of four channels in the
+ * output and 2^20 pixels under a mean; SWC_ERR_UNSUPPORTED otherwise.
+ */
+SWC_API int swc_max_pool_same(const float *Input, float *Output, int C, int B, int H, int W, swc_stream_t stream);
+SWC_API int swc_relu_mean(const float *Input, float *Output, int C, int B, int H, int W, swc_stream_t stream);
+
+/*
  * The model's first two layers in one kernel: Output [B,Hp,Wp,64] = 3x3 stride-2 max-pool of the 7x7 stride-2
  * convolution of Input [B,H,W,3] (NHWC) with Weight [64,3,7,7], both with TensorFlow's SAME padding
  * (ResNet-18-var/imagenet-resnet-transWino-prune.py:113-115); Hp = ceil(ceil(H/2)/2), Wp alike.  fp32: the products are

@@ -317,6 +317,26 @@ PyObject *pointwise(PyObject *, PyObject *const *args, Py_ssize_t count)
     END_HANDLE_TH_ERRORS
 }
 
+// max_pool(x [B,H,W,C]) and relu_mean(x [B,H,W,C])
+template <bool POOL>
+PyObject *pixels(PyObject *, PyObject *const *args, Py_ssize_t count)
+{
+    SWC_ARGS(1)
+    const at::Tensor *x = plain(args[0], at::kFloat, 4);
+    if (x == nullptr || watched() || records(*x) || !fits(x->sizes())) return none();
+    const int64_t B = x->size(0), H = x->size(1), W = x->size(2), C = x->size(3);
+    at::Tensor out;
+    int st;
+    {
+        NoGil nogil;
+        const c10::DeviceGuard guard(x->device());
+        out = POOL ? make(*x, {B, (H + 1) / 2, (W + 1) / 2, C}) : make(*x, {B, C});
+        st = (POOL ? swc_max_pool_same : swc_relu_mean)(floats(*x), floats_of(out), as_int(C), as_int(B), as_int(H), as_int(W), stream_of(*x));
+    }
+    return st == SWC_OK ? THPVariable_Wrap(std::move(out)) : none();
+    END_HANDLE_TH_ERRORS
+}
+
 using Fast = PyObject *(*)(PyObject *, PyObject *const *, Py_ssize_t);
 PyMethodDef method(const char *name, Fast f) { return {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)), METH_FASTCALL, nullptr}; }
 
@@ -328,6 +348,8 @@ PyMethodDef methods[] = {method("key", key),
                          method("conv_grad", conv_grad),
                          method("imtrans_grad", imtrans_grad),
                          method("pointwise", pointwise),
+                         method("max_pool", pixels<true>),
+                         method("relu_mean", pixels<false>),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_swc_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -54,7 +54,11 @@ def _same_pad(x, k, stride):
 
 def _max_pool_same(x):
     """3x3 stride-2 max-pool with TensorFlow SAME padding.  Where the padding falls entirely behind the
-    data (even sizes) ``ceil_mode`` gives the same windows without a padded copy of the tensor."""
+    data (even sizes) ``ceil_mode`` gives the same windows without a padded copy of the tensor.  NHWC memory on the GPU takes the
+    library's kernel (``swc_max_pool_same``)."""
+    out = _native.max_pool(x.permute(0, 2, 3, 1))
+    if out is not None:
+        return _to_nchw(out)
     pads = _same_pad(x, 3, 2)
     if pads[0] == 0 and pads[2] == 0:
         return F.max_pool2d(x, 3, 2, ceil_mode=True)
@@ -256,5 +260,5 @@ class ResNet18Var(torch.nn.Module):
             x = x.contiguous(memory_format=torch.channels_last)
         for unit in self.units:
             x = unit(x)
-        x = torch.relu(x).mean(dim=(2, 3))
-        return self.linear(x)
+        mean = _native.relu_mean(x.permute(0, 2, 3, 1))
+        return self.linear(mean if mean is not None else torch.relu(x).mean(dim=(2, 3)))

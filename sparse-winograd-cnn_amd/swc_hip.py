@@ -38,6 +38,7 @@ C_SYMBOLS = (
     "swc_winograd2x2_imtrans_grad_op_shape", "swc_winograd2x2_imtrans_grad_op_compute",
     "swc_winograd2x2_conv_grad", "swc_winograd2x2_imtrans_grad", "swc_winograd2x2_imtrans_grad_relu_input",
     "swc_winograd2x2_relu_conv", "swc_winograd2x2_pointwise_conv", "swc_winograd2x2_relu_pointwise_conv", "swc_stem_conv_pool",
+    "swc_max_pool_same", "swc_relu_mean",
 )
 # The two C++-linkage launchers with the reference's exact signatures (Itanium mangling).
 CXX_SYMBOLS = (
@@ -108,6 +109,9 @@ def lib():
         L.swc_winograd2x2_pointwise_conv.argtypes = [fp] * 3 + [i32, ctypes.c_longlong, i32, vp]
         L.swc_winograd2x2_relu_pointwise_conv.restype = i32
         L.swc_winograd2x2_relu_pointwise_conv.argtypes = [fp] * 5 + [i32, ctypes.c_longlong, i32, vp]
+        for f in (L.swc_max_pool_same, L.swc_relu_mean):
+            f.restype = i32
+            f.argtypes = [fp] * 2 + [i32] * 4 + [vp]
         L.swc_stem_conv_pool.restype = i32
         L.swc_stem_conv_pool.argtypes = [fp] * 3 + [i32] * 3 + [vp]
         L.swc_winograd2x2_conv_grad_static.restype = i32

@@ -137,3 +137,27 @@ def test_relu_pointwise_conv(shape, affine):
         got = resnet18_var.relu_pointwise_conv(y.to(dev), w1.to(dev), (a1.to(dev), b1.to(dev)) if affine else None).cpu()
         want = torch.relu(y) @ w1.t()
         assert torch.equal(torch.nan_to_num(got, 7.5, 9.5, 1.5), torch.nan_to_num(want, 7.5, 9.5, 1.5))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1, 1, 1, 4), (2, 1, 5, 64), (1, 2, 2, 68), (3, 7, 10, 64), (2, 14, 9, 132), (1, 17, 16, 512), (2, 5, 6, 30)])
+def test_model_pools(shape):
+    # Odd and even sides (padding in front or not), sums shorter than, as long as and longer than their sixteen parts, channels that are
+    # no whole workgroup, and 30 channels, which take torch's operators.  The mean adds n numbers: n * 2^-24 of their mean.
+    import resnet18_var
+    B, H, W, C = shape
+    x = torch.randn(shape, generator=torch.Generator().manual_seed(7))
+    nchw = x.permute(0, 3, 1, 2)
+    dev = torch.device("cuda:0")
+    pads = resnet18_var._same_pad(nchw, 3, 2)
+    for bad in (None, float("nan"), float("inf"), float("-inf")):
+        if bad is not None:
+            x[0, H // 2, W // 2, C // 2] = bad
+        got = resnet18_var._max_pool_same(nchw.to(dev)).cpu()
+        want = torch.nn.functional.max_pool2d(torch.nn.functional.pad(nchw, pads, value=float("-inf")), 3, 2)
+        assert torch.equal(torch.nan_to_num(got, 7.5), torch.nan_to_num(want, 7.5))
+        mean = resnet18_var._native.relu_mean(x.to(dev))
+        assert (mean is None) == (C % 4 != 0)
+        if mean is not None:
+            want = torch.relu(x.double()).mean(dim=(1, 2))
+            assert torch.allclose(mean.cpu().double(), want, rtol=H * W * 2.0 ** -24 + 2.0 ** -23, atol=0, equal_nan=True)
