@@ -167,6 +167,13 @@ SWC_API int swc_winograd2x2_conv_prepared(const float *Input, const float *Weigh
                                           const float *Scale, const float *Shift, const float *Residual, int residual_relu,
                                           int C, int B, int nH, int nW, int K, int pad_h, int pad_w, swc_stream_t stream);
 SWC_API int swc_winograd2x2_conv_pieces_gain(int C, int B, int nH, int nW, int K);
+/* The same for bf16 operands (swc_winograd2x2_conv_bf16): weights rounded to bf16, to nearest even, in that order. */
+SWC_API size_t swc_winograd2x2_weight_pieces_bf16_bytes(int C, int K);
+SWC_API int swc_winograd2x2_weight_pieces_bf16(const float *Weight, void *Pieces, int C, int K, swc_stream_t stream);
+SWC_API int swc_winograd2x2_conv_prepared_bf16(const float *Input, const float *Weight, const void *Pieces, float *Output, const float *Scale,
+                                               const float *Shift, const float *Residual, int residual_relu, int C, int B, int nH,
+                                               int nW, int K, int pad_h, int pad_w, swc_stream_t stream);
+SWC_API int swc_winograd2x2_conv_pieces_bf16_gain(int C, int B, int nH, int nW, int K);
 
 /*
  * Same contract as swc_winograd2x2_conv, with both GEMM operands rounded to bf16

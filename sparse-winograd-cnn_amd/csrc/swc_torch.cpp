@@ -157,8 +157,8 @@ PyObject *conv(PyObject *, PyObject *const *args, Py_ssize_t count)
     at::Tensor pieces;
     if (ok && args[7] != Py_None && !for_this_call) {
         const at::Tensor *p = plain(args[7], at::kByte, 1);
-        if (p == nullptr || bf16 || p->device() != I->device() ||
-            static_cast<size_t>(p->size(0)) != swc_winograd2x2_weight_pieces_bytes(as_int(C), as_int(K)))
+        if (p == nullptr || p->device() != I->device() ||
+            static_cast<size_t>(p->size(0)) != (bf16 ? swc_winograd2x2_weight_pieces_bf16_bytes : swc_winograd2x2_weight_pieces_bytes)(as_int(C), as_int(K)))
             return none();
         pieces = *p;
     }
@@ -175,7 +175,7 @@ PyObject *conv(PyObject *, PyObject *const *args, Py_ssize_t count)
             st = swc_winograd2x2_weight_pieces(floats(*W), pieces.mutable_data_ptr(), as_int(C), as_int(K), stream);
         }
         if (st == SWC_OK && pieces.defined())
-            st = swc_winograd2x2_conv_prepared(floats(*I), floats(*W), pieces.const_data_ptr(), floats_of(out), scale, shift, residual, residual_relu,
+            st = (bf16 ? swc_winograd2x2_conv_prepared_bf16 : swc_winograd2x2_conv_prepared)(floats(*I), floats(*W), pieces.const_data_ptr(), floats_of(out), scale, shift, residual, residual_relu,
                                                as_int(C), as_int(B), as_int(nH), as_int(nW), as_int(K), 1, 1, stream);
         else if (st == SWC_OK)
             st = swc_winograd2x2_conv_epilogue(floats(*I), floats(*W), floats_of(out), scale, shift, residual, residual_relu, as_int(C), as_int(B),
@@ -185,16 +185,18 @@ PyObject *conv(PyObject *, PyObject *const *args, Py_ssize_t count)
     END_HANDLE_TH_ERRORS
 }
 
-// pieces_gain(I, K): swc_winograd2x2_conv_pieces_gain for I [16,B,nH,nW,C], 0 where that is not I's shape
+// pieces_gain(I, K, bf16 operands): swc_winograd2x2_conv_pieces_gain or its bf16 sibling for I [16,B,nH,nW,C], 0 where that is not I's shape
 PyObject *pieces_gain(PyObject *, PyObject *const *args, Py_ssize_t count)
 {
-    SWC_ARGS(2)
+    SWC_ARGS(3)
     const long K = PyLong_AsLong(args[1]);
     if (K == -1 && PyErr_Occurred()) return nullptr;
     const at::Tensor *I = plain(args[0], at::kFloat, 5);
+    const int bf16 = PyObject_IsTrue(args[2]);
+    if (bf16 < 0) return nullptr;
     if (I == nullptr || I->size(0) != 16 || !fits(I->sizes()) || !fits({K})) return PyLong_FromLong(0);
     const c10::DeviceGuard guard(I->device());
-    return PyLong_FromLong(swc_winograd2x2_conv_pieces_gain(as_int(I->size(4)), as_int(I->size(1)), as_int(I->size(2)), as_int(I->size(3)), as_int(K)));
+    return PyLong_FromLong((bf16 ? swc_winograd2x2_conv_pieces_bf16_gain : swc_winograd2x2_conv_pieces_gain)(as_int(I->size(4)), as_int(I->size(1)), as_int(I->size(2)), as_int(I->size(3)), as_int(K)));
     END_HANDLE_TH_ERRORS
 }
 

@@ -93,9 +93,11 @@ ConvChoice choose_conv(const void *Input, const void *Weight, const void *Output
     // (39572x128->64 101.5 us against 95.6), for 15 %.  bf16 operands: 6 us + 9 per 64 channels at best (one tile per CU), at 32 channels as little as the split
     // forms' 6.5 to 8.5 + 4.1 to 5.  A direct form is offered only where it takes less.
     const double per64 = static_cast<double>(C) / 64;
+    // bf16 operands on more 64x64 tiles than CUs: the CUs share what the ring kernels are bound by, four fifths of a round for each one more.
+    const double tiles = static_cast<double>((M + 63) / 64) * ((K + 63) / 64) / device_cus(), ring_rounds = tiles > 1 ? 1 + 0.8 * (tiles - 1) : 1;
     const double scale = pick.tiling != TILING_WIDE48 && pick.tiling != TILING_WIDE48X64 ? 1.0 : C > 128 ? 0.9 : 0.85;
     choice.wide_scale = scale;
-    if (pick.tiling != TILING_SYNC) choice.whole_us = BF16 ? 6.0 + 9.0 * per64 : scale * (6.0 + 3.75 * pick.cost * per64);
+    if (pick.tiling != TILING_SYNC) choice.whole_us = BF16 ? (6.0 + 9.0 * per64) * ring_rounds : scale * (6.0 + 3.75 * pick.cost * per64);
     return choice;
 }
 
@@ -120,10 +122,10 @@ int conv_entry(const float *Input, const float *Weight, float *Output, int C, in
     hipStream_t s = static_cast<hipStream_t>(stream);
     const ConvChoice choice = choose_conv<BF16>(Input, Weight, Output, ep.residual, M, C, K);
     if (weight_pieces != nullptr) {
-        const PiecesChoice pieces = choose_pieces(Input, Weight, weight_pieces, Output, ep.residual, M, C, K);
+        const PiecesChoice pieces = choose_pieces(Input, Weight, weight_pieces, Output, ep.residual, M, C, K, BF16);
         if (pieces_gain(pieces, choice) > 0) {
             note_conv_kernel(kPiecesNames[pieces.form], kPiecesNames[pieces.form]);
-            return launch_pieces(pieces, Input, Weight, weight_pieces, Output, M, C, K, nW, ep.scale, ep.shift, ep.residual, ep.residual_relu, s);
+            return launch_pieces(pieces, BF16, Input, Weight, weight_pieces, Output, M, C, K, nW, ep.scale, ep.shift, ep.residual, ep.residual_relu, s);
         }
     }
     const TilingChoice &pick = choice.whole;
@@ -197,17 +199,36 @@ extern "C" int swc_winograd2x2_conv_prepared(const float *Input, const float *We
     return swc::conv_entry<false>(Input, Weight, Output, C, B, nH, nW, K, pad_h, pad_w, ep, stream, Pieces);
 }
 
-extern "C" int swc_winograd2x2_conv_pieces_gain(int C, int B, int nH, int nW, int K)
+extern "C" int swc_winograd2x2_conv_prepared_bf16(const float *Input, const float *Weight, const void *Pieces, float *Output, const float *Scale,
+                                                  const float *Shift, const float *Residual, int residual_relu, int C, int B, int nH,
+                                                  int nW, int K, int pad_h, int pad_w, swc_stream_t stream)
 {
-    using namespace swc;
+    swc::ConvEpilogue ep;
+    ep.scale = Scale;
+    ep.shift = Shift;
+    ep.residual = Residual;
+    ep.residual_relu = residual_relu != 0;
+    return swc::conv_entry<true>(Input, Weight, Output, C, B, nH, nW, K, pad_h, pad_w, ep, stream, Pieces);
+}
+
+namespace swc {
+namespace {
+template <bool BF16>
+int gain_of(int C, int B, int nH, int nW, int K)
+{
     if (C <= 0 || B <= 0 || nH <= 0 || nW <= 0 || K <= 0) return 0;
     const size_t M = static_cast<size_t>(B) * nH * nW;
     if (M >= (1ull << 31)) return 0;
-    const ConvChoice choice = choose_conv<false>(nullptr, nullptr, nullptr, nullptr, M, C, K);
-    const PiecesChoice pieces = choose_pieces(nullptr, nullptr, nullptr, nullptr, nullptr, M, C, K);
+    const ConvChoice choice = choose_conv<BF16>(nullptr, nullptr, nullptr, nullptr, M, C, K);
+    const PiecesChoice pieces = choose_pieces(nullptr, nullptr, nullptr, nullptr, nullptr, M, C, K, BF16);
     const double gain = pieces_gain(pieces, choice);
     return gain > 2.5 + 1.2 / (1 << 20) * 16 * C * K ? 2 : gain > 0 ? 1 : 0;
 }
+}  // namespace
+}  // namespace swc
+
+extern "C" int swc_winograd2x2_conv_pieces_gain(int C, int B, int nH, int nW, int K) { return swc::gain_of<false>(C, B, nH, nW, K); }
+extern "C" int swc_winograd2x2_conv_pieces_bf16_gain(int C, int B, int nH, int nW, int K) { return swc::gain_of<true>(C, B, nH, nW, K); }
 
 extern "C" int swc_winograd2x2_weights_bf16(const float *Weight, unsigned short *Weight16t, int C, int K,
                                             swc_stream_t stream)

@@ -34,10 +34,10 @@ size_t steps_of(int C) { return (static_cast<size_t>(C) + 31) / 32; }
 size_t groups_of(int K) { return (static_cast<size_t>(K) + 63) / 64; }
 
 // Bytes of the pieces of W [16,C,K]; 0 where the offsets within a position's 64 columns would not fit 31 bits.
-size_t pieces_bytes(int C, int K)
+size_t pieces_bytes(int C, int K, bool bf16 = false)
 {
     if (C <= 0 || K <= 0 || C > (1 << 17) || steps_of(C) * groups_of(K) >= (1ull << 27)) return 0;
-    return 16 * groups_of(K) * steps_of(C) * (4 * kPieces * 1024 + sizeof(float));
+    return 16 * groups_of(K) * steps_of(C) * (bf16 ? 4 * 1024 : 4 * kPieces * 1024 + sizeof(float));
 }
 
 // 16-byte loads of TI and the pieces, 32-bit byte offsets into a position's planes and 31-bit ones into the output; W itself is
@@ -49,6 +49,37 @@ bool pieces_eligible(const void *TI, const void *Wt, const void *Wp, const void 
            M * 16 * static_cast<size_t>(K) < (1ull << 31);
 }
 
+}  // namespace
+
+namespace {
+// bf16 operands, us (through what else runs / pieces; in brackets behind the transform).  One round of 32-row tiles, 3.6 + 3.3 per 64
+// channels, from 512 channels and 512 columns on (960x512->384 44.0 / 44.8 behind the transform), against split32
+//   1024x512->512 37.9 / 30.0 (47.7 / 42.5)
+// where the planes are few enough for the transform to leave them in the Infinity Cache (3200x384->72, 79 MB: 30.2 / 26.7, but 52.9 / 54.8).  Below,
+// some are faster (1568x256->256 27.7 / 25.6 behind the transform) and some slower (1392x128->320 17.7 / 23.2, 975x256->512 28.3 / 29.9).
+// More than a round of 64-row tiles, 6.8 per 64 channels less 2 each, against ring32, from 256 channels on and with columns for four tiles, which
+// share the planes
+//   4410x512->256 93.4 / 76.3 (152 / 126)      6272x512->512 203 / 181 (283 / 251)        6272x256->256 53.0 / 51.1 (95 / 85)
+//   5000x256->512 (132 / 95)                   3920x384->320 (126 / 98)                   4320x320->384 (113 / 96)
+//   12544x128->128 31.9 / 32.1: not taken
+// One round of 64-row tiles is no faster than split64 (3136x256->256 28.0 / 28.4, 2700x160->320 19.8 / 22.6).
+PiecesChoice choose_bf16(size_t M, int C, double c, size_t cus, size_t tiles_n)
+{
+    PiecesChoice best;
+    if (C % 64 != 0 || C < 256) return best;
+    auto rounds_of = [&](size_t rows, size_t high) { return static_cast<double>(((rows + high - 1) / high * tiles_n + cus - 1) / cus); };
+    if (rounds_of(M, 32) <= 1) {
+        if (C >= 512 && tiles_n >= 8 && M * C * 64 <= (64u << 20)) best = {PIECES_32, 0, 3.6 + 3.3 * c};
+        return best;
+    }
+    if (rounds_of(M, 64) <= 1 || tiles_n < 4) return best;
+    const double us64 = 6.8 * c - 2.0;
+    best = {PIECES_64, 0, rounds_of(M, 64) * us64};
+    const size_t whole = M / 64 * tiles_n / cus, main_m = whole * cus / tiles_n;
+    const double us = static_cast<double>(whole) * us64 + rounds_of(M - main_m * 64, 32) * 3.6 * c;
+    if (main_m * 64 < M && us < best.us) best = {PIECES_64_32, main_m, us};
+    return best;
+}
 }  // namespace
 
 // A workgroup fills a CU, so a launch takes rounds of tiles over the CUs.  Measured per round, 64-row tiles: 8 us + 8.25 per 64
@@ -64,7 +95,7 @@ bool pieces_eligible(const void *TI, const void *Wt, const void *Wp, const void 
 // Over 209 random shapes the choice made here was 5 % faster on the geometric mean where the best of all is 6 %.  Left out: fewer than
 // 64 channels (10000x32->48 14.7 us against 15.6, 3456x48->512 34 against 42), and planes that exceed the Infinity Cache and are
 // read by one column of tiles, which last as long as their bytes take (21756x320->64 129 us against 143.5, 14175x512->64 124 against 129).
-PiecesChoice choose_pieces(const void *TI, const void *Wt, const void *Wp, const void *Out, const void *residual, size_t M, int C, int K)
+PiecesChoice choose_pieces(const void *TI, const void *Wt, const void *Wp, const void *Out, const void *residual, size_t M, int C, int K, bool bf16)
 {
     PiecesChoice best;
     if (!pieces_eligible(TI, Wt, Wp, Out, residual, M, C, K)) return best;
@@ -76,6 +107,7 @@ PiecesChoice choose_pieces(const void *TI, const void *Wt, const void *Wp, const
     const size_t cus = device_cus(), tiles_n = groups_of(K);
     if (C < 64 || (tiles_n == 1 && M * C * 64 > kInfinityCacheBytes)) return best;
     const double c = static_cast<double>(C) / 64;
+    if (bf16) return choose_bf16(M, C, c, cus, tiles_n);
     auto rounds_of = [&](size_t rows, size_t high) { return static_cast<double>(((rows + high - 1) / high * tiles_n + cus - 1) / cus); };
     auto us64 = [&](double rounds) { return 1.0 + rounds * (8.0 + 8.25 * c); };
     const double us32 = 2.5 + 0.4 * c + rounds_of(M, 32) * (2.5 + 5.9 * c);
@@ -93,7 +125,7 @@ PiecesChoice choose_pieces(const void *TI, const void *Wt, const void *Wp, const
     return best;
 }
 
-int launch_pieces(const PiecesChoice &pick, const float *TI, const float *Wt, const void *Wp, float *Out, size_t M, int C, int K, int nW,
+int launch_pieces(const PiecesChoice &pick, bool bf16, const float *TI, const float *Wt, const void *Wp, float *Out, size_t M, int C, int K, int nW,
                   const float *scale, const float *shift, const float *residual, int residual_relu, hipStream_t s)
 {
     ConvEpilogue ep;
@@ -102,6 +134,21 @@ int launch_pieces(const PiecesChoice &pick, const float *TI, const float *Wt, co
     ep.residual = residual;
     ep.residual_relu = residual_relu;
     const bool ragged = C % 16 != 0, deep = steps_of(C) % 2 == 0 && !ragged;
+    if (bf16) {
+        const bool whole = C % 64 == 0;   // otherwise what lies beyond C is read as zero: beside it there may be an infinity
+        using R32 = PiecesCfg<1, 2, true, 1>;
+        using R64 = PiecesCfg<2, 2, true, 1>;
+        using D32 = PiecesCfg<1, 4, false, 1>;
+        using D64 = PiecesCfg<2, 4, false, 1>;
+        switch (pick.form) {   // twice the half steps on their way where C takes them
+            case PIECES_64: return whole ? launch_as<D64>(TI, Wt, Wp, Out, M, C, K, nW, 0, ep, s) : launch_as<R64>(TI, Wt, Wp, Out, M, C, K, nW, 0, ep, s);
+            case PIECES_32: return whole ? launch_as<D32>(TI, Wt, Wp, Out, M, C, K, nW, 0, ep, s) : launch_as<R32>(TI, Wt, Wp, Out, M, C, K, nW, 0, ep, s);
+            case PIECES_64_32:
+                return whole ? launch_as<D64, D32>(TI, Wt, Wp, Out, M, C, K, nW, pick.main_m, ep, s)
+                            : launch_as<R64, R32>(TI, Wt, Wp, Out, M, C, K, nW, pick.main_m, ep, s);
+            default: return SWC_ERR_UNSUPPORTED;
+        }
+    }
     switch (pick.form) {
         case PIECES_64:
             return ragged ? launch_as<PiecesCfg<2, 2, true>>(TI, Wt, Wp, Out, M, C, K, nW, 0, ep, s)
@@ -119,16 +166,31 @@ int launch_pieces(const PiecesChoice &pick, const float *TI, const float *Wt, co
 
 }  // namespace swc
 
-extern "C" size_t swc_winograd2x2_weight_pieces_bytes(int C, int K) { return swc::pieces_bytes(C, K); }
-
-extern "C" int swc_winograd2x2_weight_pieces(const float *Weight, void *Pieces, int C, int K, swc_stream_t stream)
+namespace swc {
+namespace {
+template <int NP>
+int make_pieces(const float *Weight, void *Pieces, int C, int K, swc_stream_t stream)
 {
-    using namespace swc;
     if (Weight == nullptr || Pieces == nullptr) return SWC_ERR_NULL_POINTER;
     if (C <= 0 || K <= 0 || pieces_bytes(C, K) == 0) return SWC_ERR_BAD_DIMS;
     if (!aligned16(Pieces)) return SWC_ERR_UNSUPPORTED;
     const unsigned groups = static_cast<unsigned>(groups_of(K)), steps = static_cast<unsigned>(steps_of(C));
-    weight_pieces_kernel<<<dim3(16 * groups * steps), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(Weight, static_cast<char *>(Pieces), C,
-                                                                                                        K, groups, steps);
+    weight_pieces_kernel<NP><<<dim3(16 * groups * steps), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(
+        Weight, static_cast<char *>(Pieces), C, K, groups, steps);
     return check_launch();
+}
+}  // namespace
+}  // namespace swc
+
+extern "C" size_t swc_winograd2x2_weight_pieces_bytes(int C, int K) { return swc::pieces_bytes(C, K); }
+extern "C" size_t swc_winograd2x2_weight_pieces_bf16_bytes(int C, int K) { return swc::pieces_bytes(C, K, true); }
+
+extern "C" int swc_winograd2x2_weight_pieces(const float *Weight, void *Pieces, int C, int K, swc_stream_t stream)
+{
+    return swc::make_pieces<swc::kPieces>(Weight, Pieces, C, K, stream);
+}
+
+extern "C" int swc_winograd2x2_weight_pieces_bf16(const float *Weight, void *Pieces, int C, int K, swc_stream_t stream)
+{
+    return swc::make_pieces<1>(Weight, Pieces, C, K, stream);
 }

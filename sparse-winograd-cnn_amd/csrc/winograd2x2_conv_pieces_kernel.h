@@ -29,10 +29,15 @@ namespace {
 // a wave's step, of 56 bytes a clock at most.  With both operands in the L1 (timed on a copy) 14x14x256 at batch 64 takes 36.8 us
 // instead of 43.6.  With 32 rows a step is 16 KiB for 24 MFMAs, which is bound by the L2 alone; twice the half steps on their way
 // (HB 4, registers allow it there) make 7x7x512 at batch 64 57.4 -> 55.3 us.
+//
+// bf16 operands are the same with one piece (NP 1) and one product: no second look at the operands, whose rounding the caller asked
+// for, and the sums of even and odd half steps by themselves, so that a sum is rounded as often as with 32 indices to an instruction.
+// That form is bound by what the L2 hands a CU, of which prepared weights are half.
 constexpr int kPieces = 3;
 
-template <int TM_, int HB_, bool RAGGED_>
+template <int TM_, int HB_, bool RAGGED_, int NP_ = kPieces>
 struct PiecesCfg {
+    static constexpr int NP = NP_;
     static constexpr int TM = TM_, TN = 2;
     static constexpr int HB = HB_, RA = HB / 2;              // half steps of weights and of TI on their way
     static constexpr bool RAGGED = RAGGED_;                  // C is no multiple of 16
@@ -41,21 +46,22 @@ struct PiecesCfg {
     static constexpr int NT = 512;
     static constexpr int STAGE = WM * 16;                    // floats a wave turns A round in: all rows x 16 indices
     static constexpr int LDS_BYTES = 8 * (E + STAGE) * 4;
-    static constexpr int HALF_BYTES = TN * kPieces * 1024;        // prepared weights of 16 indices x 64 columns
+    static constexpr int HALF_BYTES = TN * NP * 1024;             // prepared weights of 16 indices x 64 columns
     static_assert(LDS_BYTES <= 160 * 1024, "a CU has 160 KiB of LDS");
 };
 
 // Eight values into pieces, each the bf16 value nearest to what the ones before leave.
-__device__ __forceinline__ void pieces_of8(const floatx4 &u, const floatx4 &w, intx4 (&out)[kPieces])
+template <int NP>
+__device__ __forceinline__ void pieces_of8(const floatx4 &u, const floatx4 &w, intx4 (&out)[NP])
 {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         floatx2 x = q < 2 ? floatx2{u[2 * q], u[2 * q + 1]} : floatx2{w[2 * q - 4], w[2 * q - 3]};
 #pragma unroll
-        for (int p = 0; p < kPieces; ++p) {
+        for (int p = 0; p < NP; ++p) {
             const bf16x2 h = __builtin_convertvector(x, bf16x2);
             out[p][q] = __builtin_bit_cast(int, h);
-            if (p + 1 == kPieces) break;
+            if (p + 1 == NP) break;
             x[0] -= static_cast<float>(h[0]);
             x[1] -= static_cast<float>(h[1]);
         }
@@ -76,7 +82,7 @@ __device__ __forceinline__ void pieces_tiles(const float *__restrict__ TI, const
                                              float *__restrict__ Out, unsigned M, int C, int K, int nW, unsigned count, TileOf tile_of,
                                              float *P, const ConvEpilogue ep)
 {
-    constexpr int TM = Cfg::TM, TN = Cfg::TN, E = Cfg::E, NP = kPieces;
+    constexpr int TM = Cfg::TM, TN = Cfg::TN, E = Cfg::E, NP = Cfg::NP;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, li = lane & 31, lg = lane >> 5;
     const unsigned groups = (static_cast<unsigned>(K) + 63) / 64, steps = (static_cast<unsigned>(C) + 31) / 32;
@@ -143,7 +149,7 @@ __device__ __forceinline__ void pieces_tiles(const float *__restrict__ TI, const
                 *reinterpret_cast<floatx2 *>(&P[wave * E + (tm * 32 + 8 * (r / 4) + 4 * lg + r % 4) * 64 + 2 * li]) = v;
             }
     };
-    auto again_in_fp32 = [&](const __amdgpu_buffer_rsrc_t a_desc, const __amdgpu_buffer_rsrc_t b_desc) __attribute__((always_inline)) {
+    [[maybe_unused]] auto again_in_fp32 = [&](const __amdgpu_buffer_rsrc_t a_desc, const __amdgpu_buffer_rsrc_t b_desc) __attribute__((always_inline)) {
         zero_acc();
         const int n = static_cast<int>(t.tn_id) * Cfg::WN + 2 * li;
         const unsigned b_off = (static_cast<unsigned>(lg * 4) * K + (n + 2 <= K ? n : K - 2)) * 4u;
@@ -170,7 +176,7 @@ __device__ __forceinline__ void pieces_tiles(const float *__restrict__ TI, const
     };
 
     // the largest magnitudes of W, one for every 32 indices x 64 columns, behind the pieces
-    const float *const w_most = reinterpret_cast<const float *>(Wp + static_cast<size_t>(16) * groups * p_bytes);
+    [[maybe_unused]] const float *const w_most = reinterpret_cast<const float *>(Wp + static_cast<size_t>(16) * groups * p_bytes);
 
     floatx4 fr[TM][2];   // raw operands of the half step behind the one multiplied
     auto put_a = [&](auto slot_tag) __attribute__((always_inline)) {
@@ -190,11 +196,11 @@ __device__ __forceinline__ void pieces_tiles(const float *__restrict__ TI, const
     float most = 0.f;    // the largest magnitude among the operands of a lane
     auto take_a = [&](int tm, int to) __attribute__((always_inline)) {
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
+        for (int q = 0; q < (NP == 1 ? 0 : 2); ++q)
 #pragma unroll
             for (int i = 0; i < 4; i += 2)
                 most = __builtin_fmaxf(__builtin_fmaxf(most, __builtin_fabsf(fr[tm][q][i])), __builtin_fabsf(fr[tm][q][i + 1]));
-        pieces_of8(fr[tm][0], fr[tm][1], as[to]);
+        pieces_of8<NP>(fr[tm][0], fr[tm][1], as[to]);
     };
     auto multiply = [&](int tm, int from, auto buf_tag) __attribute__((always_inline)) {
         constexpr int buf = decltype(buf_tag)::value;
@@ -202,17 +208,25 @@ __device__ __forceinline__ void pieces_tiles(const float *__restrict__ TI, const
             return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, x), __builtin_bit_cast(bf16x8, y), c, 0, 0, 0);
         };
         const intx4(&a)[NP] = as[from];
+        if constexpr (NP == 1) {
+#pragma unroll
+            for (int tn = 0; tn < TN; ++tn) {
+                floatx16 &sum = buf % 2 == 0 ? acc[tm][tn] : crs[tm][tn];
+                sum = mfma(a[0], bs[buf][tn][0], sum);
+            }
+            return;
+        }
         constexpr int order[5][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}};   // l.h, h.l, m.m, m.h, h.m
 #pragma unroll
         for (int i = 0; i < 5; ++i)
 #pragma unroll
-            for (int tn = 0; tn < TN; ++tn) crs[tm][tn] = mfma(a[order[i][0]], bs[buf][tn][order[i][1]], crs[tm][tn]);
+            for (int tn = 0; tn < TN; ++tn) crs[tm][tn] = mfma(a[order[i][0] % NP], bs[buf][tn][order[i][1] % NP], crs[tm][tn]);
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = mfma(a[0], bs[buf][tn][0], acc[tm][tn]);
     };
     auto interleave = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 6 * TN; ++i) {
+        for (int i = 0; i < (NP == 1 ? 0 : 6 * TN); ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // a matrix instruction,
             __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);   // five vector ones
         }
@@ -271,6 +285,15 @@ __device__ __forceinline__ void pieces_tiles(const float *__restrict__ TI, const
                 load_b(ks_tag, pn, dead ? 0 : hn + ks);
                 __builtin_amdgcn_sched_barrier(0);
             });
+        }
+        if constexpr (NP == 1) {
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+                for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[tm][tn][r] = acc[tm][tn][r] + crs[tm][tn][r];
+            return;
         }
         float none = 0.f, low = __builtin_inff();   // NaN where a sum is not finite; the smallest sum
 #pragma unroll
@@ -368,7 +391,8 @@ __global__ __launch_bounds__(Main::NT) __attribute__((amdgpu_waves_per_eu(2, 2))
 
 // W [16,C,K] into pieces, in the order in which a wave reads them: [position][64 columns][16 indices][tn][piece][lane][8], and
 // behind them the largest magnitude of every 32 indices x 64 columns.  A workgroup takes those of one position; what lies
-// beyond C or K is zero.  Bound by memory: 10 bytes a value, 2.5 us and 1.2 us for every 2^20 values (512x512: 7.6 us).
+// beyond C or K is zero.  With one piece there are no magnitudes.  Bound by memory: 10 bytes a value, 2.5 us and 1.2 us for every 2^20 values (512x512: 7.6 us).
+template <int NP>
 __global__ __launch_bounds__(256) void weight_pieces_kernel(const float *__restrict__ Wt, char *__restrict__ Wp, int C, int K, unsigned groups,
                                                             unsigned steps)
 {
@@ -383,17 +407,18 @@ __global__ __launch_bounds__(256) void weight_pieces_kernel(const float *__restr
         v[i / 4][i % 4] = n < K && k + i < C ? Wt[(static_cast<size_t>(pos) * C + k + i) * K + n] : 0.f;
         most = __builtin_fmaxf(most, __builtin_fabsf(v[i / 4][i % 4]));
     }
-    intx4 out[kPieces];
-    pieces_of8(v[0], v[1], out);
-    char *const to = Wp + (((static_cast<size_t>(pg) * steps + s) * 2 + ks) * 2 + tn) * (kPieces * 1024) + lane * 16;
+    intx4 out[NP];
+    pieces_of8<NP>(v[0], v[1], out);
+    char *const to = Wp + (((static_cast<size_t>(pg) * steps + s) * 2 + ks) * 2 + tn) * (NP * 1024) + lane * 16;
 #pragma unroll
-    for (int p = 0; p < kPieces; ++p) *reinterpret_cast<intx4 *>(to + p * 1024) = out[p];
+    for (int p = 0; p < NP; ++p) *reinterpret_cast<intx4 *>(to + p * 1024) = out[p];
+    if (NP == 1) return;
 #pragma unroll
     for (int d = 32; d > 0; d /= 2) most = __builtin_fmaxf(most, __shfl_xor(most, d));
     if (lane == 0) most_of[threadIdx.x >> 6] = most;
     __syncthreads();
     if (threadIdx.x == 0) {
-        float *const w_most = reinterpret_cast<float *>(Wp + static_cast<size_t>(16) * groups * steps * (4 * kPieces * 1024));
+        float *const w_most = reinterpret_cast<float *>(Wp + static_cast<size_t>(16) * groups * steps * (4 * NP * 1024));
         w_most[blockIdx.x] = __builtin_fmaxf(__builtin_fmaxf(most_of[0], most_of[1]), __builtin_fmaxf(most_of[2], most_of[3]));
     }
 }

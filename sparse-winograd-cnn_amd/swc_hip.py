@@ -28,7 +28,8 @@ C_SYMBOLS = (
     "swc_winograd2x2_imtrans", "swc_winograd2x2_imtrans_affine", "swc_winograd2x2_conv", "swc_winograd2x2_conv_bf16",
     "swc_winograd2x2_conv_epilogue",
     "swc_winograd2x2_weight_pieces_bytes", "swc_winograd2x2_weight_pieces", "swc_winograd2x2_conv_prepared",
-    "swc_winograd2x2_conv_pieces_gain",
+    "swc_winograd2x2_conv_pieces_gain", "swc_winograd2x2_weight_pieces_bf16_bytes", "swc_winograd2x2_weight_pieces_bf16",
+    "swc_winograd2x2_conv_prepared_bf16", "swc_winograd2x2_conv_pieces_bf16_gain",
     "swc_winograd2x2_imtrans_bf16out", "swc_winograd2x2_weights_bf16", "swc_winograd2x2_conv_bf16in",
     "swc_winograd2x2_conv_bf16in_ws", "swc_winograd2x2_conv_bf16in_workspace_floats",
     "swc_winograd2x2_relu_conv_bf16",
@@ -125,14 +126,18 @@ def lib():
             f.argtypes = [fp, fp, fp, fp, vp] + [i32] * 7 + [vp]
         L.swc_winograd2x2_conv_epilogue.restype = i32
         L.swc_winograd2x2_conv_epilogue.argtypes = [fp] * 6 + [i32] * 9 + [vp]
-        L.swc_winograd2x2_weight_pieces_bytes.restype = ctypes.c_size_t
-        L.swc_winograd2x2_weight_pieces_bytes.argtypes = [i32] * 2
-        L.swc_winograd2x2_weight_pieces.restype = i32
-        L.swc_winograd2x2_weight_pieces.argtypes = [fp, fp, i32, i32, vp]
-        L.swc_winograd2x2_conv_prepared.restype = i32
-        L.swc_winograd2x2_conv_prepared.argtypes = [fp] * 7 + [i32] * 8 + [vp]
-        L.swc_winograd2x2_conv_pieces_gain.restype = i32
-        L.swc_winograd2x2_conv_pieces_gain.argtypes = [i32] * 5
+        for f in (L.swc_winograd2x2_weight_pieces_bytes, L.swc_winograd2x2_weight_pieces_bf16_bytes):
+            f.restype = ctypes.c_size_t
+            f.argtypes = [i32] * 2
+        for f in (L.swc_winograd2x2_weight_pieces, L.swc_winograd2x2_weight_pieces_bf16):
+            f.restype = i32
+            f.argtypes = [fp, fp, i32, i32, vp]
+        for f in (L.swc_winograd2x2_conv_prepared, L.swc_winograd2x2_conv_prepared_bf16):
+            f.restype = i32
+            f.argtypes = [fp] * 7 + [i32] * 8 + [vp]
+        for f in (L.swc_winograd2x2_conv_pieces_gain, L.swc_winograd2x2_conv_pieces_bf16_gain):
+            f.restype = i32
+            f.argtypes = [i32] * 5
         L.swc_winograd2x2_imtrans_bf16out.restype = i32
         L.swc_winograd2x2_imtrans_bf16out.argtypes = [fp, fp, fp, fp] + [i32] * 7 + [vp]
         L.swc_winograd2x2_weights_bf16.restype = i32

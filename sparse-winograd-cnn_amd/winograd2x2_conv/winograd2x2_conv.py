@@ -81,7 +81,8 @@ def _forward(I, W, precision, out, scale=None, shift=None, residual=None, residu
             if precision == "fp32" and swc_hip.lib().swc_winograd2x2_conv_pieces_gain(C, B, nH, nW, shape[3]) == 2:
                 pieces = winograd2x2_weight_pieces(W)
         if pieces is not None:
-            st = swc_hip.lib().swc_winograd2x2_conv_prepared(
+            prepared = swc_hip.lib().swc_winograd2x2_conv_prepared_bf16 if precision == "bf16" else swc_hip.lib().swc_winograd2x2_conv_prepared
+            st = prepared(
                 I.data_ptr(), W.data_ptr(), pieces.data_ptr(), out.data_ptr(), None if scale is None else scale.data_ptr(),
                 None if shift is None else shift.data_ptr(), None if residual is None else residual.data_ptr(),
                 int(bool(residual_relu)), C, B, nH, nW, shape[3], 1, 1, stream)
@@ -98,18 +99,21 @@ def _forward(I, W, precision, out, scale=None, shift=None, residual=None, residu
     return out
 
 
-def winograd2x2_weight_pieces(W):
+def winograd2x2_weight_pieces(W, precision="fp32"):
     """W [16,C,K] float32 -> the bytes ``winograd2x2_conv(..., pieces=...)`` multiplies with: every weight as three bfloat16
-    values whose sum it is.  Prepare once per weight update."""
+    values whose sum it is, or with ``precision="bf16"`` rounded to one.  Prepare once per weight update."""
     W = swc_hip.require_cuda_f32(W, "W", 3)
     if W.shape[0] != 16:
         raise ValueError("W must have shape [16,C,K]")
-    n = swc_hip.lib().swc_winograd2x2_weight_pieces_bytes(W.shape[1], W.shape[2])
+    L = swc_hip.lib()
+    size, make = {"fp32": (L.swc_winograd2x2_weight_pieces_bytes, L.swc_winograd2x2_weight_pieces),
+                  "bf16": (L.swc_winograd2x2_weight_pieces_bf16_bytes, L.swc_winograd2x2_weight_pieces_bf16)}[precision]
+    n = size(W.shape[1], W.shape[2])
     if n == 0:
         raise ValueError("W of shape %s is empty or too large to be taken apart" % (tuple(W.shape),))
     out = torch.empty(n, dtype=torch.uint8, device=W.device)
     with swc_hip.on_device(W.device) as stream:
-        st = swc_hip.lib().swc_winograd2x2_weight_pieces(W.data_ptr(), out.data_ptr(), W.shape[1], W.shape[2], stream)
+        st = make(W.data_ptr(), out.data_ptr(), W.shape[1], W.shape[2], stream)
     swc_hip.check(st, "winograd2x2_weight_pieces")
     return out
 
@@ -235,8 +239,8 @@ def winograd2x2_conv(I, W, precision="fp32", out=None, scale=None, shift=None, r
     The bf16-stored kernel gets a temporary of the size its launcher asks for (most shapes: none), as the
     reference's op allocates its launcher's (winograd2x2_conv_op.cc:57-60); ``workspace=False`` calls it without.
 
-    ``pieces`` (fp32 only): what ``winograd2x2_weight_pieces`` made of this W, which is then multiplied with where that is
-    the faster way, or True: made here where even that is faster.  The same result to fp32 rounding.
+    ``pieces``: what ``winograd2x2_weight_pieces`` made of this W for this precision, which is then multiplied with where that is
+    the faster way, or True: made here where even that is faster (fp32 only).  The same result to fp32 rounding.
 
     ``precision="bf16"`` rounds both GEMM operands to bf16 (fp32 accumulate).  Differentiable
     through ``winograd2x2_conv_grad`` when an input requires grad.
@@ -250,11 +254,10 @@ def winograd2x2_conv(I, W, precision="fp32", out=None, scale=None, shift=None, r
     if residual_relu and residual is None:
         raise ValueError("residual_relu needs a residual")
     if pieces is not None and pieces is not True:
-        if precision != "fp32":
-            raise ValueError("pieces are fp32 weights'")
+        size = swc_hip.lib().swc_winograd2x2_weight_pieces_bf16_bytes if precision == "bf16" else swc_hip.lib().swc_winograd2x2_weight_pieces_bytes
         if not isinstance(W, torch.Tensor) or W.dim() != 3 or pieces.dtype != torch.uint8 or pieces.device != W.device or \
-                not pieces.is_contiguous() or pieces.numel() != swc_hip.lib().swc_winograd2x2_weight_pieces_bytes(*W.shape[1:]):
-            raise ValueError("pieces must be what winograd2x2_weight_pieces made of W")
+                not pieces.is_contiguous() or pieces.numel() != size(*W.shape[1:]):
+            raise ValueError("pieces must be what winograd2x2_weight_pieces made of W for this precision")
     if (scale is not None or residual is not None) and needs_grad:
         raise NotImplementedError("the scale/shift/residual epilogue is forward only")
     if needs_grad:

@@ -78,11 +78,11 @@ class WinogradConv(torch.nn.Module):
         return cached[1]
 
     def weight_pieces(self):
-        """W*mask taken apart for the fp32 convolution; cached like masked_weight()."""
-        key = self._weight_key()
+        """W*mask taken apart for the fp32 convolution, or rounded and put in order for the one with bf16 operands; cached like masked_weight()."""
+        key = (self._weight_key(), self.precision)
         cached = self._pieces
         if cached is None or cached[0] != key:
-            cached = (key, winograd2x2_conv.winograd2x2_conv.winograd2x2_weight_pieces(self.masked_weight()))
+            cached = (key, winograd2x2_conv.winograd2x2_conv.winograd2x2_weight_pieces(self.masked_weight(), self.precision))
             self._pieces = cached
         return cached[1]
 
@@ -110,11 +110,11 @@ class WinogradConv(torch.nn.Module):
             pieces = True
         else:
             w = self.masked_weight()
-            if self.precision == "fp32":
-                # the cached pieces where W*mask is cached too, pieces made for this call where W itself is used
-                if self.mask is None:
-                    pieces = True
-                elif _native.pieces_gain(x, self.out_channel) and x.device == w.device and x.shape[4] == w.shape[1]:
+            # the cached pieces where W*mask is cached too, pieces made for this call where W itself is used
+            if self.mask is None:
+                pieces = True
+            elif self.precision in ("fp32", "bf16"):
+                if _native.pieces_gain(x, self.out_channel, self.precision == "bf16") and x.device == w.device and x.shape[4] == w.shape[1]:
                     pieces = self.weight_pieces()
         scale, shift = affine if affine is not None else (None, None)
         return winograd2x2_conv.winograd2x2_conv.winograd2x2_conv(x, w, self.precision, None, scale, shift, residual, residual_relu, True, pieces)

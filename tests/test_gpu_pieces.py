@@ -179,3 +179,62 @@ def test_pieces_that_are_not_the_weights_are_refused():
             winograd2x2_conv(ti, w, pieces=bad)
     with pytest.raises(ValueError):
         winograd2x2_conv(ti, w, precision="bf16", pieces=pieces)
+
+
+@pytest.mark.parametrize("form", ["pieces32", "pieces64", "pieces64+32"])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 4, 4), (1, 4, 8, 48, 64), (2, 5, 6, 64, 68), (1, 13, 5, 80, 132), (2, 8, 8, 128, 64), (3, 9, 7, 320, 200)])
+def test_bf16_operands(shape, form):
+    # Rows, columns and channels below, at and beyond a tile (32 or 64 rows, 64 columns, half steps of 16 indices, four of them on their
+    # way where C % 64 == 0).  Whole numbers are exact in bf16 and in any order of the sums; for others the kernel's products are those of
+    # the rounded operands, summed in fp32: at most C roundings of 2^-24 each for sums of at most sum|a b|.
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv, winograd2x2_weight_pieces
+    import swc_hip
+    B, nH, nW, C, K = shape
+    gen = torch.Generator().manual_seed(17)
+    dev = torch.device("cuda:0")
+    whole = [torch.randint(-4, 5, s, generator=gen).float() for s in ((16, B, nH, nW, C), (16, C, K))]
+    real = [torch.relu(torch.randn((16, B, nH, nW, C), generator=gen)), torch.randn((16, C, K), generator=gen)]
+    lib = swc_hip.lib()
+
+    def conv(ti, w, name):
+        pieces = winograd2x2_weight_pieces(w.to(dev), "bf16")
+        assert lib.swc_winograd2x2_conv_force_tiling(name.encode() if name else None) == 0
+        try:
+            return winograd2x2_conv(ti.to(dev), w.to(dev), "bf16", pieces=pieces if name else None).cpu()
+        finally:
+            lib.swc_winograd2x2_conv_force_tiling(None)
+    assert torch.equal(conv(*whole, form), conv(*whole, None))
+    ti, w = (v.bfloat16().double() for v in real)
+
+    def out_of(p):   # A^T p A in float64, p [16,B,nH,nW,K]; with magnitudes for the bound
+        return p.reshape(4, 4, B, nH, nW, K)
+    a = torch.tensor([[1, 1, 1, 0], [0, 1, -1, -1]], dtype=torch.float64)
+    p = out_of(torch.matmul(ti.reshape(16, -1, C), w))
+    size = out_of(torch.matmul(ti.reshape(16, -1, C).abs(), w.abs()))
+    fold = lambda m, q: torch.einsum("ai,bj,ijnhwk->nhawbk", m, m, q).reshape(B, 2 * nH, 2 * nW, K)   # noqa: E731
+    got = conv(*real, form).double()
+    assert ((got - fold(a, p)).abs() <= (C + 16) * 2.0 ** -24 * fold(a.abs(), size)).all()
+    # an infinity stays in its own tile's outputs
+    bad = real[0].clone()
+    bad[5, 0, nH - 1, nW - 1, 0] = float("inf")
+    got, want = conv(bad, real[1], form), conv(bad, real[1], None)
+    assert torch.equal(got.isfinite(), want.isfinite())
+    assert (~got.isfinite()).sum() == 4 * K
+
+
+@pytest.mark.parametrize("masked", [True, False])
+def test_a_bf16_layer_is_the_op_on_its_weights(masked):
+    # 7x7x512 at batch 64 is multiplied with the layer's prepared weights where it has a mask; a write to them is noticed.
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv
+    from winograd_conv import WinogradConv
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(23)
+    ti = torch.randint(0, 5, (16, 64, 4, 4, 512), device=dev, generator=gen).float()
+    mask = (torch.rand((16, 512, 512), device=dev, generator=gen) < 0.3).float() if masked else None
+    layer = WinogradConv(512, 512, mask=mask, W_init=torch.randint(-4, 5, (16, 512, 512), device=dev, generator=gen).float(), device=dev, precision="bf16")
+    with torch.no_grad():
+        for _ in range(2):
+            w = layer.W.detach() if mask is None else layer.W.detach() * mask
+            assert torch.equal(layer(ti), winograd2x2_conv(ti, w, "bf16"))
+            assert (layer._pieces is not None) == masked
+            layer.W.mul_(2)
