@@ -310,7 +310,8 @@ SWC_API int swc_winograd2x2_relu_conv_bf16(const float *Input, const float *InSc
 SWC_API int swc_winograd2x2_pointwise_conv(const float *Input, const float *Weight, float *Output, int C, long long M,
                                            int K, swc_stream_t stream);
 /* The same of relu(Input), or with Scale and Shift [C] of relu(Input*Scale + Shift), applied as the input is read: the ReLU or BNReLU
- * in front of those shortcuts (:125, :151, :176, :201).  With Scale and Shift, C <= 4096 (SWC_ERR_UNSUPPORTED beyond). */
+ * in front of those shortcuts (:125, :151, :176, :201), product and sum each rounded.  With Scale and Shift, C <= 4096
+ * (SWC_ERR_UNSUPPORTED beyond). */
 SWC_API int swc_winograd2x2_relu_pointwise_conv(const float *Input, const float *Scale, const float *Shift, const float *Weight,
                                                 float *Output, int C, long long M, int K, swc_stream_t stream);
 

@@ -522,8 +522,18 @@ constexpr int async_lds_bytes()
 // independent, so its launcher may deal groups of positions to different workgroups.
 // ACT (dgrad mode): what A's values go through between LDS and the matrix instruction.  RING_RELU: relu(a), with NaN kept;
 // RING_AFFINE_RELU: relu(a*ep.scale[r] + ep.shift[r]) by reduction index r, both vectors kept in LDS behind the ring (2*R floats).
-// One to three vector instructions per 64-cycle matrix instruction, which hides them.
+// Two to four vector instructions per 64-cycle matrix instruction.
 enum RingAct { RING_PLAIN = 0, RING_RELU = 1, RING_AFFINE_RELU = 2 };
+
+// a*scale + shift with the product and the sum each rounded, as a pass of its own in front of the product (torch.addcmul) does: the
+// values are the same to the bit.
+__device__ __forceinline__ float scaled(float a, float scale, float shift)
+{
+#pragma clang fp contract(off)
+    const float product = a * scale;
+    return product + shift;
+}
+
 template <typename Cfg, int NSTAGE, bool BF16, int MODE, int NPOS = 16, int ACT = RING_PLAIN>
 __device__ __forceinline__ void conv_ring_body(const float *__restrict__ TI, const float *__restrict__ Wt,
                                                float *__restrict__ Out, size_t M, int R, int N, int nW, const size_t m0,
@@ -848,8 +858,7 @@ __device__ __forceinline__ void conv_ring_body(const float *__restrict__ TI, con
                 float av = t == 0 ? a4.x : t == 1 ? a4.y : t == 2 ? a4.z : a4.w;
                 if constexpr (ACT == RING_AFFINE_RELU) {
                     const float4 sc = F.scale[k8l], sh = F.shift[k8l];
-                    av = t == 0 ? __builtin_fmaf(av, sc.x, sh.x) : t == 1 ? __builtin_fmaf(av, sc.y, sh.y)
-                       : t == 2 ? __builtin_fmaf(av, sc.z, sh.z) : __builtin_fmaf(av, sc.w, sh.w);
+                    av = t == 0 ? scaled(av, sc.x, sh.x) : t == 1 ? scaled(av, sc.y, sh.y) : t == 2 ? scaled(av, sc.z, sh.z) : scaled(av, sc.w, sh.w);
                 }
                 if constexpr (ACT != RING_PLAIN) av = av < 0.0f ? 0.0f : av;
                 float bv;

@@ -139,6 +139,20 @@ def test_relu_pointwise_conv(shape, affine):
         assert torch.equal(torch.nan_to_num(got, 7.5, 9.5, 1.5), torch.nan_to_num(want, 7.5, 9.5, 1.5))
 
 
+@pytest.mark.parametrize("affine", [False, True])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 32, 1), (2, 9, 11, 64, 64), (1, 8, 8, 96, 72), (1, 2, 3, 4128, 8)])
+def test_relu_pointwise_conv_rounds_as_separate_passes(shape, affine):
+    # The same bits as the BatchNorm's product and sum, the ReLU and the product one after the other, whichever way is taken: a model's
+    # later layers turn a last bit into another bf16 rounding.
+    import resnet18_var
+    B, H, W, C, K = shape
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    x, w = torch.randn((B, H, W, C), device="cuda", generator=gen), torch.randn((K, C), device="cuda", generator=gen)
+    a, b = torch.rand(C, device="cuda", generator=gen) + 0.5, torch.randn(C, device="cuda", generator=gen) * 0.1
+    got = resnet18_var.relu_pointwise_conv(x, w, (a, b) if affine else None)
+    assert torch.equal(got, resnet18_var.pointwise_conv(torch.relu(torch.addcmul(b, x, a) if affine else x), w))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape", [(1, 1, 1, 4), (2, 1, 5, 64), (1, 2, 2, 68), (3, 7, 10, 64), (2, 14, 9, 132), (1, 17, 16, 512), (2, 5, 6, 30)])
 def test_model_pools(shape):
