@@ -13,11 +13,16 @@
 #include <ATen/core/Tensor.h>
 #include <ATen/core/grad_mode.h>
 #include <ATen/ops/empty.h>
+#include <ATen/ops/record_stream.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+
+#include <atomic>
+#include <memory>
 
 #include "../../include/winograd2x2.h"
 
@@ -108,6 +113,96 @@ PyObject *key(PyObject *, PyObject *const *args, Py_ssize_t count)
         entries[i] = {t._version() + 1, 256 * static_cast<int64_t>(t.device().type()) + t.device().index(), t.const_data_ptr()};
     }
     return PyBytes_FromStringAndSize(reinterpret_cast<const char *>(entries), count * static_cast<Py_ssize_t>(sizeof(Entry)));
+    END_HANDLE_TH_ERRORS
+}
+
+// A place in a stream, behind which a tensor has been written; no event for a tensor that is not on the GPU.
+struct Mark {
+    hipEvent_t event = nullptr;
+    hipStream_t stream = nullptr;
+    std::atomic<bool> reached{false};
+    ~Mark()
+    {
+        if (event != nullptr) (void)hipEventDestroy(event);
+    }
+};
+constexpr const char *kMark = "swc.mark";
+
+bool hip_ok(hipError_t st)
+{
+    if (st == hipSuccess) return true;
+    (void)hipGetLastError();
+    PyErr_SetString(PyExc_RuntimeError, hipGetErrorString(st));
+    return false;
+}
+
+bool capturing(hipStream_t stream)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess) (void)hipGetLastError();
+    return status != hipStreamCaptureStatusNone;
+}
+
+// mark(tensor): the place the current stream is at on the tensor's device, or None while that stream records a graph.
+PyObject *mark(PyObject *, PyObject *const *args, Py_ssize_t count)
+{
+    SWC_ARGS(1)
+    if (!THPVariable_Check(args[0])) {
+        PyErr_SetString(PyExc_TypeError, "a tensor");
+        return nullptr;
+    }
+    const at::Tensor &t = THPVariable_Unpack(args[0]);
+    auto m = std::make_unique<Mark>();
+    if (t.is_cuda()) {
+        const c10::DeviceGuard guard(t.device());
+        m->stream = static_cast<hipStream_t>(stream_of(t));
+        if (capturing(m->stream)) return none();
+        if (!hip_ok(hipEventCreateWithFlags(&m->event, hipEventDisableTiming)) || !hip_ok(hipEventRecord(m->event, m->stream))) return nullptr;
+    }
+    PyObject *capsule = PyCapsule_New(m.get(), kMark, [](PyObject *o) { delete static_cast<Mark *>(PyCapsule_GetPointer(o, kMark)); });
+    if (capsule != nullptr) m.release();
+    return capsule;
+    END_HANDLE_TH_ERRORS
+}
+
+// here(tensor, mark): the tensor, for use on the current stream, which waits for the mark where it is another than the mark's.  A
+// stream that records a graph cannot wait for what was recorded outside of it: then this thread waits.
+PyObject *here(PyObject *, PyObject *const *args, Py_ssize_t count)
+{
+    SWC_ARGS(2)
+    Mark *m = static_cast<Mark *>(PyCapsule_GetPointer(args[1], kMark));
+    if (m == nullptr) return nullptr;
+    if (!THPVariable_Check(args[0])) {
+        PyErr_SetString(PyExc_TypeError, "a tensor");
+        return nullptr;
+    }
+    const at::Tensor &t = THPVariable_Unpack(args[0]);
+    Py_INCREF(args[0]);
+    if (m->event == nullptr) return args[0];
+    const c10::hip::HIPStream current = c10::hip::getCurrentHIPStream(t.device().index());
+    if (current.stream() == m->stream) return args[0];
+    hipError_t st = hipSuccess;
+    {
+        NoGil nogil;
+        const c10::DeviceGuard guard(t.device());
+        if (!m->reached) {
+            // both calls are allowed while a stream is captured, here or in another thread, only in the relaxed mode
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+            const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess, records = capturing(current.stream());
+            st = records ? hipEventSynchronize(m->event) : hipEventQuery(m->event);
+            if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+            if (st == hipSuccess) {
+                m->reached = true;
+            } else if (st == hipErrorNotReady) {
+                (void)hipGetLastError();
+                st = hipStreamWaitEvent(current.stream(), m->event, 0);
+            }
+        }
+        if (st == hipSuccess) t.record_stream(c10::Stream(c10::Stream::UNSAFE, t.device(), current.id()));   // of torch's own device type
+    }
+    if (hip_ok(st)) return args[0];
+    Py_DECREF(args[0]);
+    return nullptr;
     END_HANDLE_TH_ERRORS
 }
 
@@ -343,6 +438,8 @@ using Fast = PyObject *(*)(PyObject *, PyObject *const *, Py_ssize_t);
 PyMethodDef method(const char *name, Fast f) { return {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)), METH_FASTCALL, nullptr}; }
 
 PyMethodDef methods[] = {method("key", key),
+                         method("mark", mark),
+                         method("here", here),
                          method("imtrans", imtrans),
                          method("conv", conv),
                          method("pieces_gain", pieces_gain),

@@ -53,6 +53,12 @@ class WinogradConv(torch.nn.Module):
         self._masked = None
         self._bf16 = None
 
+    def __getstate__(self):
+        return dict(self.__dict__, _masked=None, _bf16=None, _pieces=None)   # made anew by the copy
+
+    def __setstate__(self, state):
+        super().__setstate__(dict(state, _masked=None, _bf16=None, _pieces=None))   # also for a state that holds them in another form
+
     def refresh(self):
         """Drop the cached W*mask, its bf16 copy and its pieces.  Not needed after in-place updates of W or mask made on
         the tensors themselves or on ``detach()``ed views of them (optimizer steps, ``load_state_dict``,
@@ -64,27 +70,32 @@ class WinogradConv(torch.nn.Module):
         self._bf16 = None
         self._pieces = None
 
-    def _weight_key(self):
-        # In-place writes bump _version; a replaced or moved tensor changes data_ptr / device.
-        return _native.key(self.W, self.mask)
+    def _derived(self, slot, key, make):
+        """What ``make`` makes of the weights that ``key`` stands for, kept in ``slot`` with a mark behind it in the stream that wrote it:
+        a call on another stream may find it before it has been written, or drop it (the weights changed) while that stream's kernels
+        read it, and ``here`` sees to both.  While a graph is captured nothing is kept: what the capture records is written when the
+        graph runs, and other calls would read it before."""
+        kept = getattr(self, slot)
+        if kept is not None and kept[0] == key:
+            return _native.here(kept[1], kept[2])
+        tensor = make()
+        mark = _native.mark(tensor)
+        if mark is not None:
+            setattr(self, slot, (key, tensor, mark))
+        return tensor
 
     def bf16_weight(self):
         """W*mask as the [16,K,C] bfloat16 tensor the bf16-stored kernel reads; cached like masked_weight()."""
-        key = self._weight_key()
-        cached = self._bf16
-        if cached is None or cached[0] != key:
-            cached = (key, winograd2x2_conv.winograd2x2_conv.winograd2x2_weights_bf16(self.masked_weight()))
-            self._bf16 = cached
-        return cached[1]
+        return self._derived("_bf16", _native.key(self.W, self.mask),
+                             lambda: winograd2x2_conv.winograd2x2_conv.winograd2x2_weights_bf16(self.masked_weight()))
 
     def weight_pieces(self):
         """W*mask taken apart for the fp32 convolution, or rounded and put in order for the one with bf16 operands; cached like masked_weight()."""
-        key = (self._weight_key(), self.precision)
-        cached = self._pieces
-        if cached is None or cached[0] != key:
-            cached = (key, winograd2x2_conv.winograd2x2_conv.winograd2x2_weight_pieces(self.masked_weight(), self.precision))
-            self._pieces = cached
-        return cached[1]
+        return self._pieces_of(self.masked_weight())
+
+    def _pieces_of(self, masked):
+        return self._derived("_pieces", (_native.key(self.W, self.mask), self.precision),
+                             lambda: winograd2x2_conv.winograd2x2_conv.winograd2x2_weight_pieces(masked, self.precision))
 
     def masked_weight(self):
         """W*mask without autograd history, recomputed only when W or mask changed since the last call (a write
@@ -92,12 +103,7 @@ class WinogradConv(torch.nn.Module):
         W, mask = self.W, self.mask
         if mask is None:
             return W.detach()   # shares W's version counter: a write to what is handed out is noticed
-        key = _native.key(W, mask)
-        cached = self._masked
-        if cached is None or cached[0] != key:
-            cached = (key, (W.detach() * mask).contiguous())
-            self._masked = cached
-        return cached[1]
+        return self._derived("_masked", _native.key(W, mask), lambda: (W.detach() * mask).contiguous())
 
     def forward(self, x, affine=None, residual=None, residual_relu=False):
         """``affine=(scale, shift)`` and ``residual`` (forward only) are applied to the result inside
@@ -115,6 +121,6 @@ class WinogradConv(torch.nn.Module):
                 pieces = True
             elif self.precision in ("fp32", "bf16"):
                 if _native.pieces_gain(x, self.out_channel, self.precision == "bf16") and x.device == w.device and x.shape[4] == w.shape[1]:
-                    pieces = self.weight_pieces()
+                    pieces = self._pieces_of(w)
         scale, shift = affine if affine is not None else (None, None)
         return winograd2x2_conv.winograd2x2_conv.winograd2x2_conv(x, w, self.precision, None, scale, shift, residual, residual_relu, True, pieces)

@@ -238,3 +238,92 @@ def test_a_bf16_layer_is_the_op_on_its_weights(masked):
             assert torch.equal(layer(ti), winograd2x2_conv(ti, w, "bf16"))
             assert (layer._pieces is not None) == masked
             layer.W.mul_(2)
+
+
+def masked_layer(precision, C):
+    """A masked layer, planes of a shape whose convolution uses kept pieces and of one whose does not, and the former's output in float64."""
+    from winograd_conv import WinogradConv
+    gen = torch.Generator(device="cuda").manual_seed(29)
+    B, n = (64, 7) if precision == "fp32" else (128, 8)
+    ti = torch.randn((16, B, n, n, C), device="cuda", generator=gen).relu_()
+    w = torch.randn((16, C, C), device="cuda", generator=gen) * 0.05
+    layer = WinogradConv(C, C, mask=(torch.rand((16, C, C), device="cuda", generator=gen) < 0.3).float(), W_init=w, device="cuda", precision=precision)
+    wm, t = layer.W.detach() * layer.mask, ti.reshape(16, -1, C)
+    if precision == "bf16":
+        wm, t = wm.bfloat16(), t.bfloat16()
+    p = torch.bmm(t.double(), wm.double()).reshape(4, 4, -1, C)
+    r = torch.stack([p[0] + p[1] + p[2], p[1] - p[2] - p[3]])
+    want = torch.stack([r[:, 0] + r[:, 1] + r[:, 2], r[:, 1] - r[:, 2] - r[:, 3]], 1).reshape(2, 2, B, n, n, C)
+    return layer, ti, ti[:, :1, :2, :2].contiguous(), want.permute(2, 3, 0, 4, 1, 5).reshape(B, 2 * n, 2 * n, C)
+
+
+LAYERS = [("fp32", 256), ("bf16", 512)]
+
+
+def close(y, want):   # sums of at most 512 products in fp32, from the same operands
+    return (y.double() - want).norm() <= 1e-6 * want.norm()
+
+
+@pytest.mark.parametrize("precision,C", LAYERS)
+@pytest.mark.parametrize("warm", [True, False])
+def test_kept_weights_are_there_on_every_stream(precision, C, warm):
+    """What a layer keeps is made on the stream of the call that first wants it; a call on another stream may follow at once."""
+    layer, ti, small, want = masked_layer(precision, C)
+    busy = torch.ones((4096, 4096), device="cuda")
+    with torch.no_grad():
+        if warm:
+            layer(small)
+        assert layer._pieces is None
+        torch.cuda.synchronize()
+        streams = [torch.cuda.Stream() for _ in range(3)]
+        with torch.cuda.stream(streams[0]):
+            for _ in range(20):
+                busy = torch.mm(busy, busy).clamp_(max=1)
+            outputs = [layer(ti), layer(ti)]
+        for s in streams[1:]:
+            with torch.cuda.stream(s):
+                outputs.append(layer(ti))
+        torch.cuda.synchronize()
+        outputs.append(layer(ti))
+        assert all(close(y, want) for y in outputs)
+
+
+@pytest.mark.parametrize("precision,C", LAYERS)
+@pytest.mark.parametrize("warm", [True, False])
+def test_a_capture_keeps_no_weights(precision, C, warm):
+    """Weights that a capture would make are written when the graph runs: nothing of them may be kept for eager calls.  What eager
+    calls kept before is used in a capture."""
+    layer, ti, small, want = masked_layer(precision, C)
+    with torch.no_grad():
+        if warm:
+            layer(small)
+        torch.cuda.synchronize()
+        for kept in (False, True):
+            before = layer._masked, layer._pieces
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                y = layer(ti)
+            assert (layer._masked, layer._pieces) == before and (layer._pieces is None) == (not kept)
+            assert close(layer(ti), want)
+            for _ in range(3):
+                y.zero_()
+                graph.replay()
+                layer(small)
+                torch.cuda.synchronize()
+                assert close(y, want)
+            layer(ti)
+
+
+def test_a_copied_layer_brings_no_kept_weights():
+    import copy
+    import pickle
+    layer, ti, _, want = masked_layer("fp32", 256)
+    with torch.no_grad():
+        layer(ti)
+        assert layer._masked is not None
+        for other in (copy.deepcopy(layer), pickle.loads(pickle.dumps(layer))):
+            assert (other._masked, other._bf16, other._pieces) == (None, None, None)
+            assert close(other(ti), want)
+        state = dict(layer.__getstate__(), _masked=(b"", torch.zeros_like(layer.W)), _pieces=None)   # as layers kept them before
+        other.__setstate__(state)
+        assert close(other(ti), want)
