@@ -70,6 +70,10 @@ class WinogradConv(torch.nn.Module):
         self._bf16 = None
         self._pieces = None
 
+    def _weight_key(self):
+        # In-place writes bump _version; a replaced or moved tensor changes data_ptr / device.
+        return _native.key(self.W, self.mask)
+
     def _derived(self, slot, key, make):
         """What ``make`` makes of the weights that ``key`` stands for, kept in ``slot`` with a mark behind it in the stream that wrote it:
         a call on another stream may find it before it has been written, or drop it (the weights changed) while that stream's kernels
@@ -86,7 +90,7 @@ class WinogradConv(torch.nn.Module):
 
     def bf16_weight(self):
         """W*mask as the [16,K,C] bfloat16 tensor the bf16-stored kernel reads; cached like masked_weight()."""
-        return self._derived("_bf16", _native.key(self.W, self.mask),
+        return self._derived("_bf16", self._weight_key(),
                              lambda: winograd2x2_conv.winograd2x2_conv.winograd2x2_weights_bf16(self.masked_weight()))
 
     def weight_pieces(self):
@@ -94,7 +98,7 @@ class WinogradConv(torch.nn.Module):
         return self._pieces_of(self.masked_weight())
 
     def _pieces_of(self, masked):
-        return self._derived("_pieces", (_native.key(self.W, self.mask), self.precision),
+        return self._derived("_pieces", (self._weight_key(), self.precision),
                              lambda: winograd2x2_conv.winograd2x2_conv.winograd2x2_weight_pieces(masked, self.precision))
 
     def masked_weight(self):
