@@ -71,6 +71,23 @@ def test_direct_forms(oracle, forced, form, shape, precision):
     assert np.array_equal(ep, oracle.affine(got, scale, shift) + np.maximum(res, 0))
 
 
+@pytest.mark.parametrize("C", [32, 36, 40, 60, 64, 96, 100, 124, 128, 176])
+def test_bf16_single_tiles_with_every_end_of_a_block(forced, C):
+    # Blocks of 32 indices that are turned round in LDS, and blocks of 64 that are not where C ends in the second half of one.  Whole
+    # numbers are exact in bf16 and in any order of the sums.
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv
+    gen = torch.Generator(device="cuda").manual_seed(63)
+    ti = torch.randint(-4, 5, (16, 1, 7, 11, C), device="cuda", generator=gen).float()
+    w = torch.randint(-4, 5, (16, C, 36), device="cuda", generator=gen).float()
+    assert forced.swc_winograd2x2_conv_force_tiling(b"direct16x16") == 0
+    got = winograd2x2_conv(ti, w, "bf16")
+    assert forced.swc_winograd2x2_conv_last_form() == b"direct16x16"
+    p = torch.matmul(ti.reshape(16, -1, C).double().cpu(), w.double().cpu()).reshape(4, 4, 7, 11, 36)
+    a = torch.tensor([[1, 1, 1, 0], [0, 1, -1, -1]], dtype=torch.float64)
+    want = torch.einsum("ai,bj,ijhwk->hawbk", a, a, p).reshape(1, 14, 22, 36)
+    assert torch.equal(got.cpu().double(), want)
+
+
 @pytest.mark.parametrize("shape,precision,want", [
     ((1, 8, 8, 64, 64), "fp32", "direct16x16"),       # 16 tiles of 16x16
     ((5, 14, 16, 96, 72), "fp32", "direct16x32"),     # 350 tiles of 16x16, 210 of 16x32
@@ -86,6 +103,11 @@ def test_direct_forms(oracle, forced, form, shape, precision):
     ((64, 7, 7, 256, 256), "bf16", "split64"),        # 196 tiles of 64x64
     ((64, 14, 14, 128, 128), "bf16", "whole"),        # 392
     ((64, 14, 14, 32, 64), "bf16", "whole"),          # below 64 channels the ring takes less
+    # channels that are no multiple of 32, which no ring kernel takes: a round behind the first counts as what it takes
+    ((18, 16, 16, 72, 384), "bf16", "direct32x64"),   # 4 rounds, 16x64 tiles would be 7
+    ((1, 5483, 1, 208, 256), "bf16", "direct32x64"),  # 3 and 6
+    ((1, 2427, 1, 100, 96), "bf16", "split32"),       # 1 round, 16x32 tiles 2
+    ((1, 14094, 1, 72, 128), "bf16", "direct32x64"),  # 4 and 7
 ])
 def test_the_launcher_picks_the_smallest_tile_that_needs_one_round(forced, shape, precision, want):
     from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv
