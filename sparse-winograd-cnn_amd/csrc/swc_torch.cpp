@@ -116,25 +116,41 @@ PyObject *key(PyObject *, PyObject *const *args, Py_ssize_t count)
     END_HANDLE_TH_ERRORS
 }
 
-// A place in a stream, behind which a tensor has been written; no event for a tensor that is not on the GPU.
+// Behind which work a tensor has been written: the stream, and an event in it once another stream has asked.  An event at once would
+// cost every write 2 us of the host and 3 of the GPU; one that is recorded later is behind more of that stream's work than needed.
 struct Mark {
-    hipEvent_t event = nullptr;
     hipStream_t stream = nullptr;
+    hipEvent_t event = nullptr;   // made and read under the interpreter's lock
+    bool gpu = false;
     std::atomic<bool> reached{false};
     ~Mark()
     {
         if (event != nullptr) (void)hipEventDestroy(event);
     }
+    hipError_t record()
+    {
+        hipEvent_t e;
+        hipError_t st = hipEventCreateWithFlags(&e, hipEventDisableTiming);
+        if (st != hipSuccess) return st;
+        st = hipEventRecord(e, stream);
+        if (st == hipSuccess)
+            event = e;
+        else
+            (void)hipEventDestroy(e);
+        return st;
+    }
 };
 constexpr const char *kMark = "swc.mark";
 
-bool hip_ok(hipError_t st)
-{
-    if (st == hipSuccess) return true;
-    (void)hipGetLastError();
-    PyErr_SetString(PyExc_RuntimeError, hipGetErrorString(st));
-    return false;
-}
+// What is asked about streams here is allowed while a stream is captured, by this thread or another, only in the relaxed mode.
+struct Relaxed {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool changed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    ~Relaxed()
+    {
+        if (changed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
 
 bool capturing(hipStream_t stream)
 {
@@ -143,7 +159,14 @@ bool capturing(hipStream_t stream)
     return status != hipStreamCaptureStatusNone;
 }
 
-// mark(tensor): the place the current stream is at on the tensor's device, or None while that stream records a graph.
+PyObject *hip_error(hipError_t st)
+{
+    (void)hipGetLastError();
+    PyErr_SetString(PyExc_RuntimeError, hipGetErrorString(st));
+    return nullptr;
+}
+
+// mark(tensor): behind what the current stream has been given on the tensor's device, or None while that stream records a graph.
 PyObject *mark(PyObject *, PyObject *const *args, Py_ssize_t count)
 {
     SWC_ARGS(1)
@@ -155,9 +178,15 @@ PyObject *mark(PyObject *, PyObject *const *args, Py_ssize_t count)
     auto m = std::make_unique<Mark>();
     if (t.is_cuda()) {
         const c10::DeviceGuard guard(t.device());
-        m->stream = static_cast<hipStream_t>(stream_of(t));
+        const Relaxed relaxed;
+        const c10::hip::HIPStream current = c10::hip::getCurrentHIPStream(t.device().index());
+        m->gpu = true;
+        m->stream = current.stream();
         if (capturing(m->stream)) return none();
-        if (!hip_ok(hipEventCreateWithFlags(&m->event, hipEventDisableTiming)) || !hip_ok(hipEventRecord(m->event, m->stream))) return nullptr;
+        // torch's own streams live as long as the process; one from elsewhere may be gone when it would be asked
+        const bool own = m->stream == nullptr || c10::hip::getStreamFromExternal(m->stream, t.device().index()).id() != current.id();
+        const hipError_t st = own ? hipSuccess : m->record();
+        if (st != hipSuccess) return hip_error(st);
     }
     PyObject *capsule = PyCapsule_New(m.get(), kMark, [](PyObject *o) { delete static_cast<Mark *>(PyCapsule_GetPointer(o, kMark)); });
     if (capsule != nullptr) m.release();
@@ -165,8 +194,9 @@ PyObject *mark(PyObject *, PyObject *const *args, Py_ssize_t count)
     END_HANDLE_TH_ERRORS
 }
 
-// here(tensor, mark): the tensor, for use on the current stream, which waits for the mark where it is another than the mark's.  A
-// stream that records a graph cannot wait for what was recorded outside of it: then this thread waits.
+// here(tensor, mark): the tensor, for use on the current stream, which waits for the mark where it is another than the mark's; a
+// stream that records a graph cannot wait for what was recorded outside of it, then this thread waits.  None where there is no telling,
+// since the mark's stream records a graph by now.
 PyObject *here(PyObject *, PyObject *const *args, Py_ssize_t count)
 {
     SWC_ARGS(2)
@@ -177,32 +207,35 @@ PyObject *here(PyObject *, PyObject *const *args, Py_ssize_t count)
         return nullptr;
     }
     const at::Tensor &t = THPVariable_Unpack(args[0]);
-    Py_INCREF(args[0]);
-    if (m->event == nullptr) return args[0];
-    const c10::hip::HIPStream current = c10::hip::getCurrentHIPStream(t.device().index());
-    if (current.stream() == m->stream) return args[0];
-    hipError_t st = hipSuccess;
-    {
-        NoGil nogil;
-        const c10::DeviceGuard guard(t.device());
-        if (!m->reached) {
-            // both calls are allowed while a stream is captured, here or in another thread, only in the relaxed mode
-            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-            const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess, records = capturing(current.stream());
-            st = records ? hipEventSynchronize(m->event) : hipEventQuery(m->event);
-            if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
-            if (st == hipSuccess) {
-                m->reached = true;
-            } else if (st == hipErrorNotReady) {
-                (void)hipGetLastError();
-                st = hipStreamWaitEvent(current.stream(), m->event, 0);
+    if (m->gpu) {
+        const c10::hip::HIPStream current = c10::hip::getCurrentHIPStream(t.device().index());
+        if (current.stream() != m->stream) {
+            const c10::DeviceGuard guard(t.device());
+            if (!m->reached) {
+                const Relaxed relaxed;
+                hipError_t st = hipSuccess;
+                if (m->event == nullptr) {
+                    if (capturing(m->stream)) return none();
+                    st = m->record();
+                }
+                if (st == hipSuccess) {
+                    const bool wait = capturing(current.stream());
+                    NoGil nogil;
+                    st = wait ? hipEventSynchronize(m->event) : hipEventQuery(m->event);
+                }
+                if (st == hipSuccess) {
+                    m->reached = true;
+                } else if (st == hipErrorNotReady) {
+                    (void)hipGetLastError();
+                    st = hipStreamWaitEvent(current.stream(), m->event, 0);
+                }
+                if (st != hipSuccess) return hip_error(st);
             }
+            t.record_stream(c10::Stream(c10::Stream::UNSAFE, t.device(), current.id()));   // of torch's own device type
         }
-        if (st == hipSuccess) t.record_stream(c10::Stream(c10::Stream::UNSAFE, t.device(), current.id()));   // of torch's own device type
     }
-    if (hip_ok(st)) return args[0];
-    Py_DECREF(args[0]);
-    return nullptr;
+    Py_INCREF(args[0]);
+    return args[0];
     END_HANDLE_TH_ERRORS
 }
 

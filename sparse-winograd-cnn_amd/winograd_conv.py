@@ -74,15 +74,11 @@ class WinogradConv(torch.nn.Module):
         # In-place writes bump _version; a replaced or moved tensor changes data_ptr / device.
         return _native.key(self.W, self.mask)
 
-    def _derived(self, slot, key, make):
-        """What ``make`` makes of the weights that ``key`` stands for, kept in ``slot`` with a mark behind it in the stream that wrote it:
-        a call on another stream may find it before it has been written, or drop it (the weights changed) while that stream's kernels
+    def _keep(self, slot, key, tensor):
+        """``tensor``, made of the weights that ``key`` stands for, kept in ``slot`` with a mark behind it in the stream that wrote it: a
+        call on another stream may find it before it has been written, or drop it (the weights changed) while that stream's kernels
         read it, and ``here`` sees to both.  While a graph is captured nothing is kept: what the capture records is written when the
         graph runs, and other calls would read it before."""
-        kept = getattr(self, slot)
-        if kept is not None and kept[0] == key:
-            return _native.here(kept[1], kept[2])
-        tensor = make()
         mark = _native.mark(tensor)
         if mark is not None:
             setattr(self, slot, (key, tensor, mark))
@@ -90,16 +86,22 @@ class WinogradConv(torch.nn.Module):
 
     def bf16_weight(self):
         """W*mask as the [16,K,C] bfloat16 tensor the bf16-stored kernel reads; cached like masked_weight()."""
-        return self._derived("_bf16", self._weight_key(),
-                             lambda: winograd2x2_conv.winograd2x2_conv.winograd2x2_weights_bf16(self.masked_weight()))
+        kept, key = self._bf16, self._weight_key()
+        tensor = _native.here(kept[1], kept[2]) if kept is not None and kept[0] == key else None
+        if tensor is not None:
+            return tensor
+        return self._keep("_bf16", key, winograd2x2_conv.winograd2x2_conv.winograd2x2_weights_bf16(self.masked_weight()))
 
     def weight_pieces(self):
         """W*mask taken apart for the fp32 convolution, or rounded and put in order for the one with bf16 operands; cached like masked_weight()."""
         return self._pieces_of(self.masked_weight())
 
     def _pieces_of(self, masked):
-        return self._derived("_pieces", (self._weight_key(), self.precision),
-                             lambda: winograd2x2_conv.winograd2x2_conv.winograd2x2_weight_pieces(masked, self.precision))
+        kept, key = self._pieces, (self._weight_key(), self.precision)
+        tensor = _native.here(kept[1], kept[2]) if kept is not None and kept[0] == key else None
+        if tensor is not None:
+            return tensor
+        return self._keep("_pieces", key, winograd2x2_conv.winograd2x2_conv.winograd2x2_weight_pieces(masked, self.precision))
 
     def masked_weight(self):
         """W*mask without autograd history, recomputed only when W or mask changed since the last call (a write
@@ -107,7 +109,11 @@ class WinogradConv(torch.nn.Module):
         W, mask = self.W, self.mask
         if mask is None:
             return W.detach()   # shares W's version counter: a write to what is handed out is noticed
-        return self._derived("_masked", _native.key(W, mask), lambda: (W.detach() * mask).contiguous())
+        kept, key = self._masked, _native.key(W, mask)
+        tensor = _native.here(kept[1], kept[2]) if kept is not None and kept[0] == key else None
+        if tensor is not None:
+            return tensor
+        return self._keep("_masked", key, (W.detach() * mask).contiguous())
 
     def forward(self, x, affine=None, residual=None, residual_relu=False):
         """``affine=(scale, shift)`` and ``residual`` (forward only) are applied to the result inside

@@ -266,7 +266,8 @@ def close(y, want):   # sums of at most 512 products in fp32, from the same oper
 
 @pytest.mark.parametrize("precision,C", LAYERS)
 @pytest.mark.parametrize("warm", [True, False])
-def test_kept_weights_are_there_on_every_stream(precision, C, warm):
+@pytest.mark.parametrize("external", [True, False])
+def test_kept_weights_are_there_on_every_stream(precision, C, warm, external):
     """What a layer keeps is made on the stream of the call that first wants it; a call on another stream may follow at once."""
     layer, ti, small, want = masked_layer(precision, C)
     busy = torch.ones((4096, 4096), device="cuda")
@@ -276,6 +277,11 @@ def test_kept_weights_are_there_on_every_stream(precision, C, warm):
         assert layer._pieces is None
         torch.cuda.synchronize()
         streams = [torch.cuda.Stream() for _ in range(3)]
+        if external:   # a stream that is not torch's
+            import ctypes
+            hip, handle = ctypes.CDLL("libamdhip64.so.7"), ctypes.c_void_p()
+            assert hip.hipStreamCreateWithFlags(ctypes.byref(handle), 1) == 0
+            streams[0] = torch.cuda.ExternalStream(handle.value)
         with torch.cuda.stream(streams[0]):
             for _ in range(20):
                 busy = torch.mm(busy, busy).clamp_(max=1)
@@ -286,6 +292,10 @@ def test_kept_weights_are_there_on_every_stream(precision, C, warm):
         torch.cuda.synchronize()
         outputs.append(layer(ti))
         assert all(close(y, want) for y in outputs)
+        layer.W.mul_(1)   # makes anew, and drops what other streams have read
+        with torch.cuda.stream(streams[1]):
+            assert close(layer(ti), want) and close(layer(ti), want)
+        torch.cuda.synchronize()
 
 
 @pytest.mark.parametrize("precision,C", LAYERS)
