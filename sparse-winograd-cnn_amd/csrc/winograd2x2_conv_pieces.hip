@@ -6,6 +6,16 @@
 namespace swc {
 namespace {
 
+// Columns of tiles that are gone through together.  Every panel of them reads all rows of TI again, and an XCD with the same panel's
+// weights reads what they take: up to seven columns, in panels about as wide, and eight where the pieces of all fit two L2s (8 MiB).
+// Behind the transform, in panels of four and the rest / so: 1600x192->320 37.7 us / 33.7, 910x128->448 26.8 / 23.5, 2016x64->512 28.3 / 24.7;
+// but 637x512->512 59.3 / 62.1 in one panel.
+size_t panel_width(size_t tiles_n, int C)
+{
+    const size_t most = tiles_n == 8 && tiles_n * 64 * C * 16 * 2 * kPieces <= (8u << 20) ? 8 : 7, panels = (tiles_n + most - 1) / most;
+    return (tiles_n + panels - 1) / panels;
+}
+
 template <typename Main, typename Tail = Main>
 int launch_as(const float *TI, const float *Wt, const void *Wp, float *Out, size_t M, int C, int K, int nW, size_t main_m, const ConvEpilogue &ep,
               hipStream_t stream)
@@ -24,11 +34,12 @@ int launch_as(const float *TI, const float *Wt, const void *Wp, float *Out, size
     const size_t main_wgs = main_m * tiles_n < cus ? main_m * tiles_n : cus;
     conv_pieces_kernel<Main, Tail><<<dim3(static_cast<unsigned>(main_wgs + tail_m * tiles_n)), dim3(Main::NT), Main::LDS_BYTES, stream>>>(
         TI, Wt, static_cast<const char *>(Wp), Out, static_cast<unsigned>(M), C, K, nW, static_cast<unsigned>(main_m),
-        static_cast<unsigned>(main_wgs), static_cast<unsigned>(tail_m), static_cast<unsigned>(tiles_n), ep);
+        static_cast<unsigned>(main_wgs), static_cast<unsigned>(tail_m), static_cast<unsigned>(tiles_n), static_cast<unsigned>(panel_width(tiles_n, C)), ep);
     return check_launch();
 }
 
 constexpr size_t kInfinityCacheBytes = 256u << 20;
+constexpr size_t kStreamedPlanes = 64u << 20;   // beyond so many bytes the transform stores past the caches
 
 size_t steps_of(int C) { return (static_cast<size_t>(C) + 31) / 32; }
 size_t groups_of(int K) { return (static_cast<size_t>(K) + 63) / 64; }
@@ -62,6 +73,7 @@ namespace {
 //   4410x512->256 93.4 / 76.3 (152 / 126)      6272x512->512 203 / 181 (283 / 251)        6272x256->256 53.0 / 51.1 (95 / 85)
 //   5000x256->512 (132 / 95)                   3920x384->320 (126 / 98)                   4320x320->384 (113 / 96)
 //   12544x128->128 31.9 / 32.1: not taken
+// and whole rounds alone only where the transform streams the planes (below, behind it, 3596x256->512 65.1 / 66.5, 3195x320->512 76.4 / 78.0).
 // One round of 64-row tiles is no faster than split64 (3136x256->256 28.0 / 28.4, 2700x160->320 19.8 / 22.6).
 PiecesChoice choose_bf16(size_t M, int C, double c, size_t cus, size_t tiles_n)
 {
@@ -78,12 +90,13 @@ PiecesChoice choose_bf16(size_t M, int C, double c, size_t cus, size_t tiles_n)
     const size_t whole = M / 64 * tiles_n / cus, main_m = whole * cus / tiles_n;
     const double us = static_cast<double>(whole) * us64 + rounds_of(M - main_m * 64, 32) * 3.6 * c;
     if (main_m * 64 < M && us < best.us) best = {PIECES_64_32, main_m, us};
+    if (best.form == PIECES_64 && M * C * 64 <= kStreamedPlanes) best = PiecesChoice();
     return best;
 }
 }  // namespace
 
 // A workgroup fills a CU, so a launch takes rounds of tiles over the CUs.  Measured per round, 64-row tiles: 8 us + 8.25 per 64
-// channels, 1 us more in all; 32-row tiles: 2.5 + 5.9, and 2.5 + 0.4 more in all.  Where 64-row tiles make more than a round, whole
+// channels, 1 us more in all; 32-row tiles: 3.7 + 5.9, and 1.3 + 0.4 more in all.  Where 64-row tiles make more than a round, whole
 // rounds of them and the rest in one round of 32-row ones, 5 + 6.9.  Against what runs on W itself:
 //   14x14x256 -> 256, batch 64    split64       57.5 us   pieces64      43.5 us
 //   7x7x512 -> 512, batch 64      split32       66.5      pieces32      55.4 (58.5)
@@ -110,7 +123,10 @@ PiecesChoice choose_pieces(const void *TI, const void *Wt, const void *Wp, const
     if (bf16) return choose_bf16(M, C, c, cus, tiles_n);
     auto rounds_of = [&](size_t rows, size_t high) { return static_cast<double>(((rows + high - 1) / high * tiles_n + cus - 1) / cus); };
     auto us64 = [&](double rounds) { return 1.0 + rounds * (8.0 + 8.25 * c); };
-    const double us32 = 2.5 + 0.4 * c + rounds_of(M, 32) * (2.5 + 5.9 * c);
+    // Streamed planes come from memory, which one column of 32-row tiles after the other does not hide: 14 us (2100x512->96 52 us, behind the
+    // transform 81; split32 60 and 76).
+    const bool streamed = M * C * 64 > kStreamedPlanes;
+    const double us32 = 1.3 + 0.4 * c + rounds_of(M, 32) * (3.7 + 5.9 * c) + (streamed ? 14.0 : 0.0);
     best = {PIECES_64, 0, us64(rounds_of(M, 64))};
     if (us32 < best.us) best = {PIECES_32, 0, us32};
     const size_t whole = M / 64 * tiles_n / cus, main_m = whole * cus / tiles_n;

@@ -355,14 +355,13 @@ __device__ __forceinline__ void pieces_tiles(const float *__restrict__ TI, const
 }
 
 // Tile `id` of those that cover the rows from row0 on, end exclusive.  The 32 workgroups of an XCD have consecutive tiles: they
-// share their L2's copy of the rows and the weights best where they are about as many tiles high as wide.
+// share their L2's copy of the rows and the weights, `wide` columns at a time (see panel_width).
 template <typename Cfg>
-__device__ __forceinline__ PieceTile piece_tile(unsigned id, unsigned tiles_m, unsigned tiles_n, unsigned row0, unsigned end)
+__device__ __forceinline__ PieceTile piece_tile(unsigned id, unsigned tiles_m, unsigned tiles_n, unsigned wide, unsigned row0, unsigned end)
 {
-    constexpr unsigned kPanel = 4;
-    const unsigned panel = id / (tiles_m * kPanel), width = tiles_n - panel * kPanel < kPanel ? tiles_n - panel * kPanel : kPanel;
-    const unsigned in = id - panel * tiles_m * kPanel, m0 = row0 + in / width * Cfg::WM;
-    return PieceTile{m0, end - m0 < Cfg::WM ? end - m0 : Cfg::WM, panel * kPanel + in % width};
+    const unsigned panel = id / (tiles_m * wide), width = tiles_n - panel * wide < wide ? tiles_n - panel * wide : wide;
+    const unsigned in = id - panel * tiles_m * wide, m0 = row0 + in / width * Cfg::WM;
+    return PieceTile{m0, end - m0 < Cfg::WM ? end - m0 : Cfg::WM, panel * wide + in % width};
 }
 
 // The first main_wgs workgroups take the main_m * tiles_n tiles of Main, one after the other where there are more of them, those
@@ -370,7 +369,7 @@ __device__ __forceinline__ PieceTile piece_tile(unsigned id, unsigned tiles_m, u
 template <typename Main, typename Tail>
 __global__ __launch_bounds__(Main::NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void conv_pieces_kernel(
     const float *__restrict__ TI, const float *__restrict__ Wt, const char *__restrict__ Wp, float *__restrict__ Out, unsigned M, int C,
-    int K, int nW, unsigned main_m, unsigned main_wgs, unsigned tail_m, unsigned tiles_n, ConvEpilogue ep)
+    int K, int nW, unsigned main_m, unsigned main_wgs, unsigned tail_m, unsigned tiles_n, unsigned wide, ConvEpilogue ep)
 {
     extern __shared__ __attribute__((aligned(16))) float P[];   // [8][E] and the staging tiles
     const unsigned n_main = main_m * tiles_n;
@@ -378,12 +377,12 @@ __global__ __launch_bounds__(Main::NT) __attribute__((amdgpu_waves_per_eu(2, 2))
     if (std::is_same<Main, Tail>::value || blockIdx.x < main_wgs) {
         auto tile_of = [&](unsigned i) __attribute__((always_inline)) {
             const unsigned before = i * main_wgs, here = n_main - before < main_wgs ? n_main - before : main_wgs;
-            return piece_tile<Main>(before + xcd_swizzle(blockIdx.x, here), main_m, tiles_n, 0, main_rows);
+            return piece_tile<Main>(before + xcd_swizzle(blockIdx.x, here), main_m, tiles_n, wide, 0, main_rows);
         };
         pieces_tiles<Main>(TI, Wt, Wp, Out, M, C, K, nW, (n_main - blockIdx.x + main_wgs - 1) / main_wgs, tile_of, P, ep);
     } else if constexpr (!std::is_same<Main, Tail>::value) {
         auto tile_of = [&](unsigned) __attribute__((always_inline)) {
-            return piece_tile<Tail>(xcd_swizzle(blockIdx.x - main_wgs, tail_m * tiles_n), tail_m, tiles_n, main_rows, M);
+            return piece_tile<Tail>(xcd_swizzle(blockIdx.x - main_wgs, tail_m * tiles_n), tail_m, tiles_n, wide, main_rows, M);
         };
         pieces_tiles<Tail>(TI, Wt, Wp, Out, M, C, K, nW, 1, tile_of, P, ep);
     }

@@ -51,6 +51,47 @@ def test_pieces_forms(oracle, forced, form, shape):  # noqa: F811
     assert np.array_equal(buf.cpu().numpy(), got + res)
 
 
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("C,K", [(16, 320), (16, 448), (16, 512), (192, 512), (16, 576), (16, 832)])
+def test_panels_of_columns(forced, form, C, K):  # noqa: F811
+    """5, 7, 8, 9 and 13 columns of tiles: in one panel, in two of four (the weights of 192 channels are too large for one), five and
+    four, seven and six.  Whole numbers are exact in any order of the sums."""
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv, winograd2x2_weight_pieces
+    gen = torch.Generator(device="cuda").manual_seed(86)
+    ti = torch.randint(-4, 5, (16, 3, 7, 11, C), device="cuda", generator=gen).float()
+    w = torch.randint(-4, 5, (16, C, K), device="cuda", generator=gen).float()
+    assert forced.swc_winograd2x2_conv_force_tiling(b"direct32x64") == 0
+    want = winograd2x2_conv(ti, w)
+    assert forced.swc_winograd2x2_conv_force_tiling(form.encode()) == 0
+    assert torch.equal(winograd2x2_conv(ti, w, pieces=winograd2x2_weight_pieces(w)), want)
+    assert forced.swc_winograd2x2_conv_last_form().decode() == form
+
+
+@pytest.mark.parametrize("shape,precision,want", [
+    ((64, 4, 4, 512, 512), "fp32", "pieces32"),
+    ((64, 5, 5, 192, 320), "fp32", "pieces32"),        # five columns of tiles
+    ((21, 25, 4, 512, 96), "fp32", "split32"),         # planes beyond 64 MiB and 32-row tiles
+    ((54, 13, 13, 64, 256), "fp32", "pieces64+32"),    # five rounds of 32-row tiles are no faster than short16
+    ((64, 7, 7, 256, 256), "fp32", "pieces64"),
+    ((128, 7, 7, 512, 512), "fp32", "pieces64+32"),    # three rounds of 64-row tiles over two panels, the rest in 32-row ones
+    ((64, 4, 4, 512, 512), "bf16", "pieces32"),
+    ((4, 29, 31, 256, 512), "bf16", "whole"),          # two rounds of 64-row tiles, planes of 59 MB
+    ((128, 7, 7, 256, 256), "bf16", "pieces64"),       # two, 103 MB
+    ((128, 7, 7, 512, 512), "bf16", "pieces64+32"),
+    ((64, 7, 7, 256, 256), "bf16", "split64"),
+])
+def test_where_prepared_weights_are_used(forced, shape, precision, want):  # noqa: F811
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv, winograd2x2_weight_pieces
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the picks are those of 256 CUs")
+    B, nH, nW, C, K = shape
+    w = torch.ones((16, C, K), device="cuda")
+    winograd2x2_conv(torch.ones((16, B, nH, nW, C), device="cuda"), w, precision, pieces=winograd2x2_weight_pieces(w, precision))
+    assert forced.swc_winograd2x2_conv_last_form().decode() == want
+    gain = {"fp32": forced.swc_winograd2x2_conv_pieces_gain, "bf16": forced.swc_winograd2x2_conv_pieces_bf16_gain}[precision]
+    assert (gain(C, B, nH, nW, K) > 0) == want.startswith("pieces")
+
+
 @pytest.mark.parametrize("C", [64, 72, 256, 512])
 @pytest.mark.parametrize("density", [0.1, 0.3, 1.0])
 @pytest.mark.parametrize("magnitude", [(1.0, 0.05), (1e-6, 1e-5), (3e4, 20.0)])
