@@ -166,6 +166,21 @@ PyObject *hip_error(hipError_t st)
     return nullptr;
 }
 
+// capturing(tensor): whether the current stream on the tensor's device records a graph.
+PyObject *is_capturing(PyObject *, PyObject *const *args, Py_ssize_t count)
+{
+    SWC_ARGS(1)
+    if (!THPVariable_Check(args[0])) {
+        PyErr_SetString(PyExc_TypeError, "a tensor");
+        return nullptr;
+    }
+    const at::Tensor &t = THPVariable_Unpack(args[0]);
+    if (!t.is_cuda()) return PyBool_FromLong(0);
+    const c10::DeviceGuard guard(t.device());
+    return PyBool_FromLong(capturing(static_cast<hipStream_t>(stream_of(t))));
+    END_HANDLE_TH_ERRORS
+}
+
 // mark(tensor): behind what the current stream has been given on the tensor's device, or None while that stream records a graph.
 PyObject *mark(PyObject *, PyObject *const *args, Py_ssize_t count)
 {
@@ -264,6 +279,29 @@ PyObject *imtrans(PyObject *, PyObject *const *args, Py_ssize_t count)
                                                 stream_of(*I));
         else
             st = swc_winograd2x2_imtrans(floats(*I), floats_of(out), as_int(C), as_int(B), as_int(H), as_int(W), 1, 1, relu, stream_of(*I));
+    }
+    return st == SWC_OK ? THPVariable_Wrap(std::move(out)) : none();
+    END_HANDLE_TH_ERRORS
+}
+
+// weight_pieces(W, bf16 operands)
+PyObject *weight_pieces(PyObject *, PyObject *const *args, Py_ssize_t count)
+{
+    SWC_ARGS(2)
+    const at::Tensor *W = plain(args[0], at::kFloat, 3);
+    const int bf16 = PyObject_IsTrue(args[1]);
+    if (bf16 < 0) return nullptr;
+    if (W == nullptr || watched() || W->size(0) != 16 || !fits(W->sizes())) return none();
+    const int C = as_int(W->size(1)), K = as_int(W->size(2));
+    const size_t bytes = (bf16 ? swc_winograd2x2_weight_pieces_bf16_bytes : swc_winograd2x2_weight_pieces_bytes)(C, K);
+    if (bytes == 0) return none();
+    at::Tensor out;
+    int st;
+    {
+        NoGil nogil;
+        const c10::DeviceGuard guard(W->device());
+        out = make(*W, {static_cast<int64_t>(bytes)}, at::kByte);
+        st = (bf16 ? swc_winograd2x2_weight_pieces_bf16 : swc_winograd2x2_weight_pieces)(floats(*W), out.mutable_data_ptr(), C, K, stream_of(*W));
     }
     return st == SWC_OK ? THPVariable_Wrap(std::move(out)) : none();
     END_HANDLE_TH_ERRORS
@@ -471,10 +509,12 @@ using Fast = PyObject *(*)(PyObject *, PyObject *const *, Py_ssize_t);
 PyMethodDef method(const char *name, Fast f) { return {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)), METH_FASTCALL, nullptr}; }
 
 PyMethodDef methods[] = {method("key", key),
+                         method("capturing", is_capturing),
                          method("mark", mark),
                          method("here", here),
                          method("imtrans", imtrans),
                          method("conv", conv),
+                         method("weight_pieces", weight_pieces),
                          method("pieces_gain", pieces_gain),
                          method("conv_stored", conv_stored),
                          method("conv_grad", conv_grad),

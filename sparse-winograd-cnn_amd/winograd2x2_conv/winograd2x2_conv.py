@@ -102,6 +102,10 @@ def _forward(I, W, precision, out, scale=None, shift=None, residual=None, residu
 def winograd2x2_weight_pieces(W, precision="fp32"):
     """W [16,C,K] float32 -> the bytes ``winograd2x2_conv(..., pieces=...)`` multiplies with: every weight as three bfloat16
     values whose sum it is, or with ``precision="bf16"`` rounded to one.  Prepare once per weight update."""
+    if precision in PRECISIONS:
+        out = _native.weight_pieces(W, precision == "bf16")
+        if out is not None:
+            return out
     W = swc_hip.require_cuda_f32(W, "W", 3)
     if W.shape[0] != 16:
         raise ValueError("W must have shape [16,C,K]")

@@ -378,3 +378,32 @@ def test_a_copied_layer_brings_no_kept_weights():
         state = dict(layer.__getstate__(), _masked=(b"", torch.zeros_like(layer.W)), _pieces=None)   # as layers kept them before
         other.__setstate__(state)
         assert close(other(ti), want)
+
+
+def test_pieces_that_do_not_pay_for_one_call_are_made_by_the_second():
+    import swc_hip
+    from winograd_conv import WinogradConv
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the gains are those of 256 CUs")
+    assert swc_hip.lib().swc_winograd2x2_conv_pieces_gain(512, 64, 4, 4, 512) == 1
+    gen = torch.Generator(device="cuda").manual_seed(30)
+    layer = WinogradConv(512, 512, mask=(torch.rand((16, 512, 512), device="cuda", generator=gen) < 0.3).float(), device="cuda")
+    ti = torch.randn((16, 64, 4, 4, 512), device="cuda", generator=gen).relu_()
+    form = swc_hip.lib().swc_winograd2x2_conv_last_form
+    with torch.no_grad():
+        for _ in range(2):
+            first = layer(ti)
+            assert layer._pieces is None and form() == b"split32"
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):   # would make them at every replay
+                y = layer(ti)
+            assert layer._pieces is None and form() == b"split32"
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, first)
+            second = layer(ti)
+            assert layer._pieces is not None and form() == b"pieces32"
+            assert (second - first).norm() <= 1e-6 * first.norm()
+            layer.W.mul_(2)
+            layer._pieces = None
