@@ -319,7 +319,7 @@ SWC_API int swc_winograd2x2_relu_pointwise_conv(const float *Input, const float 
  * 3x3 stride-2 max-pool over NHWC pixels with TensorFlow's SAME padding, Output [B,ceil(H/2),ceil(W/2),C], and the mean over all pixels of
  * relu(Input), Output [B,C]: the model's pools (imagenet-resnet-transWino-prune.py:115 and behind stages 2 and 3) and its last layer before the
  * classifier.  NaN propagates in both.  C % 4 == 0 and 16-byte aligned operands, below 2^31 groups of four channels in the
- * output and 2^20 pixels under a mean; SWC_ERR_UNSUPPORTED otherwise.
+ * output and at most 1024 pixels under a mean; SWC_ERR_UNSUPPORTED otherwise.
  */
 SWC_API int swc_max_pool_same(const float *Input, float *Output, int C, int B, int H, int W, swc_stream_t stream);
 SWC_API int swc_relu_mean(const float *Input, float *Output, int C, int B, int H, int W, swc_stream_t stream);

@@ -175,3 +175,17 @@ def test_model_pools(shape):
         if mean is not None:
             want = torch.relu(x.double()).mean(dim=(1, 2))
             assert torch.allclose(mean.cpu().double(), want, rtol=H * W * 2.0 ** -24 + 2.0 ** -23, atol=0, equal_nan=True)
+
+
+@pytest.mark.parametrize("shape", [(2, 32, 32, 68), (1, 33, 32, 64), (1, 64, 64, 64)])
+def test_relu_mean_up_to_its_longest_chain(shape):
+    # 1024 pixels are sums of 64 terms in sixteen parts, four more additions and a division, all of one sign: 69 * 2^-24.  Beyond, the
+    # library's reduction runs.
+    import resnet18_var
+    B, H, W, C = shape
+    x = torch.randn(shape, generator=torch.Generator().manual_seed(9)) * torch.logspace(-3, 3, C)
+    got = resnet18_var._native.relu_mean(x.cuda())
+    assert (got is None) == (H * W > 1024)
+    if got is not None:
+        want = torch.relu(x.double()).mean(dim=(1, 2))
+        assert ((got.cpu().double() - want).abs() <= 69 * 2.0 ** -24 * want).all()
