@@ -61,6 +61,17 @@ const float *optional(PyObject *o, const at::Tensor &like, at::IntArrayRef sizes
     return static_cast<const float *>(t->const_data_ptr());
 }
 
+// A flag; *ok is cleared where its truth value raises, which the general path then does again in its own place.
+bool truth(PyObject *o, bool *ok)
+{
+    const int value = PyObject_IsTrue(o);
+    if (value < 0) {
+        PyErr_Clear();
+        *ok = false;
+    }
+    return value > 0;
+}
+
 bool records(const at::Tensor &t) { return at::GradMode::is_enabled() && t.requires_grad(); }
 const float *floats(const at::Tensor &t) { return static_cast<const float *>(t.const_data_ptr()); }
 float *floats_of(at::Tensor &t) { return static_cast<float *>(t.mutable_data_ptr()); }
@@ -260,9 +271,9 @@ PyObject *imtrans(PyObject *, PyObject *const *args, Py_ssize_t count)
     SWC_ARGS(5)
     const at::Tensor *I = plain(args[0], at::kFloat, 4);
     if (I == nullptr || watched() || records(*I) || !fits(I->sizes())) return none();
-    const int relu = PyObject_IsTrue(args[1]), bf16 = PyObject_IsTrue(args[4]);
     const int64_t B = I->size(0), H = I->size(1), W = I->size(2), C = I->size(3);
-    bool ok = relu >= 0 && bf16 >= 0 && (args[2] == Py_None) == (args[3] == Py_None);
+    bool ok = (args[2] == Py_None) == (args[3] == Py_None);
+    const bool relu = truth(args[1], &ok), bf16 = truth(args[4], &ok);
     const float *scale = optional(args[2], *I, {C}, &ok), *shift = optional(args[3], *I, {C}, &ok);
     if (!ok) return none();
     at::Tensor out;
@@ -315,8 +326,9 @@ PyObject *conv(PyObject *, PyObject *const *args, Py_ssize_t count)
     if (I == nullptr || W == nullptr || watched() || records(*I) || records(*W) || I->device() != W->device()) return none();
     const int64_t B = I->size(1), nH = I->size(2), nW = I->size(3), C = I->size(4), K = W->size(2);
     if (I->size(0) != 16 || W->size(0) != 16 || W->size(1) != C || !fits(I->sizes()) || !fits(W->sizes())) return none();
-    const int bf16 = PyObject_IsTrue(args[2]), residual_relu = PyObject_IsTrue(args[6]);
-    bool ok = bf16 >= 0 && residual_relu >= 0 && (args[3] == Py_None) == (args[4] == Py_None) && !(residual_relu && args[5] == Py_None);
+    bool ok = (args[3] == Py_None) == (args[4] == Py_None);
+    const bool bf16 = truth(args[2], &ok), residual_relu = truth(args[6], &ok);
+    if (residual_relu && args[5] == Py_None) ok = false;
     const float *scale = optional(args[3], *I, {K}, &ok), *shift = optional(args[4], *I, {K}, &ok),
                 *residual = optional(args[5], *I, {B, 2 * nH, 2 * nW, K}, &ok);
     const bool for_this_call = args[7] == Py_True;
@@ -374,8 +386,8 @@ PyObject *conv_stored(PyObject *, PyObject *const *args, Py_ssize_t count)
     if (I == nullptr || W == nullptr || watched() || records(*I) || records(*W) || I->device() != W->device()) return none();
     const int64_t B = I->size(1), nH = I->size(2), nW = I->size(3), C = I->size(4), K = W->size(1);
     if (I->size(0) != 16 || W->size(0) != 16 || W->size(2) != C || !fits(I->sizes()) || !fits(W->sizes())) return none();
-    const int residual_relu = PyObject_IsTrue(args[5]), workspace = PyObject_IsTrue(args[6]);
-    bool ok = residual_relu >= 0 && workspace >= 0 && (args[2] == Py_None) == (args[3] == Py_None);
+    bool ok = (args[2] == Py_None) == (args[3] == Py_None);
+    const bool residual_relu = truth(args[5], &ok), workspace = truth(args[6], &ok);
     const float *scale = optional(args[2], *I, {K}, &ok), *shift = optional(args[3], *I, {K}, &ok),
                 *residual = optional(args[4], *I, {B, 2 * nH, 2 * nW, K}, &ok);
     if (!ok) return none();
@@ -434,7 +446,10 @@ PyObject *imtrans_grad(PyObject *, PyObject *const *args, Py_ssize_t count)
     SWC_ARGS(4)
     const at::Tensor *G = plain(args[0], at::kFloat, 5);
     const long H = PyLong_AsLong(args[1]), W = PyLong_AsLong(args[2]);
-    if ((H == -1 || W == -1) && PyErr_Occurred()) return nullptr;
+    if ((H == -1 || W == -1) && PyErr_Occurred()) {   // beyond 64 bits
+        PyErr_Clear();
+        return none();
+    }
     if (G == nullptr || watched() || G->size(0) != 16 || !fits(G->sizes()) || !fits({H, W})) return none();
     const int64_t B = G->size(1), C = G->size(4);
     bool ok = (H + 1) / 2 == G->size(2) && (W + 1) / 2 == G->size(3);
@@ -464,8 +479,9 @@ PyObject *pointwise(PyObject *, PyObject *const *args, Py_ssize_t count)
     if (x == nullptr || w == nullptr || watched() || records(*x) || records(*w) || x->device() != w->device() || w->size(1) != x->size(3) ||
         !fits(x->sizes()) || !fits(w->sizes()))
         return none();
-    const int relu = PyObject_IsTrue(args[2]);
-    bool ok = relu >= 0 && (args[3] == Py_None) == (args[4] == Py_None) && (relu || args[3] == Py_None);
+    bool ok = (args[3] == Py_None) == (args[4] == Py_None);
+    const bool relu = truth(args[2], &ok);
+    if (!relu && args[3] != Py_None) ok = false;
     const float *scale = optional(args[3], *x, {x->size(3)}, &ok), *shift = optional(args[4], *x, {x->size(3)}, &ok);
     if (!ok) return none();
     at::Tensor out;

@@ -82,6 +82,23 @@ def test_what_is_not_plain_takes_the_general_path():
         torch.func.vmap(lambda t: winograd2x2_imTrans(t))(o["x"].unsqueeze(0))
 
 
+def test_arguments_that_raise_do_so_as_in_the_general_path():
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv, winograd2x2_weights_bf16
+    from winograd2x2_imTrans.winograd2x2_imTrans import winograd2x2_imTrans, winograd2x2_imTrans_grad
+    o = operands()
+    neither = torch.ones(2)   # no truth value
+    ti16, w16 = o["ti"].bfloat16(), winograd2x2_weights_bf16(o["w"])
+    for call in (lambda: winograd2x2_imTrans(o["x"], relu=neither), lambda: winograd2x2_imTrans(o["x"], relu=neither, out_dtype=torch.bfloat16),
+                 lambda: winograd2x2_conv(o["ti"], o["w"], residual=o["res"], residual_relu=neither),
+                 lambda: winograd2x2_conv(ti16, w16, residual=o["res"], residual_relu=neither),
+                 lambda: winograd2x2_conv(ti16, w16, workspace=neither)):
+        with pytest.raises(RuntimeError, match="ambiguous"):
+            call()
+    for H, W in ((2 ** 70, 10), (7, -2 ** 70), (7, -1)):
+        with pytest.raises(ValueError, match="do not tile"):
+            winograd2x2_imTrans_grad(o["ti"], H, W)
+
+
 def test_gradients_through_both_paths():
     from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv_grad
     from winograd2x2_imTrans.winograd2x2_imTrans import winograd2x2_imTrans_grad
