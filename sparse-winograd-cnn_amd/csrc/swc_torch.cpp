@@ -1,7 +1,7 @@
 // The host side of the Python ops in native code: operand checks, allocation and launch in one call for the plain case.
 //
 // A call that is anything but plain -- another type than torch.Tensor, another device or dtype, a view that is not contiguous,
-// gradients to be recorded, a mode that watches calls, shapes that do not fit, a status that is not SWC_OK -- gets None back,
+// gradients to be recorded, a tangent, a mode or trace that watches calls, shapes that do not fit, a status that is not SWC_OK -- gets None back,
 // and the Python code around it, which has the whole rules and the messages, goes its own way.
 //
 // What it saves, times of a pass that the host bounds: the layer pair 1x16x16x64 23.3 -> 13.2 us, a training step 3x6x6x32 188.8 -> 96.9,
@@ -15,6 +15,7 @@
 #include <ATen/ops/empty.h>
 #include <ATen/ops/record_stream.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
@@ -33,7 +34,12 @@ struct NoGil {   // launches and allocations run without the interpreter's lock,
     ~NoGil() { PyEval_RestoreThread(state); }
 };
 
-bool watched() { return at::impl::torch_function_mode_enabled() || c10::impl::TorchDispatchModeTLS::any_modes_set(); }
+// A mode that watches calls, or a trace that records them.
+bool watched()
+{
+    return at::impl::torch_function_mode_enabled() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+           c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer);
+}
 
 const c10::DispatchKeySet kWrappers({c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot, c10::DispatchKey::Functionalize,
                                      c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
@@ -46,6 +52,7 @@ const at::Tensor *plain(PyObject *o, at::ScalarType dtype, int64_t rank)
     const at::Tensor &t = THPVariable_Unpack(o);
     if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || t.scalar_type() != dtype || t.dim() != rank) return nullptr;
     if (t.key_set().has_any(kWrappers) || !t.has_storage() || !t.is_contiguous()) return nullptr;
+    if (t._fw_grad(0).defined()) return nullptr;   // carries a tangent of forward-mode differentiation
     return &t;
 }
 

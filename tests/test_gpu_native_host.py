@@ -99,6 +99,24 @@ def test_arguments_that_raise_do_so_as_in_the_general_path():
             winograd2x2_imTrans_grad(o["ti"], H, W)
 
 
+def test_tangents_and_traces_go_through_the_models_pools():
+    # Torch's operators carry a tangent on and are recorded by a trace; the library's kernels would do neither.
+    import torch.autograd.forward_ad as fwd
+    import resnet18_var
+    gen = torch.Generator(device="cuda").manual_seed(92)
+    x, t, other = (torch.randn((2, 7, 10, 64), device="cuda", generator=gen).permute(0, 3, 1, 2) for _ in range(3))
+    plain = resnet18_var._max_pool_same(x)
+    with fwd.dual_level():
+        out = fwd.unpack_dual(resnet18_var._max_pool_same(fwd.make_dual(x, t)))
+        assert torch.equal(out.primal, plain)
+        pads = resnet18_var._same_pad(x, 3, 2)
+        padded, at = torch.nn.functional.pad(x, pads, value=float("-inf")), torch.nn.functional.pad(t, pads)
+        index = torch.nn.functional.max_pool2d(padded, 3, 2, return_indices=True)[1]
+        assert torch.equal(out.tangent, at.flatten(2).gather(2, index.flatten(2)).view_as(plain))
+    traced = torch.jit.trace(resnet18_var._max_pool_same, (x,))
+    assert torch.equal(traced(other), resnet18_var._max_pool_same(other))
+
+
 def test_gradients_through_both_paths():
     from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv_grad
     from winograd2x2_imTrans.winograd2x2_imTrans import winograd2x2_imTrans_grad
