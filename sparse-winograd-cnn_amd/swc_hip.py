@@ -50,22 +50,52 @@ CXX_SYMBOLS = (
 )
 
 _lib = None
-_native = None
+
+
+def _load_native():
+    lib()
+    import torch  # noqa: F401  (its libraries are what the module is linked against)
+
+    spec = importlib.util.spec_from_file_location("_swc_torch", NATIVE_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
+
+
+def _python_key(*tensors):
+    return tuple(None if t is None else (t._version, t.data_ptr(), t.device) for t in tensors)
+
+
+def _not_built(name):
+    def call(*args):
+        if any(getattr(a, "is_cuda", False) for a in args):
+            lib()
+            raise ImportError("%s is missing: build it with `make -C %s` (or __graft_entry__.build())" % (NATIVE_PATH, CSRC))
+        return args[0] if name == "here" else {"mark": True, "capturing": False}.get(name)
+    return call
+
+
+class _Native(object):
+    """The functions of csrc/swc_torch.cpp, loaded by the first one that is used.  Where they have not been built, what is not on the GPU
+    takes the Python code around them, and what is raises."""
+
+    def __getattr__(self, name):
+        if name.startswith("__"):
+            raise AttributeError(name)
+        if not (os.path.exists(NATIVE_PATH) and os.path.exists(LIB_PATH)):
+            return _python_key if name == "key" else _not_built(name)
+        module = _load_native()
+        for f in dir(module):
+            if not f.startswith("__"):
+                setattr(self, f, getattr(module, f))
+        return getattr(module, name)
+
+
+_native = _Native()
 
 
 def native():
     """The native host side of the ops (csrc/swc_torch.cpp)."""
-    global _native
-    if _native is None:
-        lib()
-        import torch  # noqa: F401  (its libraries are what the module is linked against)
-
-        if not os.path.exists(NATIVE_PATH):
-            raise ImportError("%s is missing: build it with `make -C %s` (or __graft_entry__.build())" % (NATIVE_PATH, CSRC))
-        spec = importlib.util.spec_from_file_location("_swc_torch", NATIVE_PATH)
-        module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(module)
-        _native = module
     return _native
 
 

@@ -265,3 +265,49 @@ def test_a_layer_pickled_without_pieces_still_works():
     old.__setstate__(state)
     assert old._pieces is None
     old.refresh()
+
+
+def test_modules_import_without_a_build(tmp_path):
+    """Without the two libraries everything imports, what needs no GPU runs, and loading the library says what is missing."""
+    import shutil
+    import subprocess
+    import sys
+    pkg = os.path.dirname(os.path.abspath(swc_hip.__file__))
+    copy = tmp_path / "package"
+    shutil.copytree(pkg, copy, ignore=shutil.ignore_patterns("*.so", "build", "__pycache__"))
+    code = """
+import sys
+sys.path.insert(0, sys.argv[1])
+import torch, swc_hip, resnet18_var, winograd_conv, winograd_imtrans
+assert swc_hip.__file__.startswith(sys.argv[1])
+layer = winograd_conv.WinogradConv(4, 8, mask=torch.ones(16, 4, 8))
+assert torch.equal(layer.masked_weight(), layer.W) and layer.masked_weight() is layer.masked_weight()
+with torch.no_grad():
+    layer.W.add_(1)
+assert torch.equal(layer.masked_weight(), layer.W)
+x = torch.randn(1, 5, 6, 32)
+assert resnet18_var._max_pool_same(x).shape == (1, 5, 3, 16)
+assert resnet18_var.pointwise_conv(x, torch.randn(8, 32)).shape == (1, 5, 6, 8)
+resnet18_var._bn_affine(torch.nn.BatchNorm2d(4))
+for call, error in ((lambda: winograd_imtrans.WinogradImTrans(x), RuntimeError), (swc_hip.lib, ImportError)):
+    try:
+        call()
+    except error as e:
+        print(type(e).__name__)
+    else:
+        raise SystemExit("nothing raised")
+"""
+    out = subprocess.run([sys.executable, "-c", code, str(copy)], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, out.stderr
+    assert out.stdout.split() == ["RuntimeError", "ImportError"]
+
+
+def test_the_library_builds_without_pytorch():
+    """`make` names the library alone where there are no headers of PyTorch, and both where there are."""
+    import subprocess
+    run = lambda *a: subprocess.run(["make", "-n", "-B", "-C", swc_hip.CSRC] + list(a), capture_output=True, text=True)   # noqa: E731
+    alone, both = run("PYTHON=/bin/false"), run()
+    assert alone.returncode == 0 and both.returncode == 0
+    link = "-o " + os.path.join("..", os.path.basename(swc_hip.NATIVE_PATH))
+    assert link not in alone.stdout and "is not built" in alone.stdout and os.path.basename(swc_hip.LIB_PATH) in alone.stdout
+    assert link in both.stdout and "is not built" not in both.stdout
