@@ -78,7 +78,7 @@ namespace {
 PiecesChoice choose_bf16(size_t M, int C, double c, size_t cus, size_t tiles_n)
 {
     PiecesChoice best;
-    if (C % 64 != 0 || C < 256) return best;
+    if (C < 256) return best;
     auto rounds_of = [&](size_t rows, size_t high) { return static_cast<double>(((rows + high - 1) / high * tiles_n + cus - 1) / cus); };
     if (rounds_of(M, 32) <= 1) {
         if (C >= 512 && tiles_n >= 8 && M * C * 64 <= (64u << 20)) best = {PIECES_32, 0, 3.6 + 3.3 * c};
@@ -111,7 +111,7 @@ PiecesChoice choose_bf16(size_t M, int C, double c, size_t cus, size_t tiles_n)
 PiecesChoice choose_pieces(const void *TI, const void *Wt, const void *Wp, const void *Out, const void *residual, size_t M, int C, int K, bool bf16)
 {
     PiecesChoice best;
-    if (!pieces_eligible(TI, Wt, Wp, Out, residual, M, C, K)) return best;
+    if (!pieces_eligible(TI, Wt, Wp, Out, residual, M, C, K) || (bf16 && C % 64 != 0)) return best;
     if (const char *f = forced_conv_tiling()) {
         for (int i = PIECES_32; i < PIECES_FORMS; ++i)
             if (std::string_view(f) == kPiecesNames[i]) best = {static_cast<PiecesForm>(i), M / 128, 0.0};
@@ -151,17 +151,12 @@ int launch_pieces(const PiecesChoice &pick, bool bf16, const float *TI, const fl
     ep.residual_relu = residual_relu;
     const bool ragged = C % 16 != 0, deep = steps_of(C) % 2 == 0 && !ragged;
     if (bf16) {
-        const bool whole = C % 64 == 0;   // otherwise what lies beyond C is read as zero: beside it there may be an infinity
-        using R32 = PiecesCfg<1, 2, true, 1>;
-        using R64 = PiecesCfg<2, 2, true, 1>;
-        using D32 = PiecesCfg<1, 4, false, 1>;
+        using D32 = PiecesCfg<1, 4, false, 1>;   // C % 64 == 0: twice the half steps on their way
         using D64 = PiecesCfg<2, 4, false, 1>;
-        switch (pick.form) {   // twice the half steps on their way where C takes them
-            case PIECES_64: return whole ? launch_as<D64>(TI, Wt, Wp, Out, M, C, K, nW, 0, ep, s) : launch_as<R64>(TI, Wt, Wp, Out, M, C, K, nW, 0, ep, s);
-            case PIECES_32: return whole ? launch_as<D32>(TI, Wt, Wp, Out, M, C, K, nW, 0, ep, s) : launch_as<R32>(TI, Wt, Wp, Out, M, C, K, nW, 0, ep, s);
-            case PIECES_64_32:
-                return whole ? launch_as<D64, D32>(TI, Wt, Wp, Out, M, C, K, nW, pick.main_m, ep, s)
-                            : launch_as<R64, R32>(TI, Wt, Wp, Out, M, C, K, nW, pick.main_m, ep, s);
+        switch (pick.form) {
+            case PIECES_64: return launch_as<D64>(TI, Wt, Wp, Out, M, C, K, nW, 0, ep, s);
+            case PIECES_32: return launch_as<D32>(TI, Wt, Wp, Out, M, C, K, nW, 0, ep, s);
+            case PIECES_64_32: return launch_as<D64, D32>(TI, Wt, Wp, Out, M, C, K, nW, pick.main_m, ep, s);
             default: return SWC_ERR_UNSUPPORTED;
         }
     }

@@ -223,10 +223,10 @@ def test_pieces_that_are_not_the_weights_are_refused():
 
 
 @pytest.mark.parametrize("form", ["pieces32", "pieces64", "pieces64+32"])
-@pytest.mark.parametrize("shape", [(1, 1, 1, 4, 4), (1, 4, 8, 48, 64), (2, 5, 6, 64, 68), (1, 13, 5, 80, 132), (2, 8, 8, 128, 64), (3, 9, 7, 320, 200)])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 64, 4), (1, 4, 8, 192, 64), (2, 5, 6, 64, 68), (1, 13, 5, 128, 132), (2, 8, 8, 128, 64), (3, 9, 7, 320, 200)])
 def test_bf16_operands(shape, form):
-    # Rows, columns and channels below, at and beyond a tile (32 or 64 rows, 64 columns, half steps of 16 indices, four of them on their
-    # way where C % 64 == 0).  Whole numbers are exact in bf16 and in any order of the sums; for others the kernel's products are those of
+    # Rows and columns below, at and beyond a tile (32 or 64 rows, 64 columns), one, two, three and five times the four half steps of 16
+    # indices that are on their way.  Whole numbers are exact in bf16 and in any order of the sums; for others the kernel's products are those of
     # the rounded operands, summed in fp32: at most C roundings of 2^-24 each for sums of at most sum|a b|.
     from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv, winograd2x2_weight_pieces
     import swc_hip
@@ -241,7 +241,9 @@ def test_bf16_operands(shape, form):
         pieces = winograd2x2_weight_pieces(w.to(dev), "bf16")
         assert lib.swc_winograd2x2_conv_force_tiling(name.encode() if name else None) == 0
         try:
-            return winograd2x2_conv(ti.to(dev), w.to(dev), "bf16", pieces=pieces if name else None).cpu()
+            y = winograd2x2_conv(ti.to(dev), w.to(dev), "bf16", pieces=pieces if name else None).cpu()
+            assert name is None or lib.swc_winograd2x2_conv_last_form().decode() == name
+            return y
         finally:
             lib.swc_winograd2x2_conv_force_tiling(None)
     assert torch.equal(conv(*whole, form), conv(*whole, None))
@@ -261,6 +263,53 @@ def test_bf16_operands(shape, form):
     got, want = conv(bad, real[1], form), conv(bad, real[1], None)
     assert torch.equal(got.isfinite(), want.isfinite())
     assert (~got.isfinite()).sum() == 4 * K
+
+
+@pytest.mark.parametrize("precision,shape,form", [
+    ("bf16", (95, 7, 7, 512, 256), "pieces64+32"),     # 292 tiles: a round of 64-row ones, the rest in 32-row ones
+    ("bf16", (128, 7, 7, 512, 512), "pieces64+32"),    # three rounds, two panels of columns
+    ("bf16", (128, 7, 7, 256, 256), "pieces64"),       # two rounds, the second of 136 tiles
+    ("fp32", (128, 7, 7, 512, 512), "pieces64+32"),
+    ("fp32", (68, 28, 4, 192, 256), "pieces64"),       # two rounds
+])
+def test_several_rounds_as_the_launcher_takes_them(precision, shape, form):
+    """A workgroup's later tiles, whose operands are loaded beside the one before, panels of columns and the lower tiles behind: against
+    float64 of the operands as they are multiplied, all rows."""
+    import swc_hip
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv, winograd2x2_weight_pieces
+    B, nH, nW, C, K = shape
+    gen = torch.Generator(device="cuda").manual_seed(31)
+    ti = torch.randn((16, B, nH, nW, C), device="cuda", generator=gen).relu_()
+    w = torch.randn((16, C, K), device="cuda", generator=gen) * 0.05
+    got = winograd2x2_conv(ti, w, precision, pieces=winograd2x2_weight_pieces(w, precision))
+    if form is not None and torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert swc_hip.lib().swc_winograd2x2_conv_last_form().decode() == form
+    a, b = (ti.reshape(16, -1, C), w) if precision == "fp32" else (ti.reshape(16, -1, C).bfloat16().float(), w.bfloat16().float())
+    y = torch.zeros((2, 2, B * nH * nW, K), dtype=torch.float64, device="cuda")
+    size = torch.zeros_like(y)
+    at = torch.tensor([[1, 1, 1, 0], [0, 1, -1, -1]], dtype=torch.float64)
+    for i in range(16):
+        p, q = torch.mm(a[i].double(), b[i].double()), torch.mm(a[i].double(), b[i].double().abs())
+        for dy in range(2):
+            for dx in range(2):
+                f = float(at[dy, i // 4] * at[dx, i % 4])
+                if f:
+                    y[dy, dx] += f * p
+                    size[dy, dx] += q
+    got = got.reshape(B, nH, 2, nW, 2, K).permute(2, 4, 0, 1, 3, 5).reshape(y.shape)
+    # at most C roundings of a sum, and what nine terms and three pieces add
+    assert ((got.double() - y).abs() <= (C + 16) * 2.0 ** -24 * size).all()
+    assert (got.double() - y).norm() <= 1e-6 * y.norm()
+
+
+@pytest.mark.parametrize("C", [4, 48, 80, 96])
+def test_bf16_operands_of_other_channels_are_multiplied_with_the_weights_themselves(forced, C):  # noqa: F811
+    from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv, winograd2x2_weight_pieces
+    gen = torch.Generator(device="cuda").manual_seed(32)
+    ti, w = torch.randn((16, 2, 5, 6, C), device="cuda", generator=gen), torch.randn((16, C, 68), device="cuda", generator=gen)
+    want = winograd2x2_conv(ti, w, "bf16")
+    assert torch.equal(winograd2x2_conv(ti, w, "bf16", pieces=winograd2x2_weight_pieces(w, "bf16")), want)
+    assert not forced.swc_winograd2x2_conv_last_form().startswith(b"pieces")
 
 
 @pytest.mark.parametrize("masked", [True, False])
