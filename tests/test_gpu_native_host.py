@@ -63,12 +63,19 @@ def test_what_is_not_plain_takes_the_general_path():
         assert not winograd2x2_conv(winograd2x2_imTrans(x), w).requires_grad
     with torch.inference_mode():
         assert torch.equal(winograd2x2_conv(winograd2x2_imTrans(o["x"]), o["w"]), plain)
-    side = torch.cuda.Stream()
-    side.wait_stream(torch.cuda.current_stream())
+    # on a side stream that is busy and then writes what the ops read: launched on another, they would read zeros
+    side, late = torch.cuda.Stream(), torch.zeros_like(o["x"])
+    busy = torch.ones((4096, 4096), device="cuda")
+    torch.cuda.synchronize()
     with torch.cuda.stream(side):
-        other = winograd2x2_conv(winograd2x2_imTrans(o["x"]), o["w"])
+        for _ in range(20):
+            busy = torch.mm(busy, busy).clamp_(max=1)
+        late.copy_(o["x"])
+        other = winograd2x2_conv(winograd2x2_imTrans(late), o["w"])
+        last = winograd2x2_imTrans(other)
+        other.zero_()   # and the convolution's output is not written to once more
     side.synchronize()
-    assert torch.equal(other, plain)
+    assert torch.equal(last, winograd2x2_imTrans(plain)) and not other.any()
     for bad in (o["x"].double(), o["x"].cpu(), o["x"][0], "x"):
         with pytest.raises((TypeError, ValueError, RuntimeError)):
             winograd2x2_imTrans(bad)

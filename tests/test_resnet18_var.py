@@ -141,17 +141,23 @@ def _forward_against_oracle_path(oracle, precision, tol, batch, size, check_unfo
 LAYER_SHAPES = [(56, 64, 64), (28, 64, 128), (28, 128, 128), (14, 128, 256), (14, 256, 256), (14, 256, 512), (14, 512, 512)]
 
 
+# What a masked layer of that size runs at batch 128 on 256 CUs where it uses its prepared weights.
+PREPARED = {("fp32", 14, 128, 256): "pieces64", ("fp32", 14, 256, 512): "pieces64+32", ("fp32", 14, 512, 512): "pieces64+32",
+            ("bf16", 14, 256, 256): "pieces64", ("bf16", 14, 256, 512): "pieces64+32", ("bf16", 14, 512, 512): "pieces64+32"}
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("precision", ["fp32", "bf16", "bf16_stored"])
 @pytest.mark.parametrize("hw,C,K", LAYER_SHAPES)
 def test_layers_at_batch_128(oracle, hw, C, K, precision):
-    """Every layer shape of config 5 at its real batch (N = 128), so that the launcher makes the choice it
-    makes in the benchmark: the transform is compared bit for bit and the convolution within tolerance with
+    """Every layer shape of config 5 at its real batch (N = 128), on W itself and through the masked layer that the
+    model has, so that the launcher makes the choices it makes in the benchmark: the transform is compared bit for bit and the convolution within tolerance with
     the oracle on the first and the last two images (tiles are independent, so a slice of the batch has the
     values it would have alone; the last images sit in the ragged final row groups)."""
     import swc_hip
     from winograd2x2_conv.winograd2x2_conv import winograd2x2_conv
     from winograd2x2_imTrans.winograd2x2_imTrans import winograd2x2_imTrans
+    from winograd_conv import WinogradConv
     dev = torch.device("cuda:0")
     N, k = 128, 2
     gen = torch.Generator(device=dev).manual_seed(hw * 1000 + C + K)
@@ -164,6 +170,13 @@ def test_layers_at_batch_128(oracle, hw, C, K, precision):
     y = winograd2x2_conv(ti, w_gpu, precision="fp32" if stored else precision)
     kernel = swc_hip.lib().swc_winograd2x2_conv_last_kernel().decode()
     assert y.shape == (N, hw, hw, K)
+    layer = WinogradConv(C, K, mask=(w_gpu != 0).float(), W_init=w_gpu, device=dev, precision="bf16" if stored else precision)
+    with torch.no_grad():
+        for _ in range(2):   # the second call at the latest uses prepared weights
+            y_layer = layer(ti)
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256 and not stored:
+        form = swc_hip.lib().swc_winograd2x2_conv_last_form().decode()
+        assert PREPARED.get((precision, hw, C, K)) == (form if form.startswith("pieces") else None)
     for sl in (slice(0, k), slice(N - k, N)):
         x_cpu = x[sl].cpu().numpy()
         ti_want = oracle.imtrans(x_cpu, relu=True)
@@ -177,6 +190,7 @@ def test_layers_at_batch_128(oracle, hw, C, K, precision):
                 ti_want, w_want = oracle.round_bf16(ti_want), oracle.round_bf16(w)
         want = oracle.conv(ti_want, w_want, acc64=True)
         assert rel_max(y[sl].cpu().numpy(), want) <= 1e-4, (kernel, sl)
+        assert rel_max(y_layer[sl].cpu().numpy(), want) <= 1e-4, sl
     if precision == "fp32":
         assert kernel in ("tall16", "wide48", "wide48x64", "split64+32", "split64+48"), kernel   # no model shape is small at this batch
     if stored:
