@@ -158,8 +158,8 @@ SWC_API int swc_winograd2x2_conv_epilogue(const float *Input, const float *Weigh
  * swc_winograd2x2_weights_bf16.
  * swc_winograd2x2_conv_prepared is swc_winograd2x2_conv_epilogue with precision 0; Pieces are Weight's, or NULL, and are used
  * where that is the faster way and the operands are aligned; results agree to fp32 rounding.
- * swc_winograd2x2_conv_pieces_gain says for a shape on the current device whether it is: 0 no, 1 yes, 2 also if the pieces
- * have to be made for this call alone.
+ * swc_winograd2x2_conv_pieces_gain says for a shape on the current device whether pieces are worth making: 0 no (they are not
+ * faster, or by too little), 1 for a few calls, 2 for one call alone.
  */
 SWC_API size_t swc_winograd2x2_weight_pieces_bytes(int C, int K);
 SWC_API int swc_winograd2x2_weight_pieces(const float *Weight, void *Pieces, int C, int K, swc_stream_t stream);

@@ -184,21 +184,6 @@ PyObject *hip_error(hipError_t st)
     return nullptr;
 }
 
-// capturing(tensor): whether the current stream on the tensor's device records a graph.
-PyObject *is_capturing(PyObject *, PyObject *const *args, Py_ssize_t count)
-{
-    SWC_ARGS(1)
-    if (!THPVariable_Check(args[0])) {
-        PyErr_SetString(PyExc_TypeError, "a tensor");
-        return nullptr;
-    }
-    const at::Tensor &t = THPVariable_Unpack(args[0]);
-    if (!t.is_cuda()) return PyBool_FromLong(0);
-    const c10::DeviceGuard guard(t.device());
-    return PyBool_FromLong(capturing(static_cast<hipStream_t>(stream_of(t))));
-    END_HANDLE_TH_ERRORS
-}
-
 // mark(tensor): behind what the current stream has been given on the tensor's device, or None while that stream records a graph.
 PyObject *mark(PyObject *, PyObject *const *args, Py_ssize_t count)
 {
@@ -532,7 +517,6 @@ using Fast = PyObject *(*)(PyObject *, PyObject *const *, Py_ssize_t);
 PyMethodDef method(const char *name, Fast f) { return {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)), METH_FASTCALL, nullptr}; }
 
 PyMethodDef methods[] = {method("key", key),
-                         method("capturing", is_capturing),
                          method("mark", mark),
                          method("here", here),
                          method("imtrans", imtrans),

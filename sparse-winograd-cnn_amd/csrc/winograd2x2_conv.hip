@@ -223,8 +223,10 @@ int gain_of(int C, int B, int nH, int nW, int K)
     const PiecesChoice pieces = choose_pieces(nullptr, nullptr, nullptr, nullptr, nullptr, M, C, K, BF16);
     const double gain = pieces_gain(pieces, choice);
     // Making them: 1.2 us for every 2^20 values and 4 between two other kernels (4416x64->192 behind the transform 27.8 us on W, 29.5 on
-    // pieces made for the call), 2.5 for one bf16 value each, where W*mask has just been written.
-    return gain > (BF16 ? 2.5 : 4.0) + 1.2 / (1 << 20) * 16 * C * K ? 2 : gain > 0 ? 1 : 0;
+    // pieces made for the call), 2.5 for one bf16 value each, where W*mask has just been written.  Where a call gains less than a quarter of
+    // that, the calls that follow it may be too few.
+    const double making = (BF16 ? 2.5 : 4.0) + 1.2 / (1 << 20) * 16 * C * K;
+    return gain > making ? 2 : gain > making / 4 ? 1 : 0;
 }
 }  // namespace
 }  // namespace swc

@@ -71,7 +71,7 @@ def _not_built(name):
         if any(getattr(a, "is_cuda", False) for a in args):
             lib()
             raise ImportError("%s is missing: build it with `make -C %s` (or __graft_entry__.build())" % (NATIVE_PATH, CSRC))
-        return args[0] if name == "here" else {"mark": True, "capturing": False}.get(name)
+        return args[0] if name == "here" else True if name == "mark" else None
     return call
 
 

@@ -33,7 +33,7 @@ class WinogradConv(torch.nn.Module):
     W is a trainable parameter; gradients come from ``winograd2x2_conv_grad``.
     """
 
-    _pieces = _wanted = None   # also for a layer that was pickled without them
+    _pieces = None   # also for a layer that was pickled without it
 
     def __init__(self, in_channel, out_channel, mask=None, W_init=None, precision="fp32", device=None):
         super().__init__()
@@ -54,10 +54,10 @@ class WinogradConv(torch.nn.Module):
         self._bf16 = None
 
     def __getstate__(self):
-        return dict(self.__dict__, _masked=None, _bf16=None, _pieces=None, _wanted=None)   # made anew by the copy
+        return dict(self.__dict__, _masked=None, _bf16=None, _pieces=None)   # made anew by the copy
 
     def __setstate__(self, state):
-        super().__setstate__(dict(state, _masked=None, _bf16=None, _pieces=None, _wanted=None))   # also for a state that holds them in another form
+        super().__setstate__(dict(state, _masked=None, _bf16=None, _pieces=None))   # also for a state that holds them in another form
 
     def refresh(self):
         """Drop the cached W*mask, its bf16 copy and its pieces.  Not needed after in-place updates of W or mask made on
@@ -69,7 +69,6 @@ class WinogradConv(torch.nn.Module):
         self._masked = None
         self._bf16 = None
         self._pieces = None
-        self._wanted = None
 
     def _weight_key(self):
         # In-place writes bump _version; a replaced or moved tensor changes data_ptr / device.
@@ -95,18 +94,13 @@ class WinogradConv(torch.nn.Module):
 
     def weight_pieces(self):
         """W*mask taken apart for the fp32 convolution, or rounded and put in order for the one with bf16 operands; cached like masked_weight()."""
-        return self._pieces_of(self.masked_weight(), 2)
+        return self._pieces_of(self.masked_weight())
 
-    def _pieces_of(self, masked, gain):
-        """The pieces of ``masked`` for a call that gains by them: made at once where that alone pays (``gain`` 2), else by the second
-        call that would have used them, None for the first: the weights may change before there is another."""
+    def _pieces_of(self, masked):
         kept, key = self._pieces, (self._weight_key(), self.precision)
         tensor = _native.here(kept[1], kept[2]) if kept is not None and kept[0] == key else None
         if tensor is not None:
             return tensor
-        if gain == 1 and (self._wanted != key or _native.capturing(masked)):
-            self._wanted = key
-            return None
         return self._keep("_pieces", key, winograd2x2_conv.winograd2x2_conv.winograd2x2_weight_pieces(masked, self.precision))
 
     def masked_weight(self):
@@ -136,8 +130,7 @@ class WinogradConv(torch.nn.Module):
             if self.mask is None:
                 pieces = True
             elif self.precision in ("fp32", "bf16"):
-                gain = _native.pieces_gain(x, self.out_channel, self.precision == "bf16")
-                if gain and x.device == w.device and x.shape[4] == w.shape[1]:
-                    pieces = self._pieces_of(w, gain)
+                if _native.pieces_gain(x, self.out_channel, self.precision == "bf16") and x.device == w.device and x.shape[4] == w.shape[1]:
+                    pieces = self._pieces_of(w)
         scale, shift = affine if affine is not None else (None, None)
         return winograd2x2_conv.winograd2x2_conv.winograd2x2_conv(x, w, self.precision, None, scale, shift, residual, residual_relu, True, pieces)
