@@ -101,7 +101,11 @@ class WinogradConv(torch.nn.Module):
         tensor = _native.here(kept[1], kept[2]) if kept is not None and kept[0] == key else None
         if tensor is not None:
             return tensor
-        return self._keep("_pieces", key, winograd2x2_conv.winograd2x2_conv.winograd2x2_weight_pieces(masked, self.precision))
+        if self.mask is not None:   # the key that `masked` was made under: another thread may have written to W since
+            source = self._masked
+            key = (source[0], self.precision) if source is not None and source[1] is masked else None
+        pieces = winograd2x2_conv.winograd2x2_conv.winograd2x2_weight_pieces(masked, self.precision)
+        return self._keep("_pieces", key, pieces) if key is not None else pieces
 
     def masked_weight(self):
         """W*mask without autograd history, recomputed only when W or mask changed since the last call (a write

@@ -311,3 +311,21 @@ def test_the_library_builds_without_pytorch():
     link = "-o " + os.path.join("..", os.path.basename(swc_hip.NATIVE_PATH))
     assert link not in alone.stdout and "is not built" in alone.stdout and os.path.basename(swc_hip.LIB_PATH) in alone.stdout
     assert link in both.stdout and "is not built" not in both.stdout
+
+
+def test_pieces_are_kept_under_the_key_of_what_they_were_made_of(monkeypatch):
+    """A write to W between W*mask and its pieces, as another thread may do: the next call makes both anew."""
+    import winograd2x2_conv.winograd2x2_conv as conv
+    from winograd_conv import WinogradConv
+    monkeypatch.setattr(conv, "winograd2x2_weight_pieces", lambda masked, precision: masked.clone())
+    layer = WinogradConv(4, 8, mask=torch.ones(16, 4, 8))
+    before = layer.masked_weight()
+    with torch.no_grad():
+        layer.W.add_(1)
+    assert torch.equal(layer._pieces_of(before), before)
+    assert torch.equal(layer.weight_pieces(), layer.W) and layer.weight_pieces() is layer.weight_pieces()
+    other = before.clone()   # not what the layer keeps: used and not kept
+    with torch.no_grad():
+        layer.W.add_(1)
+    assert torch.equal(layer._pieces_of(other), other)
+    assert torch.equal(layer.weight_pieces(), layer.W)
