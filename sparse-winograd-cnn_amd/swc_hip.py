@@ -71,11 +71,17 @@ def _not_built(name):
         if any(getattr(a, "is_cuda", False) for a in args):
             lib()
             raise ImportError("%s is missing: build it with `make -C %s` (or __graft_entry__.build())" % (NATIVE_PATH, CSRC))
-        return args[0] if name == "here" else True if name == "mark" else None
+        if name == "kept":
+            return args[0][1] if args[0] is not None and args[0][0] == _python_key(*args[1:]) else None
+        return True if name == "mark" else None
     return call
 
 
-class _Native(object):
+class _Loaded(object):
+    """The loaded functions as plain attributes: a class with ``__getattr__`` looks them up twice as slowly."""
+
+
+class _Native(_Loaded):
     """The functions of csrc/swc_torch.cpp, loaded by the first one that is used.  Where they have not been built, what is not on the GPU
     takes the Python code around them, and what is raises."""
 
@@ -88,6 +94,7 @@ class _Native(object):
         for f in dir(module):
             if not f.startswith("__"):
                 setattr(self, f, getattr(module, f))
+        self.__class__ = _Loaded
         return getattr(module, name)
 
 

@@ -74,38 +74,38 @@ class WinogradConv(torch.nn.Module):
         # In-place writes bump _version; a replaced or moved tensor changes data_ptr / device.
         return _native.key(self.W, self.mask)
 
-    def _keep(self, slot, key, tensor):
+    def _keep(self, slot, key, tensor, *made_for):
         """``tensor``, made of the weights that ``key`` stands for, kept in ``slot`` with a mark behind it in the stream that wrote it: a
         call on another stream may find it before it has been written, or drop it (the weights changed) while that stream's kernels
-        read it, and ``here`` sees to both.  While a graph is captured nothing is kept: what the capture records is written when the
+        read it, and ``kept`` sees to both.  While a graph is captured nothing is kept: what the capture records is written when the
         graph runs, and other calls would read it before."""
         mark = _native.mark(tensor)
         if mark is not None:
-            setattr(self, slot, (key, tensor, mark))
+            setattr(self, slot, (key, tensor, mark) + made_for)
         return tensor
 
     def bf16_weight(self):
         """W*mask as the [16,K,C] bfloat16 tensor the bf16-stored kernel reads; cached like masked_weight()."""
-        kept, key = self._bf16, self._weight_key()
-        tensor = _native.here(kept[1], kept[2]) if kept is not None and kept[0] == key else None
+        tensor = _native.kept(self._bf16, self.W, self.mask)
         if tensor is not None:
             return tensor
-        return self._keep("_bf16", key, winograd2x2_conv.winograd2x2_conv.winograd2x2_weights_bf16(self.masked_weight()))
+        return self._keep("_bf16", self._weight_key(), winograd2x2_conv.winograd2x2_conv.winograd2x2_weights_bf16(self.masked_weight()))
 
     def weight_pieces(self):
         """W*mask taken apart for the fp32 convolution, or rounded and put in order for the one with bf16 operands; cached like masked_weight()."""
         return self._pieces_of(self.masked_weight())
 
     def _pieces_of(self, masked):
-        kept, key = self._pieces, (self._weight_key(), self.precision)
-        tensor = _native.here(kept[1], kept[2]) if kept is not None and kept[0] == key else None
+        precision, entry = self.precision, self._pieces
+        tensor = _native.kept(entry, self.W, self.mask) if entry is not None and entry[3] == precision else None
         if tensor is not None:
             return tensor
+        key = self._weight_key()
         if self.mask is not None:   # the key that `masked` was made under: another thread may have written to W since
             source = self._masked
-            key = (source[0], self.precision) if source is not None and source[1] is masked else None
-        pieces = winograd2x2_conv.winograd2x2_conv.winograd2x2_weight_pieces(masked, self.precision)
-        return self._keep("_pieces", key, pieces) if key is not None else pieces
+            key = source[0] if source is not None and source[1] is masked else None
+        pieces = winograd2x2_conv.winograd2x2_conv.winograd2x2_weight_pieces(masked, precision)
+        return self._keep("_pieces", key, pieces, precision) if key is not None else pieces
 
     def masked_weight(self):
         """W*mask without autograd history, recomputed only when W or mask changed since the last call (a write
@@ -113,11 +113,10 @@ class WinogradConv(torch.nn.Module):
         W, mask = self.W, self.mask
         if mask is None:
             return W.detach()   # shares W's version counter: a write to what is handed out is noticed
-        kept, key = self._masked, _native.key(W, mask)
-        tensor = _native.here(kept[1], kept[2]) if kept is not None and kept[0] == key else None
+        tensor = _native.kept(self._masked, W, mask)
         if tensor is not None:
             return tensor
-        return self._keep("_masked", key, (W.detach() * mask).contiguous())
+        return self._keep("_masked", _native.key(W, mask), (W.detach() * mask).contiguous())
 
     def forward(self, x, affine=None, residual=None, residual_relu=False):
         """``affine=(scale, shift)`` and ``residual`` (forward only) are applied to the result inside
