@@ -65,7 +65,7 @@ SWC_API const char *swc_winograd2x2_conv_last_kernel(void);
  * split over eight waves, on the 16-bit matrix instructions: fp32 operands in three bf16 pieces each, which hold all their
  * bits (nearer to float64 than the fp32 instructions; a tile with operands above 2^30 or sums below 2^-75 is multiplied
  * with those, operands below 2^-134 count as zero), or bf16 operands; or "pieces32" / "pieces64" / "pieces64+32": the same
- * with fp32 weights that were taken apart beforehand (swc_winograd2x2_conv_prepared). */
+ * on weights that were prepared beforehand (swc_winograd2x2_conv_prepared, swc_winograd2x2_conv_prepared_bf16). */
 SWC_API const char *swc_winograd2x2_conv_last_form(void);
 /* Diagnostic with no counterpart in the reference, for benchmarks and tests that compare the tilings: makes
  * the calling thread's later swc_winograd2x2_conv calls

@@ -1,11 +1,11 @@
 // The host side of the Python ops in native code: operand checks, allocation and launch in one call for the plain case.
 //
 // A call that is anything but plain -- another type than torch.Tensor, another device or dtype, a view that is not contiguous,
-// gradients to be recorded, a tangent, a mode or trace that watches calls, shapes that do not fit, a status that is not SWC_OK -- gets None back,
-// and the Python code around it, which has the whole rules and the messages, goes its own way.
+// gradients to be recorded, a tangent, a mode or trace that watches calls, shapes that do not fit, a status that is not SWC_OK -- gets
+// None back, and the Python code around it, which has the whole rules and the messages, goes its own way.
 //
-// What it saves, times of a pass that the host bounds: the layer pair 1x16x16x64 23.3 -> 13.2 us, a training step 3x6x6x32 188.8 -> 96.9,
-// the model with one image 713 -> 440 (ctypes calls, one Python check after the other, and keys of Python tuples before).
+// What it saves, times of a pass that the host bounds: the layer pair 1x16x16x64 23.4 -> 13.7 us, a training step 3x6x6x32 183 -> 98,
+// the model with one image 712 -> 398 (ctypes calls, one Python check after the other, and keys of Python tuples before).
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -226,7 +226,7 @@ PyObject *mark(PyObject *, PyObject *const *args, Py_ssize_t count)
 // kept(entry, *tensors): what `entry`, a tuple (key, tensor, mark, ...), holds, for use on the current stream, or None where there is no entry
 // or its key is not that of the tensors by now.  The current stream waits for the mark where it is another than the mark's; a stream that
 // records a graph cannot wait for what was recorded outside of it, then this thread waits.  None also where there is no telling, since
-// the mark's stream records a graph by now.  One call, since a layer makes it on every pass: 0.25 us less than key, comparison and wait.
+// the mark's stream records a graph by now.  One call, since a layer makes it on every pass: 0.25 us less than a key, its comparison and the wait.
 PyObject *kept(PyObject *, PyObject *const *args, Py_ssize_t count)
 {
     HANDLE_TH_ERRORS

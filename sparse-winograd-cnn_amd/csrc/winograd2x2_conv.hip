@@ -106,7 +106,8 @@ double pieces_gain(const PiecesChoice &pieces, const ConvChoice &choice)
 {
     if (pieces.form == PIECES_NONE) return -1e30;
     if (forced_conv_tiling() != nullptr) return 1e30;
-    return 0.97 * (choice.split_wins() ? choice.split.us : choice.direct != DIRECT_NONE ? choice.direct_us : choice.whole_us / choice.wide_scale) - pieces.us;
+    const double whole_us = choice.whole_us / choice.wide_scale;
+    return 0.97 * (choice.split_wins() ? choice.split.us : choice.direct != DIRECT_NONE ? choice.direct_us : whole_us) - pieces.us;
 }
 
 template <bool BF16>
@@ -125,7 +126,8 @@ int conv_entry(const float *Input, const float *Weight, float *Output, int C, in
         const PiecesChoice pieces = choose_pieces(Input, Weight, weight_pieces, Output, ep.residual, M, C, K, BF16);
         if (pieces_gain(pieces, choice) > 0) {
             note_conv_kernel(kPiecesNames[pieces.form], kPiecesNames[pieces.form]);
-            return launch_pieces(pieces, BF16, Input, Weight, weight_pieces, Output, M, C, K, nW, ep.scale, ep.shift, ep.residual, ep.residual_relu, s);
+            return launch_pieces(pieces, BF16, Input, Weight, weight_pieces, Output, M, C, K, nW, ep.scale, ep.shift, ep.residual,
+                                 ep.residual_relu, s);
         }
     }
     const TilingChoice &pick = choice.whole;

@@ -29,8 +29,9 @@ int launch_form(DirectForm form, const float *TI, const float *Wt, float *Out, s
         // C ends in the second half of one (behind the transform, 196x100->128 10.3 us against 10.9 in turned blocks of 32, 784x124->32
         // 10.9 / 11.7; but 196x96->128 10.7 / 9.7, 196x72->128 9.7 / 9.5).
         case DIRECT_16X16:
-            return K % 4 == 0 && aligned16(Wt) && !(BF16 && C % 64 > 32) ? launch_as<DirectCfg<1, 1, 8, BF16, 3, true>>(TI, Wt, Out, M, C, K, nW, ep, s)
-                                               : launch_as<DirectCfg<1, 1, 16, BF16>>(TI, Wt, Out, M, C, K, nW, ep, s);
+            return K % 4 == 0 && aligned16(Wt) && !(BF16 && C % 64 > 32)
+                       ? launch_as<DirectCfg<1, 1, 8, BF16, 3, true>>(TI, Wt, Out, M, C, K, nW, ep, s)
+                       : launch_as<DirectCfg<1, 1, 16, BF16>>(TI, Wt, Out, M, C, K, nW, ep, s);
         case DIRECT_16X32: return launch_as<DirectCfg<1, 2, 8, BF16, 3, true>>(TI, Wt, Out, M, C, K, nW, ep, s);
         case DIRECT_16X64: return launch_as<DirectCfg<1, 4, 8, BF16, 2, true>>(TI, Wt, Out, M, C, K, nW, ep, s);
         case DIRECT_32X64: return launch_as<DirectCfg<2, 4, BF16 ? 8 : 4, BF16, BF16 ? 1 : 2, !BF16>>(TI, Wt, Out, M, C, K, nW, ep, s);

@@ -34,7 +34,8 @@ int launch_as(const float *TI, const float *Wt, const void *Wp, float *Out, size
     const size_t main_wgs = main_m * tiles_n < cus ? main_m * tiles_n : cus;
     conv_pieces_kernel<Main, Tail><<<dim3(static_cast<unsigned>(main_wgs + tail_m * tiles_n)), dim3(Main::NT), Main::LDS_BYTES, stream>>>(
         TI, Wt, static_cast<const char *>(Wp), Out, static_cast<unsigned>(M), C, K, nW, static_cast<unsigned>(main_m),
-        static_cast<unsigned>(main_wgs), static_cast<unsigned>(tail_m), static_cast<unsigned>(tiles_n), static_cast<unsigned>(panel_width(tiles_n, C)), ep);
+        static_cast<unsigned>(main_wgs), static_cast<unsigned>(tail_m), static_cast<unsigned>(tiles_n),
+        static_cast<unsigned>(panel_width(tiles_n, C)), ep);
     return check_launch();
 }
 
@@ -60,9 +61,6 @@ bool pieces_eligible(const void *TI, const void *Wt, const void *Wp, const void 
            M * 16 * static_cast<size_t>(K) < (1ull << 31);
 }
 
-}  // namespace
-
-namespace {
 // bf16 operands, us (through what else runs / pieces; in brackets behind the transform).  One round of 32-row tiles, 3.6 + 3.3 per 64
 // channels, from 512 channels and 512 columns on (960x512->384 44.0 / 44.8 behind the transform), against split32
 //   1024x512->512 37.9 / 30.0 (47.7 / 42.5)
@@ -175,10 +173,8 @@ int launch_pieces(const PiecesChoice &pick, bool bf16, const float *TI, const fl
     }
 }
 
-}  // namespace swc
-
-namespace swc {
 namespace {
+
 template <int NP>
 int make_pieces(const float *Weight, void *Pieces, int C, int K, swc_stream_t stream)
 {
@@ -190,6 +186,7 @@ int make_pieces(const float *Weight, void *Pieces, int C, int K, swc_stream_t st
         Weight, static_cast<char *>(Pieces), C, K, groups, steps);
     return check_launch();
 }
+
 }  // namespace
 }  // namespace swc
 

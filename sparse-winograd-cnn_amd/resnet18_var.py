@@ -10,8 +10,10 @@ stage 5 also runs at 14x14; ReLU, global average pool, (dropout: identity at inf
 (:213-219).  Padding of the strided conv and the pools is TensorFlow's SAME (the extra pixel goes
 after, not before).
 
-Everything except the two Winograd ops, the 1x1 shortcut convolutions and conv1 + pool1 is stock PyTorch.  Activations are kept NHWC in memory
-(channels_last), so handing them to the ops and back costs no copies.  The BatchNorm in front of
+On the GPU the Winograd ops, the 1x1 shortcut convolutions with the ReLU (in 2a BatchNorm and ReLU) in front of them, conv1 + pool1, the
+max-pools behind stages 2 and 3 and the last ReLU with its mean run on the library's kernels; the classifier, and whatever those
+kernels do not take (``fold_bn=False``, the CPU, recorded gradients, tangents, traces, other types or memory orders), is stock PyTorch.
+Activations are kept NHWC in memory (channels_last), so handing them to the ops and back costs no copies.  The BatchNorm in front of
 each WinogradImTrans (inference statistics) is folded into the transform kernel as a per-channel
 scale and shift, and the BatchNorm plus residual add behind each unit's second convolution into
 that convolution's stores; ``fold_bn=False`` runs them as separate PyTorch passes instead.
