@@ -172,7 +172,7 @@ def test_layers_at_batch_128(oracle, hw, C, K, precision):
     assert y.shape == (N, hw, hw, K)
     layer = WinogradConv(C, K, mask=(w_gpu != 0).float(), W_init=w_gpu, device=dev, precision="bf16" if stored else precision)
     with torch.no_grad():
-        for _ in range(2):   # the second call at the latest uses prepared weights
+        for _ in range(2):   # the first call makes what is kept of the weights, the second uses it
             y_layer = layer(ti)
     if torch.cuda.get_device_properties(dev).multi_processor_count == 256 and not stored:
         form = swc_hip.lib().swc_winograd2x2_conv_last_form().decode()
